@@ -461,6 +461,34 @@ __global__ void __launch_bounds__(dg_block_threads(PX, PZ)) k_dg_elem(DgElemArgs
 struct DgOp;
 
 struct DgMg;
+// one neighbour block of a mixed row: offset of the block, of the
+// neighbour's unknowns, and its columns (0: none)
+struct DgNb {
+  long long a;
+  int x, n;
+};
+
+// rows of the block system in an order of launches (dependency levels): the
+// device tables of k_dg_rows and the bounds of its launches
+struct DgRowSet {
+  std::vector<int> row_ptr;   // rows of launch l: [row_ptr[l], row_ptr[l + 1])
+  std::vector<int> task_ptr;  // mixed problems: its blocks
+  int* d_rows = nullptr;
+  int* d_nbl = nullptr;
+  int4* d_tasks = nullptr;
+  DgNb* d_nb = nullptr;
+  int* d_xoff = nullptr;
+  long long* d_voff = nullptr;
+  bool built() const { return d_rows != nullptr; }
+  int launches() const { return (int)row_ptr.size() - 1; }
+  void free_all() {
+    void* ptrs[] = {d_rows, d_nbl, d_tasks, d_nb, d_xoff, d_voff};
+    for (void* p : ptrs)
+      if (p) (void)hipFree(p);
+    *this = DgRowSet();
+  }
+};
+
 struct DgProblem {
   int mesh = 0, nel = 0, px = 1, pz = 1, ns = 0, ng = 0, nsp = 0;
   double* d_nc = nullptr;    // [18][nel]
@@ -531,13 +559,7 @@ struct DgProblem {
   bool ilu_valid = false;
   double* d_ilu = nullptr;
   double* d_ilu_inv = nullptr;
-  std::vector<int> ilu_fptr, ilu_bptr;
-  int* d_ilu_frows = nullptr;
-  int* d_ilu_brows = nullptr;
-  // wave tasks of the solves per level (ilu_ftask[l] .. ilu_ftask[l + 1])
-  std::vector<int> ilu_ftask, ilu_btask;
-  int2* d_ilu_ftasks = nullptr;
-  int2* d_ilu_btasks = nullptr;
+  DgRowSet ilu_f, ilu_b;
   // batch member (uniform degree): the block-Jacobi-preconditioned system
   // M = Dinv A, b' = Dinv b as a SELL-64 problem, rows in DOF order
   Problem* bp = nullptr;
@@ -609,10 +631,11 @@ void free_dg(DgProblem& D) {
   void* ptrs[] = {D.d_nc, D.d_qv, D.d_U, D.d_coef, D.d_stiff, D.d_rhs, D.d_fnb, D.d_fcode,
                   D.d_fhf, D.d_fval, D.d_qt, D.d_qq, D.d_blk, D.d_brhs, D.d_dinv, D.d_slots,
                   D.d_gs_elems, D.d_work, D.d_grp, D.d_deg, D.d_xoff, D.d_soff, D.d_voff,
-                  D.d_qv9, D.d_ilu, D.d_ilu_inv, D.d_ilu_frows, D.d_ilu_brows,
-                  D.d_ilu_ftasks, D.d_ilu_btasks};
+                  D.d_qv9, D.d_ilu, D.d_ilu_inv};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
+  D.ilu_f.free_all();
+  D.ilu_b.free_all();
 }
 }  // namespace
 
@@ -2157,76 +2180,146 @@ __global__ void __launch_bounds__(64) k_dg_ilu_row(int cnt, const int* rows, DgI
   for (int q = lane; q < ni * ni; q += 64) Di[q] = D[q];
 }
 
-// The solves run wave tasks: a task is up to 64 / ns rows of one level with
-// the same block size ns (rows[first .. first + count)), lane = (row of the
-// task, entry of the row).  task.y = count | ns << 8.
+// ---------------------------------------------------------------------
+// Row sums of the block system, one kernel for the ILU substitutions: for
+// every row (element) e of one dependency level
+//   t = b_e - sum_q A_q x_q,   y_e = t  or  y_e = Dinv_e t,
+// q over the row's listed neighbour blocks.  A level holds a few hundred
+// rows, so the launch is bound by the latency of its longest chain of
+// loads, not by bandwidth: one lane per unknown walking its up to 200
+// columns took 39-43 us a level (16^3 mixed degrees).  Here a row's columns
+// are dealt to S >= 6 lane groups (lane = (row, group, unknown)), so a lane
+// has at most 7 columns of a block, the loads of three blocks and of the
+// inverse are in flight together, and the groups' sums meet in LDS.
+// ---------------------------------------------------------------------
+constexpr int kRowCols = 7;  // columns of a block per lane: 40 / 6 rounded up
 
-// forward (L) solve of one level, in place: t = v_i less the lower
-// neighbours' terms in ascending neighbour order, one term at a time
-__global__ void __launch_bounds__(256) k_dg_ilu_fwd(int ntask, const int2* tasks, const int* rows,
-                                                    DgIluLay Y, const double* F, double* v,
-                                                    const int* stop) {
-  if (stop && *stop) return;
-  const int g = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (g >= ntask) return;
-  const int2 tk = tasks[g];
-  const int ni = tk.y >> 8, el = lane / ni, r = lane - el * ni;
-  if (el >= (tk.y & 255)) return;
-  const int i = rows[tk.x + el];
-  int side[5];
-  const int nl = dg_sorted_sides(Y.fnb, i, true, side);
-  const long long xi = Y.xo(i);
-  double t = v[xi + r];
-  for (int q = 0; q < nl; q++) {
-    const int s = side[q], k = Y.fnb[5 * (size_t)i + s], nk = Y.nse(k);
-    const double* A = F + Y.so(i, 1 + s) + r;
-    const double* xk = v + Y.xo(k);
-#pragma unroll 2
-    for (int c = 0; c < nk; c++) t -= A[(size_t)ni * c] * xk[c];
-  }
-  v[xi + r] = t;
+// lane groups per row and rows per 256-lane block of a row of ns unknowns
+__host__ __device__ inline int row_block_rows(int ns) {
+  const int u = 256 / ns;
+  return u >= 12 ? u / 6 : 1;
 }
+__host__ __device__ inline int row_groups(int ns) { return 256 / ns / row_block_rows(ns); }
 
-// backward (U) solve of one level, in place: t = v_i less the upper
-// neighbours' terms, then v_i = inv(D_i) t summed from 0
-__global__ void __launch_bounds__(256) k_dg_ilu_bwd(int ntask, const int2* tasks, const int* rows,
-                                                    DgIluLay Y, const double* F,
-                                                    const double* Finv, double* v,
-                                                    const int* stop) {
-  if (stop && *stop) return;
-  __shared__ double Tw[4][64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int g = blockIdx.x * 4 + wave;
-  if (g >= ntask) return;
-  const int2 tk = tasks[g];
-  const int ni = tk.y >> 8, el = lane / ni, r = lane - el * ni;
-  const bool act = el < (tk.y & 255);
-  const int i = act ? rows[tk.x + el] : 0;
-  const long long xi = act ? Y.xo(i) : 0;
-  double t = 0.0;
-  if (act) {
-    int side[5];
-    const int nu = dg_sorted_sides(Y.fnb, i, false, side);
-    t = v[xi + r];
-    for (int q = 0; q < nu; q++) {
-      const int s = side[q], j = Y.fnb[5 * (size_t)i + s], nj = Y.nse(j);
-      const double* A = F + Y.so(i, 1 + s) + r;
-      const double* xj = v + Y.xo(j);
-#pragma unroll 2
-      for (int c = 0; c < nj; c++) t -= A[(size_t)ni * c] * xj[c];
+// the rows of a launch: a uniform problem lists its rows and their
+// neighbours (-1: none) per side, everything else is computed; a mixed one
+// has a task (first row, rows, block size) per 256-lane block, the rows'
+// unknowns and inverses, and five neighbour records per row
+struct DgRowList {
+  int ns;                 // uniform: block size
+  int first, cnt;         // uniform: rows [first, first + cnt); mixed: tasks
+  const int* rows;
+  const int* nbl;
+  const int4* tasks;
+  const DgNb* nb;
+  const int* xoff;
+  const long long* voff;
+};
+
+template <bool MIXED, bool INV>
+__global__ void __launch_bounds__(256) k_dg_rows(DgRowList R, const double* A, const double* Dinv,
+                                                 const double* b, double* v, const int* stop) {
+  __shared__ double part[256], tw[256];
+  const int halt = stop ? *stop : 0;
+  int ns = R.ns, p0, nrow;
+  if (MIXED) {
+    const int4 tk = R.tasks[R.first + blockIdx.x];
+    p0 = tk.x;
+    nrow = tk.y;
+    ns = tk.z;
+  } else {
+    const int rb = row_block_rows(ns);
+    p0 = R.first + blockIdx.x * rb;
+    nrow = min(rb, R.first + R.cnt - p0);
+  }
+  const int S = row_groups(ns), tpr = ns * S;
+  const int row = threadIdx.x / tpr, q0 = threadIdx.x - row * tpr;
+  const int u = q0 / ns, r = q0 - u * ns;
+  const bool act = row < nrow;
+  const int p = act ? p0 + row : p0;
+  long long a[5], di;
+  int x[5], n[5], xe;
+  if (MIXED) {
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+      const DgNb d = R.nb[5 * (size_t)p + q];
+      a[q] = d.a;
+      x[q] = d.x;
+      n[q] = d.n;
+    }
+    xe = R.xoff[p];
+    di = R.voff[p];
+  } else {
+    const int e = R.rows[p];
+    xe = e * ns;
+    di = (long long)e * ns * ns;
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+      const int nb = R.nbl[5 * (size_t)p + q];
+      a[q] = ((long long)e * 6 + 1 + q) * ns * ns;
+      n[q] = nb < 0 ? 0 : ns;
+      x[q] = nb < 0 ? xe : nb * ns;
     }
   }
-  Tw[wave][lane] = t;
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  if (act) {
-    const double* Di = Finv + Y.vo(i) + r;
-    const double* tw = &Tw[wave][el * ni];
-    double y = 0.0;
-#pragma unroll 2
-    for (int c = 0; c < ni; c++) y += Di[(size_t)ni * c] * tw[c];
-    v[xi + r] = y;
+  if (halt) return;
+  double dv[kRowCols];
+  if (INV) {
+#pragma unroll
+    for (int k = 0; k < kRowCols; k++) {
+      const int c = u + S * k;
+      dv[k] = act ? Dinv[di + (long long)(c < ns ? c : 0) * ns + r] : 0.0;
+    }
   }
+  const double t0 = act && u == 0 && b ? b[xe + r] : 0.0;
+  double acc = 0.0;
+  if (act) {
+    // columns past a block's last repeat its first one; the select drops them
+#pragma unroll
+    for (int h = 0; h < 5; h += 3) {
+      double m[3][kRowCols], w[3][kRowCols];
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+        if (h + q >= 5) continue;
+        const double* B = A + a[h + q] + r;
+        const double* y = v + x[h + q];
+#pragma unroll
+        for (int k = 0; k < kRowCols; k++) {
+          const int c = u + S * k, cc = c < n[h + q] ? c : 0;
+          m[q][k] = B[cc * ns];
+          w[q][k] = y[cc];
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+        if (h + q >= 5) continue;
+#pragma unroll
+        for (int k = 0; k < kRowCols; k++)
+          acc += u + S * k < n[h + q] ? m[q][k] * w[q][k] : 0.0;
+      }
+    }
+  }
+  part[threadIdx.x] = acc;
+  __syncthreads();
+  double t = t0;
+  if (act && u == 0)
+    for (int k = 0; k < S; k++) t -= part[threadIdx.x + k * ns];
+  if (INV) {
+    if (act && u == 0) tw[row * ns + r] = t;
+    __syncthreads();
+    acc = 0.0;
+#pragma unroll
+    for (int k = 0; k < kRowCols; k++) {
+      const int c = u + S * k;
+      if (act && c < ns) acc += dv[k] * tw[row * ns + c];
+    }
+    part[threadIdx.x] = acc;
+    __syncthreads();
+    if (act && u == 0) {
+      t = 0.0;
+      for (int k = 0; k < S; k++) t += part[threadIdx.x + k * ns];
+    }
+  }
+  if (act && u == 0) v[xe + r] = t;
 }
 
 // w = s_j v and y = w (start of a GS-smoothed operator application)
@@ -2598,11 +2691,95 @@ DgIluLay ilu_layout(const DgProblem& D) {
                   D.mixed ? D.d_voff : nullptr};
 }
 
+template <typename T>
+int row_set_up(T** d, const std::vector<T>& h) {
+  MF_HIP(hipMalloc(d, std::max<size_t>(h.size(), 1) * sizeof(T)));
+  MF_HIP(hipMemcpy(*d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
+  return 0;
+}
+
+// device tables of the rows listed launch by launch in `rows`; take(e, nb)
+// says which neighbours belong to a row's sum.  Within a launch the rows of
+// a mixed problem are ordered by block size, so that a block's rows share it
+template <class Take>
+int build_row_set(DgProblem& D, DgRowSet& R, std::vector<int> rows, std::vector<int> row_ptr,
+                  Take take) {
+  const size_t cnt = rows.size();
+  R.row_ptr = std::move(row_ptr);
+  if (!D.mixed) {
+    std::vector<int> nbl(5 * cnt);
+    for (size_t p = 0; p < cnt; p++)
+      for (int s = 0; s < 5; s++) {
+        const int nb = D.h_fnb[5 * (size_t)rows[p] + s];
+        nbl[5 * p + s] = nb >= 0 && take(rows[p], nb) ? nb : -1;
+      }
+    return row_set_up(&R.d_nbl, nbl) || row_set_up(&R.d_rows, rows) ? -2 : 0;
+  }
+  auto nse = [&D](int e) { return ns_of_deg(D.deg[e]); };
+  std::vector<int4> tasks;
+  R.task_ptr.assign(1, 0);
+  for (int l = 0; l < R.launches(); l++) {
+    const int end = R.row_ptr[l + 1];
+    std::stable_sort(rows.begin() + R.row_ptr[l], rows.begin() + end,
+                     [&](int a, int b) { return nse(a) < nse(b); });
+    for (int q = R.row_ptr[l]; q < end;) {
+      const int ns = nse(rows[q]), rb = row_block_rows(ns);
+      int c = 0;
+      while (c < rb && q + c < end && nse(rows[q + c]) == ns) c++;
+      tasks.push_back(make_int4(q, c, ns, 0));
+      q += c;
+    }
+    R.task_ptr.push_back((int)tasks.size());
+  }
+  std::vector<DgNb> nbs(5 * cnt);
+  std::vector<int> xo(cnt);
+  std::vector<long long> vo(cnt);
+  for (size_t p = 0; p < cnt; p++) {
+    const size_t e = rows[p];
+    xo[p] = (int)D.xoff[e];
+    vo[p] = D.voff[e];
+    for (int s = 0; s < 5; s++) {
+      const int nb = D.h_fnb[5 * e + s];
+      DgNb& d = nbs[5 * p + s];
+      d.a = D.soff[6 * e + 1 + s];
+      d.n = nb >= 0 && take((int)e, nb) ? nse(nb) : 0;
+      d.x = d.n ? (int)D.xoff[nb] : xo[p];
+    }
+  }
+  if (row_set_up(&R.d_tasks, tasks) || row_set_up(&R.d_nb, nbs) || row_set_up(&R.d_xoff, xo) ||
+      row_set_up(&R.d_voff, vo) || row_set_up(&R.d_rows, rows))
+    return -2;
+  return 0;
+}
+
+// launch l of the set: v_e = [Dinv_e] (b_e - sum A x) over its rows
+void launch_rows(const DgProblem& D, const DgRowSet& R, int l, const double* A, const double* Dinv,
+                 const double* b, double* v, const int* stop) {
+  hipStream_t s = stream();
+  DgRowList L{D.ns, 0, 0, R.d_rows, R.d_nbl, R.d_tasks, R.d_nb, R.d_xoff, R.d_voff};
+  const std::vector<int>& ptr = D.mixed ? R.task_ptr : R.row_ptr;
+  L.first = ptr[l];
+  L.cnt = ptr[l + 1] - ptr[l];
+  if (L.cnt == 0) return;
+  const int rb = D.mixed ? 1 : row_block_rows(D.ns);
+  const dim3 g((L.cnt + rb - 1) / rb), t(256);
+  if (D.mixed && Dinv)
+    hipLaunchKernelGGL((k_dg_rows<true, true>), g, t, 0, s, L, A, Dinv, b, v, stop);
+  else if (D.mixed)
+    hipLaunchKernelGGL((k_dg_rows<true, false>), g, t, 0, s, L, A, Dinv, b, v, stop);
+  else if (Dinv)
+    hipLaunchKernelGGL((k_dg_rows<false, true>), g, t, 0, s, L, A, Dinv, b, v, stop);
+  else
+    hipLaunchKernelGGL((k_dg_rows<false, false>), g, t, 0, s, L, A, Dinv, b, v, stop);
+}
+
 // level schedules of the ILU: the forward level of element i is one more than
 // the largest level of its lower neighbours (0 without any), the backward
 // level likewise over its upper neighbours; rows listed level by level
 int build_ilu_levels(DgProblem& D) {
-  if (D.d_ilu_frows) return 0;
+  if (D.ilu_f.built() && D.ilu_b.built()) return 0;
+  D.ilu_f.free_all();
+  D.ilu_b.free_all();
   const int nel = D.nel;
   std::vector<int> lf(nel, 0), lb(nel, 0);
   int nlf = 0, nlb = 0;
@@ -2624,45 +2801,19 @@ int build_ilu_levels(DgProblem& D) {
     lb[e] = l;
     nlb = std::max(nlb, l + 1);
   }
-  // rows level by level, by block size within a level; wave tasks of up to
-  // 64 / ns rows of one size
-  auto nse = [&D](int e) { return D.mixed ? ns_of_deg(D.deg[e]) : D.ns; };
-  auto group = [&](const std::vector<int>& lev, int nl, std::vector<int>& ptr,
-                   std::vector<int>& rows, std::vector<int>& tptr, std::vector<int2>& tasks) {
+  auto listed = [&](const std::vector<int>& lev, int nl, std::vector<int>& ptr) {
     ptr.assign(nl + 1, 0);
     for (int e = 0; e < nel; e++) ptr[lev[e] + 1]++;
     for (int l = 0; l < nl; l++) ptr[l + 1] += ptr[l];
-    std::vector<int> pos(ptr.begin(), ptr.end() - 1);
-    rows.resize(nel);
+    std::vector<int> pos(ptr.begin(), ptr.end() - 1), rows(nel);
     for (int e = 0; e < nel; e++) rows[pos[lev[e]]++] = e;
-    tptr.assign(1, 0);
-    tasks.clear();
-    for (int l = 0; l < nl; l++) {
-      std::stable_sort(rows.begin() + ptr[l], rows.begin() + ptr[l + 1],
-                       [&](int a, int b) { return nse(a) < nse(b); });
-      int q = ptr[l];
-      while (q < ptr[l + 1]) {
-        const int ns = nse(rows[q]), epw = 64 / ns;
-        int c = 0;
-        while (c < epw && q + c < ptr[l + 1] && nse(rows[q + c]) == ns) c++;
-        tasks.push_back(make_int2(q, c | ns << 8));
-        q += c;
-      }
-      tptr.push_back((int)tasks.size());
-    }
+    return rows;
   };
-  std::vector<int> fr, br;
-  std::vector<int2> ft, bt;
-  group(lf, nlf, D.ilu_fptr, fr, D.ilu_ftask, ft);
-  group(lb, nlb, D.ilu_bptr, br, D.ilu_btask, bt);
-  MF_HIP(hipMalloc(&D.d_ilu_frows, (size_t)nel * sizeof(int)));
-  MF_HIP(hipMalloc(&D.d_ilu_brows, (size_t)nel * sizeof(int)));
-  MF_HIP(hipMalloc(&D.d_ilu_ftasks, ft.size() * sizeof(int2)));
-  MF_HIP(hipMalloc(&D.d_ilu_btasks, bt.size() * sizeof(int2)));
-  MF_HIP(hipMemcpy(D.d_ilu_frows, fr.data(), (size_t)nel * sizeof(int), hipMemcpyHostToDevice));
-  MF_HIP(hipMemcpy(D.d_ilu_brows, br.data(), (size_t)nel * sizeof(int), hipMemcpyHostToDevice));
-  MF_HIP(hipMemcpy(D.d_ilu_ftasks, ft.data(), ft.size() * sizeof(int2), hipMemcpyHostToDevice));
-  MF_HIP(hipMemcpy(D.d_ilu_btasks, bt.data(), bt.size() * sizeof(int2), hipMemcpyHostToDevice));
+  std::vector<int> fp, bp;
+  const std::vector<int> fr = listed(lf, nlf, fp), br = listed(lb, nlb, bp);
+  if (build_row_set(D, D.ilu_f, fr, fp, [](int e, int nb) { return nb < e; }) ||
+      build_row_set(D, D.ilu_b, br, bp, [](int e, int nb) { return nb > e; }))
+    return -2;
   return 0;
 }
 
@@ -2677,10 +2828,10 @@ int fill_block_ilu(DgProblem& D) {
   MF_HIP(hipMalloc(&d_bad, sizeof(int)));
   MF_HIP(hipMemsetAsync(d_bad, 0, sizeof(int), s));
   const DgIluLay Y = ilu_layout(D);
-  for (size_t l = 0; l + 1 < D.ilu_fptr.size(); l++) {
-    const int c0 = D.ilu_fptr[l], cnt = D.ilu_fptr[l + 1] - c0;
+  for (int l = 0; l < D.ilu_f.launches(); l++) {
+    const int c0 = D.ilu_f.row_ptr[l], cnt = D.ilu_f.row_ptr[l + 1] - c0;
     hipLaunchKernelGGL(k_dg_ilu_row, dim3(cnt), dim3(64), 0, s, cnt,
-                       (const int*)D.d_ilu_frows + c0, Y, D.d_ilu, D.d_ilu_inv, d_bad);
+                       (const int*)D.ilu_f.d_rows + c0, Y, D.d_ilu, D.d_ilu_inv, d_bad);
   }
   int bad = 0;
   hipError_t e = hipGetLastError();
@@ -2698,20 +2849,10 @@ int fill_block_ilu(DgProblem& D) {
 
 // v = (LU)^-1 v in place: the forward levels, then the backward levels
 int dg_ilu_solve(DgProblem& D, double* v, const int* stop) {
-  hipStream_t s = stream();
-  const DgIluLay Y = ilu_layout(D);
-  for (size_t l = 0; l + 1 < D.ilu_ftask.size(); l++) {
-    const int t0 = D.ilu_ftask[l], nt = D.ilu_ftask[l + 1] - t0;
-    hipLaunchKernelGGL(k_dg_ilu_fwd, dim3((nt + 3) / 4), dim3(256), 0, s, nt,
-                       (const int2*)D.d_ilu_ftasks + t0, (const int*)D.d_ilu_frows, Y,
-                       (const double*)D.d_ilu, v, stop);
-  }
-  for (size_t l = 0; l + 1 < D.ilu_btask.size(); l++) {
-    const int t0 = D.ilu_btask[l], nt = D.ilu_btask[l + 1] - t0;
-    hipLaunchKernelGGL(k_dg_ilu_bwd, dim3((nt + 3) / 4), dim3(256), 0, s, nt,
-                       (const int2*)D.d_ilu_btasks + t0, (const int*)D.d_ilu_brows, Y,
-                       (const double*)D.d_ilu, (const double*)D.d_ilu_inv, v, stop);
-  }
+  for (int l = 0; l < D.ilu_f.launches(); l++)
+    launch_rows(D, D.ilu_f, l, D.d_ilu, nullptr, v, v, stop);
+  for (int l = 0; l < D.ilu_b.launches(); l++)
+    launch_rows(D, D.ilu_b, l, D.d_ilu, D.d_ilu_inv, v, v, stop);
   MF_HIP(hipGetLastError());
   return 0;
 }
@@ -3577,8 +3718,8 @@ int mf_dg_fill_ilu(int did, int* nlevels) {
   const int rc = fill_block_ilu(*D);
   if (rc) return rc;
   if (nlevels) {
-    nlevels[0] = (int)D->ilu_fptr.size() - 1;
-    nlevels[1] = (int)D->ilu_bptr.size() - 1;
+    nlevels[0] = D->ilu_f.launches();
+    nlevels[1] = D->ilu_b.launches();
   }
   return 0;
 }
