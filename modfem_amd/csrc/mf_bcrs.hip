@@ -93,15 +93,25 @@ __global__ void k_bcrs_lu4(int nb, const int* diag, const double* val, double* l
 
 // solve with the factors as LAPACK dgetrs ('N') does
 __device__ __forceinline__ void lu4_solve(const double* lu, const int* ip, double* b) {
-  for (int j = 0; j < 4; j++)
-    if (ip[j] != j) {
-      const double t = b[j];
-      b[j] = b[ip[j]];
-      b[ip[j]] = t;
+  // the interchanges as selects: an index known only at run time would put
+  // b in memory
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const double t = b[j];
+#pragma unroll
+    for (int i = j + 1; i < 4; i++) {
+      const bool sw = ip[j] == i;
+      const double x = b[i];
+      b[i] = sw ? t : x;
+      b[j] = sw ? x : b[j];
     }
+  }
+#pragma unroll
   for (int k = 0; k < 4; k++)
     if (b[k] != 0.0)
+#pragma unroll
       for (int i = k + 1; i < 4; i++) b[i] = __dsub_rn(b[i], __dmul_rn(b[k], lu[i + 4 * k]));
+#pragma unroll
   for (int k = 3; k >= 0; k--)
     if (b[k] != 0.0) {
       b[k] = __ddiv_rn(b[k], lu[k + 4 * k]);
@@ -137,58 +147,86 @@ __device__ __forceinline__ void bcrs_row(int r, int dir, const int* rp, const in
   for (int k = 0; k < 4; k++) out[4 * (size_t)r + k] = vloc[k];
 }
 
-// subtract the products of blocks [s0, s1) of component k in order (two
-// blocks per step, loads first)
-__device__ __forceinline__ double chain_sub(double acc, int s0, int s1, int k, const int* ci,
-                                            const double* val, const double* y) {
-  int s = s0;
-  for (; s + 2 <= s1; s += 2) {
-    const int c0 = ci[s], c1 = ci[s + 1];
-    double a0[4], a1[4], y0[4], y1[4];
-    for (int l = 0; l < 4; l++) {
-      a0[l] = val[16 * (size_t)s + k + 4 * l];
-      a1[l] = val[16 * (size_t)(s + 1) + k + 4 * l];
-      y0[l] = y[4 * (size_t)c0 + l];
-      y1[l] = y[4 * (size_t)c1 + l];
-    }
-    for (int l = 0; l < 4; l++) acc = __dsub_rn(acc, __dmul_rn(a0[l], y0[l]));
-    for (int l = 0; l < 4; l++) acc = __dsub_rn(acc, __dmul_rn(a1[l], y1[l]));
-  }
-  if (s < s1) {
-    const int c = ci[s];
-    for (int l = 0; l < 4; l++)
-      acc = __dsub_rn(acc, __dmul_rn(val[16 * (size_t)s + k + 4 * l], y[4 * (size_t)c + l]));
-  }
-  return acc;
+// lane i of every 16-lane group reads lane (i + 4 L) % 16 of its group
+template <int L>
+__device__ __forceinline__ double group_turn(double v) {
+  if (L == 0) return v;
+  constexpr int ctrl = 0x120 + 16 - 4 * L;  // DPP row_ror: lane i takes lane (i - count) % 16
+  const unsigned long long u = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)u, ctrl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), ctrl, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
 }
 
-// block Jacobi sweep: every row reads the old v; one thread per unknown, the
-// four threads of a row exchange their sums and each solves with the
-// diagonal block's factors, keeping its own component.  With a row list
-// (rows of one colour class, none sharing a block) the same kernel sweeps
-// the class in place (out = v).
-__global__ void k_bcrs_bj(int nrows, const int* rows, int dir, const int* rp, const int* ci,
-                          const int* diag, const double* val, const double* lu, const int* piv,
-                          const double* b, const double* v, double* out, const int* stop) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 4LL * nrows || (stop && *stop)) return;
-  const int r = rows ? rows[t >> 2] : (int)(t >> 2), k = (int)(t & 3);
-  const long long i = 4LL * r + k;
-  const int d = diag[r];
+// block Jacobi sweep: every row reads the old v.  With a row list (rows of
+// one colour class, none sharing a block) the same kernel sweeps the class in
+// place (out = v).  16 lanes per row, lane (l, k) owns entry (k, l) of every
+// block, so kBjChunk blocks (128 contiguous bytes each) and their vector
+// entries are in flight together; the products of component k are then
+// subtracted in R's order (blocks in sweep order, l ascending), passed
+// between the lanes of the row by DPP.  A colour class of the 24^3 box holds
+// ~1300 rows: the launch is bound by its chain of dependent loads, and one
+// thread per unknown with two blocks in flight took 11.2 us.
+constexpr int kBjChunk = 14;
+
+__global__ void __launch_bounds__(256) k_bcrs_bj(int nrows, const int* rows, int dir,
+                                                 const int* rp, const int* ci, const int* diag,
+                                                 const double* val, const double* lu,
+                                                 const int* piv, const double* b, const double* v,
+                                                 double* out, const int* stop) {
+  const int t = blockIdx.x * 16 + (threadIdx.x >> 4), e = threadIdx.x & 15, k = e & 3, l = e >> 2;
+  const int halt = stop ? *stop : 0;
+  const bool act = t < nrows;
+  const int tt = act ? t : nrows - 1;
+  const int r = rows ? rows[tt] : tt;
+  const int r0 = rp[r], r1 = rp[r + 1], d = diag[r];
+  if (halt) return;
+  // blocks in sweep order: dir 0 the lower ones, then the upper ones; dir 1
+  // the other way round
+  const int nlow = d - r0, nup = r1 - d - 1, nbk = nlow + nup;
+  const int n1 = dir == 0 ? nlow : nup;
+  const int s1 = dir == 0 ? r0 : d + 1, s2 = (dir == 0 ? d + 1 : r0) - n1;
+  double f[16];
+  int ip[4];
+#pragma unroll
+  for (int q = 0; q < 16; q++) f[q] = lu[16 * (size_t)r + q];
+#pragma unroll
+  for (int q = 0; q < 4; q++) ip[q] = piv[4 * (size_t)r + q];
+  const double bk = b ? b[4 * (size_t)r + k] : 0.0;
   double acc = 0.0;
-  if (dir == 0) {
-    acc = chain_sub(acc, rp[r], d, k, ci, val, v);
-    acc = chain_sub(acc, d + 1, rp[r + 1], k, ci, val, v);
-  } else {
-    acc = chain_sub(acc, d + 1, rp[r + 1], k, ci, val, v);
-    acc = chain_sub(acc, rp[r], d, k, ci, val, v);
+  for (int q0 = 0; q0 < nbk; q0 += kBjChunk) {
+    double a[kBjChunk], y[kBjChunk];
+    int c[kBjChunk];
+#pragma unroll
+    for (int q = 0; q < kBjChunk; q++) {
+      const int w = min(q0 + q, nbk - 1), s = w < n1 ? s1 + w : s2 + w;
+      c[q] = ci[s];
+      a[q] = val[16 * (size_t)s + e];
+    }
+#pragma unroll
+    for (int q = 0; q < kBjChunk; q++) y[q] = v[4 * (size_t)c[q] + l];
+#pragma unroll
+    for (int q = 0; q < kBjChunk; q++) {
+      const double p = __dmul_rn(a[q], y[q]);
+      double z = __dsub_rn(acc, p);
+      z = __dsub_rn(z, group_turn<1>(p));
+      z = __dsub_rn(z, group_turn<2>(p));
+      z = __dsub_rn(z, group_turn<3>(p));
+      acc = q0 + q < nbk ? z : acc;
+    }
   }
-  if (b) acc = __dadd_rn(acc, b[i]);
-  const int base = (int)(threadIdx.x & ~3u);
+  if (b) acc = __dadd_rn(acc, bk);
+  // the sums of components 0..3 sit in lanes 0..3 of the group
+  const int base = (int)(threadIdx.x & 48u);
   double y[4];
+#pragma unroll
   for (int q = 0; q < 4; q++) y[q] = __shfl(acc, base + q, 64);
-  lu4_solve(lu + 16 * (size_t)r, piv + 4 * (size_t)r, y);
-  out[i] = y[k];
+  lu4_solve(f, ip, y);
+  double o = y[0];
+  o = k == 1 ? y[1] : o;
+  o = k == 2 ? y[2] : o;
+  o = k == 3 ? y[3] : o;
+  if (act && l == 0) out[4 * (size_t)r + k] = o;
 }
 
 // block Gauss-Seidel, the rows of one level: passed blocks read the sweep's
@@ -618,7 +656,7 @@ int bcrs_sweeps(BcrsDev& M, int gs, int nr_prec, const double* b, double* v, dou
         for (int q = 0; q < ncol; q++) {
           const int c = dir == 0 ? q : ncol - 1 - q;
           const int cnt = M.col_ptr[c + 1] - M.col_ptr[c];
-          hipLaunchKernelGGL(k_bcrs_bj, dim3((4 * cnt + 255) / 256), dim3(256), 0, stream(), cnt,
+          hipLaunchKernelGGL(k_bcrs_bj, dim3((cnt + 15) / 16), dim3(256), 0, stream(), cnt,
                              M.d_col_rows + M.col_ptr[c], 0, M.d_rp, M.d_ci, M.d_diag, M.d_val,
                              M.d_lu, M.d_piv, b, v, v, stop);
         }
@@ -629,7 +667,7 @@ int bcrs_sweeps(BcrsDev& M, int gs, int nr_prec, const double* b, double* v, dou
   for (int it = 0; it < loops; it++)
     for (int dir = 0; dir < dirs; dir++) {
       if (!gs) {
-        hipLaunchKernelGGL(k_bcrs_bj, dim3(gv), dim3(256), 0, stream(), M.nb, nullptr, dir,
+        hipLaunchKernelGGL(k_bcrs_bj, dim3((M.nb + 15) / 16), dim3(256), 0, stream(), M.nb, nullptr, dir,
                            M.d_rp, M.d_ci, M.d_diag, M.d_val, M.d_lu, M.d_piv, b, v, tmp, stop);
       } else {
         const std::vector<int>& lp = M.lev_ptr[dir];
