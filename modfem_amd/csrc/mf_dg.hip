@@ -478,11 +478,11 @@ struct DgRowSet {
   int4* d_tasks = nullptr;
   DgNb* d_nb = nullptr;
   int* d_xoff = nullptr;
-  long long* d_voff = nullptr;
+  long long *d_aoff = nullptr, *d_voff = nullptr;
   bool built() const { return d_rows != nullptr; }
   int launches() const { return (int)row_ptr.size() - 1; }
   void free_all() {
-    void* ptrs[] = {d_rows, d_nbl, d_tasks, d_nb, d_xoff, d_voff};
+    void* ptrs[] = {d_rows, d_nbl, d_tasks, d_nb, d_xoff, d_aoff, d_voff};
     for (void* p : ptrs)
       if (p) (void)hipFree(p);
     *this = DgRowSet();
@@ -524,8 +524,8 @@ struct DgProblem {
   bool assembled = false, dinv_valid = false;
   // multicolour block Gauss-Seidel: elements grouped by colour (no two
   // neighbours share a colour), sweeps per application
-  std::vector<int> gs_color_ptr;
-  int* d_gs_elems = nullptr;
+  DgRowSet gs_rows;
+  DgRowSet op_rows;           // the operator's rows (mixed problems)
   int gs_sweeps = 2;
   double* d_work = nullptr;   // n, GS work vector
   Problem* P = nullptr;       // GMRES workspace over the block system
@@ -551,8 +551,6 @@ struct DgProblem {
   int qv_off[kNDeg] = {0};
   // interior slots grouped by (own degree, neighbour degree): slot_ptr[kNDeg^2 + 1]
   std::vector<int> slot_ptr;
-  // Gauss-Seidel colours split by degree: gs_cd_ptr[kNDeg c + d]
-  std::vector<int> gs_cd_ptr;
   // block ILU(0) in element order: factors on the block-row layout (d_ilu),
   // inverses of U's diagonal blocks (d_ilu_inv, inverse layout), rows by
   // level of the forward (factor, L solve) and backward (U solve) schedules
@@ -630,12 +628,11 @@ void free_dg(DgProblem& D) {
   free_dg_batch(D);
   void* ptrs[] = {D.d_nc, D.d_qv, D.d_U, D.d_coef, D.d_stiff, D.d_rhs, D.d_fnb, D.d_fcode,
                   D.d_fhf, D.d_fval, D.d_qt, D.d_qq, D.d_blk, D.d_brhs, D.d_dinv, D.d_slots,
-                  D.d_gs_elems, D.d_work, D.d_grp, D.d_deg, D.d_xoff, D.d_soff, D.d_voff,
+                  D.d_work, D.d_grp, D.d_deg, D.d_xoff, D.d_soff, D.d_voff,
                   D.d_qv9, D.d_ilu, D.d_ilu_inv};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
-  D.ilu_f.free_all();
-  D.ilu_b.free_all();
+  for (DgRowSet* R : {&D.ilu_f, &D.ilu_b, &D.gs_rows, &D.op_rows}) R->free_all();
 }
 }  // namespace
 
@@ -1853,60 +1850,63 @@ __global__ void __launch_bounds__(64) k_dg_inv(const int* elems, const long long
   }
 }
 
-// acc + (or -) sum_k B[k ld + i] x[k] over N columns, unrolled
-template <int N, int SIGN>
-__device__ __forceinline__ double colsum(double acc, const double* B, int ld, int i,
-                                         const double* x) {
+// Rows of a uniform problem, 64 / NS elements per wave, lane = (element,
+// row): the kernels of the operator and of a colour of a Gauss-Seidel sweep.
+// The sides' neighbours are read first and a side's block and vector entries
+// are requested while the side before it is summed (two sides in flight);
+// the entries of a neighbour come in pairs where NS is even (every vector
+// starts on 16 bytes).  A side without a neighbour repeats the own entries
+// and drops the products, so the loads never wait for a branch.
+template <int NS>
+struct DgSide {
+  double m[NS], x[NS];
+  __device__ __forceinline__ void load(const double* B, const double* xn, int i) {
 #pragma unroll
-  for (int k = 0; k < N; k++) {
-    if (SIGN > 0) acc += B[(size_t)k * ld + i] * x[k];
-    else acc -= B[(size_t)k * ld + i] * x[k];
+    for (int k = 0; k < NS; k++) m[k] = B[(size_t)k * NS + i];
+    if constexpr (NS % 2 == 0) {
+#pragma unroll
+      for (int k = 0; k < NS; k += 2) {
+        const double2 t = *reinterpret_cast<const double2*>(xn + k);
+        x[k] = t.x;
+        x[k + 1] = t.y;
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < NS; k++) x[k] = xn[k];
+    }
   }
-  return acc;
-}
-
-// the neighbour columns of a mixed block row: the isotropic block sizes
-// unrolled, any other size by a plain loop
-template <int SIGN>
-__device__ __forceinline__ double nb_colsum(double acc, const double* B, int ld, int i,
-                                            const double* x, int dn) {
-  switch (dn) {
-    case 0: return colsum<6, SIGN>(acc, B, ld, i, x);
-    case 4: return colsum<18, SIGN>(acc, B, ld, i, x);
-    case 8: return colsum<40, SIGN>(acc, B, ld, i, x);
-    case 9: return colsum<4, SIGN>(acc, B, ld, i, x);
-    case 10: return colsum<10, SIGN>(acc, B, ld, i, x);
-    case 11: return colsum<20, SIGN>(acc, B, ld, i, x);
+  __device__ __forceinline__ double sum(double acc) const {
+#pragma unroll
+    for (int k = 0; k < NS; k++) acc += m[k] * x[k];
+    return acc;
   }
-  const int n = ns_of_deg(dn);
-  for (int k = 0; k < n; k++) {
-    if (SIGN > 0) acc += B[(size_t)k * ld + i] * x[k];
-    else acc -= B[(size_t)k * ld + i] * x[k];
-  }
-  return acc;
-}
-
-// Layout of a block system for the operator kernels: a uniform problem has
-// rows [nel][6][NS*NS] and vectors [nel][NS] (offset arrays null); a mixed
-// one has per-element offsets of unknowns (xoff), block-row slots (soff) and
-// block inverses (voff), and the degree index of every element
-struct DgLayout {
-  const int* fnb;
-  const int* deg;
-  const long long* xoff;
-  const long long* soff;
-  const long long* voff;
 };
 
-// w = scale * Dinv (A x) for the block rows (mode 0, scale = sc[j] when sc,
-// else 1; Dinv skipped when dinv is null), or r = Dinv (b - A x) (mode 1),
-// for the cnt elements of one degree (elems, or 0..cnt-1 when null).
-// 64 / NS elements per wave, lane = (element, row).
-template <int NS, bool MIXED>
-__global__ void __launch_bounds__(256) k_dg_op(int cnt, const int* elems, DgLayout Y,
-                                               const double* blk, const double* dinv,
-                                               const double* x, const double* b, const double* sc,
-                                               int j, const int* stop, double* w, int mode) {
+// acc plus the products of the five sides of element e; `at`: the element's
+// own entries in the vector
+template <int NS>
+__device__ __forceinline__ double dg_sides(double acc, const double* Ae, const int* nb, int e,
+                                           const double* x, int i) {
+  DgSide<NS> b[2];
+  b[0].load(Ae + (size_t)NS * NS, x + (size_t)(nb[0] < 0 ? e : nb[0]) * NS, i);
+#pragma unroll
+  for (int s = 0; s < 5; s++) {
+    if (s < 4)
+      b[(s + 1) & 1].load(Ae + (size_t)(2 + s) * NS * NS,
+                          x + (size_t)(nb[s + 1] < 0 ? e : nb[s + 1]) * NS, i);
+    const double t = b[s & 1].sum(acc);
+    acc = nb[s] < 0 ? acc : t;
+  }
+  return acc;
+}
+
+// w = scale * Dinv (A x) (mode 0, scale = sc[j] when sc, else 1; Dinv skipped
+// when dinv is null), or r = Dinv (b - A x) (mode 1)
+template <int NS>
+__global__ void __launch_bounds__(256) k_dg_op(int cnt, const int* fnb, const double* blk,
+                                               const double* dinv, const double* x,
+                                               const double* b, const double* sc, int j,
+                                               const int* stop, double* w, int mode) {
   if (stop && *stop) return;
   constexpr int EPW = 64 / NS;
   __shared__ double T[4][64];
@@ -1914,27 +1914,19 @@ __global__ void __launch_bounds__(256) k_dg_op(int cnt, const int* elems, DgLayo
   const int el = lane / NS, i = lane - el * NS;
   const double s = sc ? sc[j] : 1.0;
   for (int g0 = (blockIdx.x * 4 + wave) * EPW; g0 < cnt; g0 += gridDim.x * 4 * EPW) {
-    const int gi = g0 + el;
-    const bool act = el < EPW && gi < cnt;
-    const int e = act ? (MIXED ? elems[gi] : gi) : 0;
-    const size_t xe0 = MIXED ? Y.xoff[e] : (size_t)e * NS;
+    const int e = g0 + el;
+    const bool act = el < EPW && e < cnt;
+    const size_t xe0 = (size_t)e * NS;
     double acc = 0.0;
     if (act) {
-      const double* Ae = blk + (MIXED ? Y.soff[6 * (size_t)e] : (size_t)e * 6 * NS * NS);
-      const double* xe = x + xe0;
-      for (int k = 0; k < NS; k++) acc += Ae[(size_t)k * NS + i] * xe[k];
-      for (int sd = 0; sd < 5; sd++) {
-        const int nb = Y.fnb[5 * (size_t)e + sd];
-        if (nb < 0) continue;
-        if (MIXED) {
-          acc = nb_colsum<1>(acc, blk + Y.soff[6 * (size_t)e + 1 + sd], NS, i, x + Y.xoff[nb],
-                             Y.deg[nb]);
-        } else {
-          const double* B = Ae + (size_t)(1 + sd) * NS * NS;
-          const double* xn = x + (size_t)nb * NS;
-          for (int k = 0; k < NS; k++) acc += B[(size_t)k * NS + i] * xn[k];
-        }
-      }
+      const double* Ae = blk + (size_t)e * 6 * NS * NS;
+      int nb[5];
+#pragma unroll
+      for (int q = 0; q < 5; q++) nb[q] = fnb[5 * (size_t)e + q];
+      DgSide<NS> own;
+      own.load(Ae, x + xe0, i);
+      acc = own.sum(0.0);
+      acc = dg_sides<NS>(acc, Ae, nb, e, x, i);
       if (mode == 1) acc = b[xe0 + i] - acc;
     }
     if (!dinv) {
@@ -1946,8 +1938,9 @@ __global__ void __launch_bounds__(256) k_dg_op(int cnt, const int* elems, DgLayo
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     double r = 0.0;
     if (act) {
-      const double* Di = dinv + (MIXED ? Y.voff[e] : (size_t)e * NS * NS);
+      const double* Di = dinv + (size_t)e * NS * NS;
       const double* t = &T[wave][el * NS];
+#pragma unroll
       for (int k = 0; k < NS; k++) r += Di[(size_t)k * NS + i] * t[k];
       w[xe0 + i] = (mode == 1 ? 1.0 : s) * r;
     }
@@ -1958,47 +1951,42 @@ __global__ void __launch_bounds__(256) k_dg_op(int cnt, const int* elems, DgLayo
 
 // one colour of a block Gauss-Seidel sweep (lar_perform_BJ_or_GS_iterations
 // for block storage, las_block_intf.c:2269-2460, in colour order):
-// x_e = Dinv_e (b_e - sum_s B_{e,s} x_nb(s)) for the colour's elements of
-// one degree (b null: zero right-hand side)
-template <int NS, bool MIXED>
-__global__ void __launch_bounds__(256) k_dg_gs(int cnt, const int* elems, DgLayout Y,
+// x_e = Dinv_e (b_e - sum_s B_{e,s} x_nb(s)) for rows [p0, p0 + cnt) of the
+// colour's list (b null: zero right-hand side)
+template <int NS>
+__global__ void __launch_bounds__(256) k_dg_gs(int p0, int cnt, const int* rows, const int* nbl,
                                                const double* blk, const double* dinv,
                                                const double* b, double* x, const int* stop) {
-  if (stop && *stop) return;
+  const int halt = stop ? *stop : 0;
   constexpr int EPW = 64 / NS;
   __shared__ double T[4][64];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int el = lane / NS, i = lane - el * NS;
   for (int g0 = (blockIdx.x * 4 + wave) * EPW; g0 < cnt; g0 += gridDim.x * 4 * EPW) {
-    const int gi = g0 + el;
-    const bool act = el < EPW && gi < cnt;
-    const int e = act ? elems[gi] : 0;
-    const size_t xe0 = MIXED ? Y.xoff[e] : (size_t)e * NS;
-    double acc = 0.0;
+    const bool act = el < EPW && g0 + el < cnt;
+    const int p = p0 + (act ? g0 + el : 0);
+    const int e = rows[p];
+    int nb[5];
+#pragma unroll
+    for (int q = 0; q < 5; q++) nb[q] = nbl[5 * (size_t)p + q];
+    if (halt) return;
+    const size_t xe0 = (size_t)e * NS;
+    double acc = 0.0, d[NS];
     if (act) {
-      acc = b ? b[xe0 + i] : 0.0;
-      const double* Ae = blk + (MIXED ? Y.soff[6 * (size_t)e] : (size_t)e * 6 * NS * NS);
-      for (int sd = 0; sd < 5; sd++) {
-        const int nb = Y.fnb[5 * (size_t)e + sd];
-        if (nb < 0) continue;
-        if (MIXED) {
-          acc = nb_colsum<-1>(acc, blk + Y.soff[6 * (size_t)e + 1 + sd], NS, i, x + Y.xoff[nb],
-                              Y.deg[nb]);
-        } else {
-          const double* B = Ae + (size_t)(1 + sd) * NS * NS;
-          const double* xn = x + (size_t)nb * NS;
-          for (int k = 0; k < NS; k++) acc -= B[(size_t)k * NS + i] * xn[k];
-        }
-      }
+      const double bi = b ? b[xe0 + i] : 0.0;
+      acc = bi - dg_sides<NS>(0.0, blk + (size_t)e * 6 * NS * NS, nb, e, x, i);
+      const double* Di = dinv + (size_t)e * NS * NS;
+#pragma unroll
+      for (int k = 0; k < NS; k++) d[k] = Di[(size_t)k * NS + i];
     }
     T[wave][lane] = acc;
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     double r = 0.0;
     if (act) {
-      const double* Di = dinv + (MIXED ? Y.voff[e] : (size_t)e * NS * NS);
       const double* t = &T[wave][el * NS];
-      for (int k = 0; k < NS; k++) r += Di[(size_t)k * NS + i] * t[k];
+#pragma unroll
+      for (int k = 0; k < NS; k++) r += d[k] * t[k];
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -2181,10 +2169,13 @@ __global__ void __launch_bounds__(64) k_dg_ilu_row(int cnt, const int* rows, DgI
 }
 
 // ---------------------------------------------------------------------
-// Row sums of the block system, one kernel for the ILU substitutions: for
-// every row (element) e of one dependency level
-//   t = b_e - sum_q A_q x_q,   y_e = t  or  y_e = Dinv_e t,
-// q over the row's listed neighbour blocks.  A level holds a few hundred
+// Row sums of the block system, one kernel for the ILU substitutions, the
+// Gauss-Seidel sweeps and the operator: for every listed row (element) e
+//   t = b_e - sum_q A_q x_q  (with the own block and b null: t = sum),
+//   y_e = s t  or  y_e = s Dinv_e t,
+// q over the row's listed neighbour blocks (OWN: and its own block; s =
+// sc[j], 1 without sc).  In place (y = v) a launch's rows must not be
+// neighbours: one dependency level or colour.  A level holds a few hundred
 // rows, so the launch is bound by the latency of its longest chain of
 // loads, not by bandwidth: one lane per unknown walking its up to 200
 // columns took 39-43 us a level (16^3 mixed degrees).  Here a row's columns
@@ -2192,19 +2183,27 @@ __global__ void __launch_bounds__(64) k_dg_ilu_row(int cnt, const int* rows, DgI
 // has at most 7 columns of a block, the loads of three blocks and of the
 // inverse are in flight together, and the groups' sums meet in LDS.
 // ---------------------------------------------------------------------
-constexpr int kRowCols = 7;  // columns of a block per lane: 40 / 6 rounded up
+constexpr int kRowCols = 7;  // most columns of a block per lane: 40 / 6 rounded up
 
-// lane groups per row and rows per 256-lane block of a row of ns unknowns
-__host__ __device__ inline int row_block_rows(int ns) {
-  const int u = 256 / ns;
-  return u >= 12 ? u / 6 : 1;
+// lane groups per row and rows per 256-lane block of a row of ns unknowns:
+// about three columns of an own-sized block per lane, so that short rows are
+// not split further than their loads need (with six groups for every size a
+// colour of the 20^3 box took 1.4 times as long at p = 2); the rows of a
+// mixed problem meet blocks of up to 40 columns and take six groups or more
+__host__ __device__ inline int row_block_rows(int ns, bool mixed) {
+  const int u = 256 / ns, want = mixed ? 6 : (ns + 2) / 3;
+  const int r = mixed ? u / want : (2 * u + want) / (2 * want);
+  return r > 1 ? r : 1;
 }
-__host__ __device__ inline int row_groups(int ns) { return 256 / ns / row_block_rows(ns); }
+__host__ __device__ inline int row_groups(int ns, bool mixed) {
+  return 256 / ns / row_block_rows(ns, mixed);
+}
 
 // the rows of a launch: a uniform problem lists its rows and their
 // neighbours (-1: none) per side, everything else is computed; a mixed one
-// has a task (first row, rows, block size) per 256-lane block, the rows'
-// unknowns and inverses, and five neighbour records per row
+// has a task per 256-lane block (first row, rows, block size, and the columns
+// per lane of neighbour record q in bits 3q..3q+2: the most over its rows),
+// the rows' unknowns and inverses, and five neighbour records per row
 struct DgRowList {
   int ns;                 // uniform: block size
   int first, cnt;         // uniform: rows [first, first + cnt); mixed: tasks
@@ -2213,32 +2212,38 @@ struct DgRowList {
   const int4* tasks;
   const DgNb* nb;
   const int* xoff;
+  const long long* aoff;  // the rows' own blocks
   const long long* voff;
 };
 
-template <bool MIXED, bool INV>
+template <bool MIXED, bool INV, bool OWN>
 __global__ void __launch_bounds__(256) k_dg_rows(DgRowList R, const double* A, const double* Dinv,
-                                                 const double* b, double* v, const int* stop) {
+                                                 const double* b, const double* v, double* y,
+                                                 const double* sc, int j, const int* stop) {
+  constexpr int NB = OWN ? 6 : 5;
   __shared__ double part[256], tw[256];
   const int halt = stop ? *stop : 0;
-  int ns = R.ns, p0, nrow;
+  const double s = sc ? sc[j] : 1.0;
+  int ns = R.ns, p0, nrow, cols = 0;
   if (MIXED) {
     const int4 tk = R.tasks[R.first + blockIdx.x];
     p0 = tk.x;
     nrow = tk.y;
     ns = tk.z;
+    cols = tk.w;
   } else {
-    const int rb = row_block_rows(ns);
+    const int rb = row_block_rows(ns, false);
     p0 = R.first + blockIdx.x * rb;
     nrow = min(rb, R.first + R.cnt - p0);
   }
-  const int S = row_groups(ns), tpr = ns * S;
+  const int S = row_groups(ns, MIXED), tpr = ns * S;
+  const int own = (ns + S - 1) / S;  // columns per lane of an own-sized block
   const int row = threadIdx.x / tpr, q0 = threadIdx.x - row * tpr;
   const int u = q0 / ns, r = q0 - u * ns;
   const bool act = row < nrow;
   const int p = act ? p0 + row : p0;
-  long long a[5], di;
-  int x[5], n[5], xe;
+  long long a[NB], di;
+  int x[NB], n[NB], xe;
   if (MIXED) {
 #pragma unroll
     for (int q = 0; q < 5; q++) {
@@ -2249,9 +2254,11 @@ __global__ void __launch_bounds__(256) k_dg_rows(DgRowList R, const double* A, c
     }
     xe = R.xoff[p];
     di = R.voff[p];
+    if (OWN) a[NB - 1] = R.aoff[p];
   } else {
     const int e = R.rows[p];
     xe = e * ns;
+    if (OWN) a[NB - 1] = (long long)e * 6 * ns * ns;
     di = (long long)e * ns * ns;
 #pragma unroll
     for (int q = 0; q < 5; q++) {
@@ -2261,37 +2268,47 @@ __global__ void __launch_bounds__(256) k_dg_rows(DgRowList R, const double* A, c
       x[q] = nb < 0 ? xe : nb * ns;
     }
   }
+  if (OWN) {
+    n[NB - 1] = ns;
+    x[NB - 1] = xe;
+  }
   if (halt) return;
   double dv[kRowCols];
   if (INV) {
 #pragma unroll
     for (int k = 0; k < kRowCols; k++) {
       const int c = u + S * k;
-      dv[k] = act ? Dinv[di + (long long)(c < ns ? c : 0) * ns + r] : 0.0;
+      dv[k] = 0.0;
+      if (k < own && act) dv[k] = Dinv[di + (long long)(c < ns ? c : 0) * ns + r];
     }
   }
   const double t0 = act && u == 0 && b ? b[xe + r] : 0.0;
   double acc = 0.0;
   if (act) {
-    // columns past a block's last repeat its first one; the select drops them
+    // columns past a block's last repeat its first one; the select drops
+    // them.  The column counts are the block's own: no lane-wise branches
 #pragma unroll
-    for (int h = 0; h < 5; h += 3) {
+    for (int h = 0; h < NB; h += 3) {
       double m[3][kRowCols], w[3][kRowCols];
 #pragma unroll
       for (int q = 0; q < 3; q++) {
-        if (h + q >= 5) continue;
+        if (h + q >= NB) continue;
         const double* B = A + a[h + q] + r;
-        const double* y = v + x[h + q];
+        const double* xq = v + x[h + q];
+        const int kc = MIXED && h + q < 5 ? cols >> 3 * (h + q) & 7 : own;
 #pragma unroll
         for (int k = 0; k < kRowCols; k++) {
           const int c = u + S * k, cc = c < n[h + q] ? c : 0;
-          m[q][k] = B[cc * ns];
-          w[q][k] = y[cc];
+          m[q][k] = w[q][k] = 0.0;
+          if (k < kc) {
+            m[q][k] = B[cc * ns];
+            w[q][k] = xq[cc];
+          }
         }
       }
 #pragma unroll
       for (int q = 0; q < 3; q++) {
-        if (h + q >= 5) continue;
+        if (h + q >= NB) continue;
 #pragma unroll
         for (int k = 0; k < kRowCols; k++)
           acc += u + S * k < n[h + q] ? m[q][k] * w[q][k] : 0.0;
@@ -2300,9 +2317,11 @@ __global__ void __launch_bounds__(256) k_dg_rows(DgRowList R, const double* A, c
   }
   part[threadIdx.x] = acc;
   __syncthreads();
-  double t = t0;
-  if (act && u == 0)
-    for (int k = 0; k < S; k++) t -= part[threadIdx.x + k * ns];
+  double t = 0.0;
+  if (act && u == 0) {
+    for (int k = 0; k < S; k++) t += part[threadIdx.x + k * ns];
+    if (!OWN || b) t = t0 - t;
+  }
   if (INV) {
     if (act && u == 0) tw[row * ns + r] = t;
     __syncthreads();
@@ -2310,7 +2329,7 @@ __global__ void __launch_bounds__(256) k_dg_rows(DgRowList R, const double* A, c
 #pragma unroll
     for (int k = 0; k < kRowCols; k++) {
       const int c = u + S * k;
-      if (act && c < ns) acc += dv[k] * tw[row * ns + c];
+      if (k < own && act && c < ns) acc += dv[k] * tw[row * ns + c];
     }
     part[threadIdx.x] = acc;
     __syncthreads();
@@ -2319,7 +2338,7 @@ __global__ void __launch_bounds__(256) k_dg_rows(DgRowList R, const double* A, c
       for (int k = 0; k < S; k++) t += part[threadIdx.x + k * ns];
     }
   }
-  if (act && u == 0) v[xe + r] = t;
+  if (act && u == 0) y[xe + r] = s * t;
 }
 
 // w = s_j v and y = w (start of a GS-smoothed operator application)
@@ -2338,6 +2357,126 @@ __global__ void k_dg_sub(long long n, const double* y, double* w, const int* sto
   if (stop && *stop) return;
   const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (k < n) w[k] -= y[k];
+}
+
+}  // namespace
+
+namespace {
+
+template <typename T>
+int row_set_up(T** d, const std::vector<T>& h) {
+  MF_HIP(hipMalloc(d, std::max<size_t>(h.size(), 1) * sizeof(T)));
+  MF_HIP(hipMemcpy(*d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
+  return 0;
+}
+
+// device tables of the rows listed launch by launch in `rows`; take(e, nb)
+// says which neighbours belong to a row's sum.  Within a launch the rows of
+// a mixed problem are ordered by their own and their neighbours' sizes, so
+// that a block's rows share them
+template <class Take>
+int build_row_set(DgProblem& D, DgRowSet& R, std::vector<int> rows, std::vector<int> row_ptr,
+                  Take take) {
+  const size_t cnt = rows.size();
+  R.row_ptr = std::move(row_ptr);
+  if (!D.mixed) {
+    std::vector<int> nbl(5 * cnt);
+    for (size_t p = 0; p < cnt; p++)
+      for (int s = 0; s < 5; s++) {
+        const int nb = D.h_fnb[5 * (size_t)rows[p] + s];
+        nbl[5 * p + s] = nb >= 0 && take(rows[p], nb) ? nb : -1;
+      }
+    return row_set_up(&R.d_nbl, nbl) || row_set_up(&R.d_rows, rows) ? -2 : 0;
+  }
+  auto nse = [&D](int e) { return ns_of_deg(D.deg[e]); };
+  // the sides of a row's sum, largest neighbour first: their columns (0: not
+  // in the sum), and one number to sort the rows by (own size, then columns)
+  struct Sides {
+    uint64_t key;
+    unsigned char n[5], side[5];
+  };
+  std::vector<Sides> sides(D.nel);
+  for (int e = 0; e < D.nel; e++) {
+    Sides& v = sides[e];
+    for (int s = 0; s < 5; s++) {
+      const int nb = D.h_fnb[5 * (size_t)e + s];
+      const unsigned char c = nb >= 0 && take(e, nb) ? (unsigned char)nse(nb) : 0;
+      int t = s;
+      for (; t > 0 && v.n[t - 1] < c; t--) {
+        v.n[t] = v.n[t - 1];
+        v.side[t] = v.side[t - 1];
+      }
+      v.n[t] = c;
+      v.side[t] = (unsigned char)s;
+    }
+    v.key = (uint64_t)nse(e);
+    for (int t = 0; t < 5; t++) v.key = v.key << 8 | (255 - v.n[t]);
+  }
+  std::vector<int4> tasks;
+  R.task_ptr.assign(1, 0);
+  for (int l = 0; l < R.launches(); l++) {
+    const int end = R.row_ptr[l + 1];
+    std::stable_sort(rows.begin() + R.row_ptr[l], rows.begin() + end,
+                     [&](int a, int b) { return sides[a].key < sides[b].key; });
+    for (int q = R.row_ptr[l]; q < end;) {
+      const int ns = nse(rows[q]), rb = row_block_rows(ns, true), S = row_groups(ns, true);
+      int c = 0, cols = 0;
+      for (; c < rb && q + c < end && nse(rows[q + c]) == ns; c++) {
+        for (int t = 0; t < 5; t++) {
+          const int kc = (sides[rows[q + c]].n[t] + S - 1) / S;
+          if (kc > (cols >> 3 * t & 7)) cols = (cols & ~(7 << 3 * t)) | kc << 3 * t;
+        }
+      }
+      tasks.push_back(make_int4(q, c, ns, cols));
+      q += c;
+    }
+    R.task_ptr.push_back((int)tasks.size());
+  }
+  std::vector<DgNb> nbs(5 * cnt);
+  std::vector<int> xo(cnt);
+  std::vector<long long> ao(cnt), vo(cnt);
+  for (size_t p = 0; p < cnt; p++) {
+    const size_t e = rows[p];
+    xo[p] = (int)D.xoff[e];
+    ao[p] = D.soff[6 * e];
+    vo[p] = D.voff[e];
+    for (int t = 0; t < 5; t++) {
+      const int s = sides[e].side[t];
+      DgNb& d = nbs[5 * p + t];
+      d.a = D.soff[6 * e + 1 + s];
+      d.n = sides[e].n[t];
+      d.x = d.n ? (int)D.xoff[D.h_fnb[5 * e + s]] : xo[p];
+    }
+  }
+  if (row_set_up(&R.d_tasks, tasks) || row_set_up(&R.d_nb, nbs) || row_set_up(&R.d_xoff, xo) ||
+      row_set_up(&R.d_aoff, ao) || row_set_up(&R.d_voff, vo) || row_set_up(&R.d_rows, rows))
+    return -2;
+  return 0;
+}
+
+template <bool OWN>
+void launch_row_list(const DgProblem& D, const DgRowList& L, const double* A, const double* Dinv,
+                     const double* b, const double* v, double* y, const double* sc, int j,
+                     const int* stop) {
+  if (L.cnt == 0) return;
+  const int rb = D.mixed ? 1 : row_block_rows(D.ns, false);
+  const dim3 g((L.cnt + rb - 1) / rb);
+  // the operator of a uniform problem has its own kernel (k_dg_op)
+  auto k = D.mixed ? (Dinv ? k_dg_rows<true, true, OWN> : k_dg_rows<true, false, OWN>)
+                   : (Dinv ? k_dg_rows<false, true, false> : k_dg_rows<false, false, false>);
+  hipLaunchKernelGGL(k, g, dim3(256), 0, stream(), L, A, Dinv, b, v, y, sc, j, stop);
+}
+
+DgRowList row_list(const DgProblem& D, const DgRowSet& R, int l) {
+  const std::vector<int>& ptr = D.mixed ? R.task_ptr : R.row_ptr;
+  return DgRowList{D.ns,      ptr[l], ptr[l + 1] - ptr[l], R.d_rows,  R.d_nbl,
+                   R.d_tasks, R.d_nb, R.d_xoff,            R.d_aoff, R.d_voff};
+}
+
+// launch l of the set, in place: v_e = [Dinv_e] (b_e - sum A x) over its rows
+void launch_rows(const DgProblem& D, const DgRowSet& R, int l, const double* A, const double* Dinv,
+                 const double* b, double* v, const int* stop) {
+  launch_row_list<false>(D, row_list(D, R, l), A, Dinv, b, v, v, nullptr, 0, stop);
 }
 
 }  // namespace
@@ -2368,10 +2507,6 @@ static int with_ns(int d, F& f) {
 struct DgOp : ExtOp {
   DgProblem* D = nullptr;
   int precon = 1;
-  DgLayout layout() const {
-    return DgLayout{D->d_fnb, D->mixed ? D->d_deg : nullptr, D->mixed ? D->d_xoff : nullptr,
-                    D->mixed ? D->d_soff : nullptr, D->mixed ? D->d_voff : nullptr};
-  }
   int grid(int cnt, int ns) const {
     const int epw = 64 / ns;
     const long long waves = (cnt + epw - 1) / epw;
@@ -2383,52 +2518,55 @@ struct DgOp : ExtOp {
   double* w_ = nullptr;
   int j_ = 0, mode_ = 0, color_ = -1;
   template <int NS>
-  int run(int d) {
-    if (color_ < 0) {  // operator over the elements of degree d
-      const int c0 = D->grp_ptr[d], cnt = D->grp_ptr[d + 1] - c0;
-      if (D->mixed)
-        hipLaunchKernelGGL((k_dg_op<NS, true>), dim3(grid(cnt, NS)), dim3(256), 0, stream(), cnt,
-                           (const int*)D->d_grp + c0, layout(), D->d_blk,
-                           precon == 1 ? D->d_dinv : nullptr, x_, b_, sc_, j_, stop_, w_, mode_);
-      else
-        hipLaunchKernelGGL((k_dg_op<NS, false>), dim3(grid(cnt, NS)), dim3(256), 0, stream(), cnt,
-                           nullptr, layout(), D->d_blk, precon == 1 ? D->d_dinv : nullptr, x_, b_,
-                           sc_, j_, stop_, w_, mode_);
-    } else {  // the elements of degree d in colour color_
-      const size_t k = kNDeg * (size_t)color_ + d;
-      const int c0 = D->gs_cd_ptr[k], cnt = D->gs_cd_ptr[k + 1] - c0;
-      if (D->mixed)
-        hipLaunchKernelGGL((k_dg_gs<NS, true>), dim3(grid(cnt, NS)), dim3(256), 0, stream(), cnt,
-                           (const int*)D->d_gs_elems + c0, layout(), D->d_blk, D->d_dinv, b_, w_,
-                           stop_);
-      else
-        hipLaunchKernelGGL((k_dg_gs<NS, false>), dim3(grid(cnt, NS)), dim3(256), 0, stream(), cnt,
-                           (const int*)D->d_gs_elems + c0, layout(), D->d_blk, D->d_dinv, b_, w_,
-                           stop_);
+  int run(int) {
+    if (color_ < 0) {
+      hipLaunchKernelGGL(k_dg_op<NS>, dim3(grid(D->nel, NS)), dim3(256), 0, stream(), D->nel,
+                         D->d_fnb, D->d_blk, precon == 1 ? D->d_dinv : nullptr, x_, b_, sc_, j_,
+                         stop_, w_, mode_);
+    } else {
+      const DgRowSet& R = D->gs_rows;
+      const int c0 = R.row_ptr[color_], cnt = R.row_ptr[color_ + 1] - c0;
+      hipLaunchKernelGGL(k_dg_gs<NS>, dim3(grid(cnt, NS)), dim3(256), 0, stream(), c0, cnt,
+                         R.d_rows, R.d_nbl, D->d_blk, D->d_dinv, b_, w_, stop_);
     }
     MF_HIP(hipGetLastError());
     return 0;
   }
   int op(const double* x, const double* b, const double* sc, int j, const int* stop, double* w,
          int mode) {
+    if (D->mixed) {
+      DgRowSet& R = D->op_rows;
+      if (!R.built()) {
+        // one launch over all degrees, rows in the order of their blocks
+        std::vector<int> rows(D->nel);
+        for (int e = 0; e < D->nel; e++) rows[e] = e;
+        std::stable_sort(rows.begin(), rows.end(),
+                         [this](int a, int c) { return D->deg[a] < D->deg[c]; });
+        R.free_all();
+        if (build_row_set(*D, R, rows, {0, D->nel}, [](int, int) { return true; })) return -2;
+      }
+      launch_row_list<true>(*D, row_list(*D, R, 0), D->d_blk, precon == 1 ? D->d_dinv : nullptr,
+                            mode == 1 ? b : nullptr, x, w, mode == 1 ? nullptr : sc, j, stop);
+      MF_HIP(hipGetLastError());
+      return 0;
+    }
     x_ = x; b_ = b; sc_ = sc; j_ = j; stop_ = stop; w_ = w; mode_ = mode; color_ = -1;
-    for (int d = 0; d < kNDeg; d++)
-      if (D->grp_ptr[d + 1] > D->grp_ptr[d] && with_ns(d, *this)) return -2;
-    return 0;
+    return with_ns(D->deg[0], *this);
   }
   int sweeps(const double* b, double* y, const int* stop) {
-    const int ncol = (int)D->gs_color_ptr.size() - 1;
     b_ = b; w_ = y; stop_ = stop;
+    int rc = 0;
     for (int k = 0; k < D->gs_sweeps; k++)
-      for (int c = 0; c < ncol; c++)
-        for (int d = 0; d < kNDeg; d++) {
-          const size_t q = kNDeg * (size_t)c + d;
-          if (D->gs_cd_ptr[q + 1] == D->gs_cd_ptr[q]) continue;
-          color_ = c;
-          if (with_ns(d, *this)) return -2;
-        }
+      for (int c = 0; c < D->gs_rows.launches() && rc == 0; c++) {
+        color_ = c;
+        if (D->mixed)
+          launch_rows(*D, D->gs_rows, c, D->d_blk, D->d_dinv, b, y, stop);
+        else
+          rc = with_ns(D->deg[0], *this);
+      }
     color_ = -1;
-    return 0;
+    MF_HIP(hipGetLastError());
+    return rc;
   }
   int run_mg(const double* x, const double* b, const double* sc, int j, const int* stop,
              double* w, int mode);
@@ -2621,10 +2759,9 @@ int launch_inv_t(DgProblem& D, int d, int* d_bad) {
 // greedy colouring of the element graph (elements sharing a face get
 // different colours), elements listed colour by colour
 int build_gs_colors(DgProblem& D) {
-  if (D.d_gs_elems) return 0;
-  const size_t nf = 5 * (size_t)D.nel;
-  std::vector<int> fnb(nf);
-  MF_HIP(hipMemcpy(fnb.data(), D.d_fnb, nf * sizeof(int), hipMemcpyDeviceToHost));
+  if (D.gs_rows.built()) return 0;
+  D.gs_rows.free_all();
+  const std::vector<int>& fnb = D.h_fnb;
   std::vector<int> col(D.nel, -1);
   int ncol = 0;
   for (int e = 0; e < D.nel; e++) {
@@ -2638,17 +2775,12 @@ int build_gs_colors(DgProblem& D) {
     col[e] = c;
     ncol = std::max(ncol, c + 1);
   }
-  D.gs_color_ptr.assign(ncol + 1, 0);
-  for (int e = 0; e < D.nel; e++) D.gs_color_ptr[col[e] + 1]++;
-  for (int c = 0; c < ncol; c++) D.gs_color_ptr[c + 1] += D.gs_color_ptr[c];
-  // within a colour, elements grouped by degree (ascending element order in each group)
-  D.gs_cd_ptr.assign(kNDeg * (size_t)ncol + 1, 0);
-  for (int e = 0; e < D.nel; e++) D.gs_cd_ptr[kNDeg * (size_t)col[e] + D.deg[e] + 1]++;
-  for (size_t k = 0; k + 1 < D.gs_cd_ptr.size(); k++) D.gs_cd_ptr[k + 1] += D.gs_cd_ptr[k];
-  std::vector<int> pos(D.gs_cd_ptr.begin(), D.gs_cd_ptr.end() - 1), elems(D.nel);
-  for (int e = 0; e < D.nel; e++) elems[pos[kNDeg * (size_t)col[e] + D.deg[e]]++] = e;
-  MF_HIP(hipMalloc(&D.d_gs_elems, (size_t)D.nel * sizeof(int)));
-  MF_HIP(hipMemcpy(D.d_gs_elems, elems.data(), (size_t)D.nel * sizeof(int), hipMemcpyHostToDevice));
+  std::vector<int> ptr(ncol + 1, 0);
+  for (int e = 0; e < D.nel; e++) ptr[col[e] + 1]++;
+  for (int c = 0; c < ncol; c++) ptr[c + 1] += ptr[c];
+  std::vector<int> pos(ptr.begin(), ptr.end() - 1), elems(D.nel);
+  for (int e = 0; e < D.nel; e++) elems[pos[col[e]]++] = e;
+  if (build_row_set(D, D.gs_rows, elems, ptr, [](int, int) { return true; })) return -2;
   if (!D.d_work) MF_HIP(hipMalloc(&D.d_work, (size_t)D.ndof * sizeof(double)));
   return 0;
 }
@@ -2689,88 +2821,6 @@ DgIluLay ilu_layout(const DgProblem& D) {
   return DgIluLay{D.d_fnb, D.d_fcode, D.mixed ? D.d_deg : nullptr, D.mixed ? 0 : D.ns,
                   D.mixed ? D.d_xoff : nullptr, D.mixed ? D.d_soff : nullptr,
                   D.mixed ? D.d_voff : nullptr};
-}
-
-template <typename T>
-int row_set_up(T** d, const std::vector<T>& h) {
-  MF_HIP(hipMalloc(d, std::max<size_t>(h.size(), 1) * sizeof(T)));
-  MF_HIP(hipMemcpy(*d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
-  return 0;
-}
-
-// device tables of the rows listed launch by launch in `rows`; take(e, nb)
-// says which neighbours belong to a row's sum.  Within a launch the rows of
-// a mixed problem are ordered by block size, so that a block's rows share it
-template <class Take>
-int build_row_set(DgProblem& D, DgRowSet& R, std::vector<int> rows, std::vector<int> row_ptr,
-                  Take take) {
-  const size_t cnt = rows.size();
-  R.row_ptr = std::move(row_ptr);
-  if (!D.mixed) {
-    std::vector<int> nbl(5 * cnt);
-    for (size_t p = 0; p < cnt; p++)
-      for (int s = 0; s < 5; s++) {
-        const int nb = D.h_fnb[5 * (size_t)rows[p] + s];
-        nbl[5 * p + s] = nb >= 0 && take(rows[p], nb) ? nb : -1;
-      }
-    return row_set_up(&R.d_nbl, nbl) || row_set_up(&R.d_rows, rows) ? -2 : 0;
-  }
-  auto nse = [&D](int e) { return ns_of_deg(D.deg[e]); };
-  std::vector<int4> tasks;
-  R.task_ptr.assign(1, 0);
-  for (int l = 0; l < R.launches(); l++) {
-    const int end = R.row_ptr[l + 1];
-    std::stable_sort(rows.begin() + R.row_ptr[l], rows.begin() + end,
-                     [&](int a, int b) { return nse(a) < nse(b); });
-    for (int q = R.row_ptr[l]; q < end;) {
-      const int ns = nse(rows[q]), rb = row_block_rows(ns);
-      int c = 0;
-      while (c < rb && q + c < end && nse(rows[q + c]) == ns) c++;
-      tasks.push_back(make_int4(q, c, ns, 0));
-      q += c;
-    }
-    R.task_ptr.push_back((int)tasks.size());
-  }
-  std::vector<DgNb> nbs(5 * cnt);
-  std::vector<int> xo(cnt);
-  std::vector<long long> vo(cnt);
-  for (size_t p = 0; p < cnt; p++) {
-    const size_t e = rows[p];
-    xo[p] = (int)D.xoff[e];
-    vo[p] = D.voff[e];
-    for (int s = 0; s < 5; s++) {
-      const int nb = D.h_fnb[5 * e + s];
-      DgNb& d = nbs[5 * p + s];
-      d.a = D.soff[6 * e + 1 + s];
-      d.n = nb >= 0 && take((int)e, nb) ? nse(nb) : 0;
-      d.x = d.n ? (int)D.xoff[nb] : xo[p];
-    }
-  }
-  if (row_set_up(&R.d_tasks, tasks) || row_set_up(&R.d_nb, nbs) || row_set_up(&R.d_xoff, xo) ||
-      row_set_up(&R.d_voff, vo) || row_set_up(&R.d_rows, rows))
-    return -2;
-  return 0;
-}
-
-// launch l of the set: v_e = [Dinv_e] (b_e - sum A x) over its rows
-void launch_rows(const DgProblem& D, const DgRowSet& R, int l, const double* A, const double* Dinv,
-                 const double* b, double* v, const int* stop) {
-  hipStream_t s = stream();
-  DgRowList L{D.ns, 0, 0, R.d_rows, R.d_nbl, R.d_tasks, R.d_nb, R.d_xoff, R.d_voff};
-  const std::vector<int>& ptr = D.mixed ? R.task_ptr : R.row_ptr;
-  L.first = ptr[l];
-  L.cnt = ptr[l + 1] - ptr[l];
-  if (L.cnt == 0) return;
-  const int rb = D.mixed ? 1 : row_block_rows(D.ns);
-  const dim3 g((L.cnt + rb - 1) / rb), t(256);
-  if (D.mixed && Dinv)
-    hipLaunchKernelGGL((k_dg_rows<true, true>), g, t, 0, s, L, A, Dinv, b, v, stop);
-  else if (D.mixed)
-    hipLaunchKernelGGL((k_dg_rows<true, false>), g, t, 0, s, L, A, Dinv, b, v, stop);
-  else if (Dinv)
-    hipLaunchKernelGGL((k_dg_rows<false, true>), g, t, 0, s, L, A, Dinv, b, v, stop);
-  else
-    hipLaunchKernelGGL((k_dg_rows<false, false>), g, t, 0, s, L, A, Dinv, b, v, stop);
 }
 
 // level schedules of the ILU: the forward level of element i is one more than
@@ -3816,7 +3866,7 @@ int mf_dg_set_gs(int did, int nsweeps, int* ncolors) {
   }
   D->gs_sweeps = nsweeps;
   if (build_gs_colors(*D)) return -2;
-  if (ncolors) *ncolors = (int)D->gs_color_ptr.size() - 1;
+  if (ncolors) *ncolors = D->gs_rows.launches();
   return 0;
 }
 

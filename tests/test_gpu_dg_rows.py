@@ -38,23 +38,32 @@ def blocks_of(row, ns, cols):
     return [np.asarray(r).T for r in row]
 
 
-def substitute(rows, nb, xo, b, dtype):
-    """forward then backward substitution in element order"""
-    v = b.astype(dtype).copy()
+def substitute(rows, nb, xo, b):
+    """forward then backward substitution in element order in extended
+    precision, and a running bound of what any order of the float64 sums can
+    be off: a sum of up to 240 products is off by gamma = 240 roundings of the
+    sum of magnitudes, and carries the errors of the values it reads"""
+    g = 240 * 2.0 ** -53
+    v, eb = b.astype(np.longdouble), np.zeros(len(b))
     nel = len(rows)
-    for e in range(nel):
-        for s in range(5):
-            k = nb[e, s]
-            if 0 <= k < e:
-                v[xo[e]:xo[e + 1]] -= rows[e][1 + s].astype(dtype) @ v[xo[k]:xo[k + 1]]
-    for e in range(nel - 1, -1, -1):
-        t = v[xo[e]:xo[e + 1]].copy()
-        for s in range(5):
-            k = nb[e, s]
-            if k > e:
-                t -= rows[e][1 + s].astype(dtype) @ v[xo[k]:xo[k + 1]]
-        v[xo[e]:xo[e + 1]] = rows[e][0].astype(dtype) @ t
-    return v
+    for back in (False, True):
+        for e in range(nel - 1, -1, -1) if back else range(nel):
+            me = slice(xo[e], xo[e + 1])
+            t, mag, off = v[me].copy(), np.abs(v[me].astype(float)), eb[me].copy()
+            for s in range(5):
+                k = nb[e, s]
+                if (k > e) if back else (0 <= k < e):
+                    A, at = rows[e][1 + s], slice(xo[k], xo[k + 1])
+                    t -= A.astype(np.longdouble) @ v[at]
+                    mag += np.abs(A) @ np.abs(v[at].astype(float))
+                    off += np.abs(A) @ eb[at]
+            off += g * mag
+            if back:
+                D = rows[e][0]
+                off = np.abs(D) @ off + g * (np.abs(D) @ np.abs(t.astype(float)))
+                t = D.astype(np.longdouble) @ t
+            v[me], eb[me] = t, off
+    return v, eb
 
 
 @pytest.mark.parametrize("dims", [(1, 1, 1), (3, 2, 3)])
@@ -67,16 +76,9 @@ def test_substitutions_at_every_block_size(case, dims):
     xo = dg.xoff
     rows = [blocks_of(dg.ilu_row(e), xo[e + 1] - xo[e], None) for e in range(dg.nel)]
     b = np.random.default_rng(3).normal(size=dg.ndof)
-    ref = substitute(rows, nb, xo, b, np.longdouble)
-    f64 = substitute(rows, nb, xo, b, np.float64)
-    v = dg.ilu_apply(b)
-    # a row sums at most 240 products: the error of any order of the sum is
-    # within a small factor of float64's own error on the same factors, plus
-    # 240 roundings of the result
-    scale = float(np.abs(ref).max())
-    own = float(np.abs(f64 - ref).max())
-    err = float(np.abs(v - ref).max())
-    print("  error %.1e, float64 %.1e of %.1e" % (err, own, scale), flush=True)
-    assert err <= 8 * own + 240 * 2.0 ** -53 * scale
+    ref, bound = substitute(rows, nb, xo, b)
+    err = np.abs(dg.ilu_apply(b) - ref).astype(float)
+    print("  largest error / bound %.2g" % (err / bound).max(), flush=True)
+    assert (err <= bound).all()
     dg.free()
     mesh.free()
