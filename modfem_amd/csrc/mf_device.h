@@ -270,7 +270,7 @@ struct Batch {
   GmresStat* d_stat = nullptr;
   GmresStat* h_pinned = nullptr;
   int nblk = 0, cap = 0, blk_cap = 0;
-  size_t lds = 0;
+  int max_blk = 0;  // blocks of the largest member
   hipGraphExec_t exec = nullptr;
   hipGraph_t graph = nullptr;
   int cycles = 0;

@@ -12,15 +12,22 @@
 // basis V is (m+1) vectors with a padded stride ldv (multiple of 64 doubles)
 // so that every vector starts 512-byte aligned.
 //
-// One Arnoldi step j is four launches on the library stream:
-//   k_op_dots    w = s_j D^-1 A V_j written to V_{j+1}; per-block partial
-//                dot products V_i . w for i <= j.  Rows are processed in
-//                tiles: a tile's CRS entries are streamed coalesced into LDS
-//                products, then one lane owns one row for the row sum, the
-//                scaling and the dot products.
-//   k_fin_dots   one block: h_i = s_i sum(partials), c_i = h_i s_i
-//   k_update     w -= sum_i c_i V_i, per-block partial ||w||^2
-//   k_fin_update one block: h_{j+1,j} = ||w||, Givens rotations, stopping test
+// One Arnoldi step j is two launches on the library stream (three for large
+// systems, whose many partial dots are reduced once by k_fin_dots):
+//   k_op_dots_sell / k_op_dots_one
+//                w = s_j D^-1 A V_j written to V_{j+1}; per-block partial
+//                dot products V_i . w for i <= j on the matrix cores.  An
+//                extra block finishes step j - 1 meanwhile: h_{j,j-1}, Givens
+//                rotations, stopping test
+//   k_update     h_i = s_i sum(partials), c_i = h_i s_i; w -= sum_i c_i V_i,
+//                per-block partial ||w||^2.  Its blocks run over the rows
+//                backwards, so that the last rows an operator launch touched
+//                (and those the update touched last, for the next operator)
+//                are still in the 256 MB cache: 2.15 M rows, m = 50: operator
+//                213 -> 206 us, update 87 -> 84 us on average
+//   k_fin_update finishes the last step of a cycle
+// Measured per step (m = 30, Jacobi; four launches before): 9,261 rows 29.8
+// -> 16.4 us, 117,649 rows 32.4 -> 23.1 us.
 // The basis vectors stay unnormalised (scale factors s_i = 1/||V_i||), so no
 // separate normalisation pass is needed.  Every kernel of a step returns at
 // once when the stopping flag is set, so a whole restart cycle is enqueued
@@ -145,63 +152,194 @@ __global__ void __launch_bounds__(SB) k_residual_sell(SolveArgs A) {
   residual_any(A, s0, s1, lb);
 }
 
-// Arnoldi step j, part 1 (SELL-64).  Phase 1: w = s_j D^-1 A V_j for the
-// block's slices, written to V_{j+1} and staged in LDS.  Phase 2: wavefront q
-// forms V_i . w over the block's rows for i = q, q+SW, ..., streaming V_i with
-// four independent accumulators and one wave-wide sum per i, so the number of
-// basis vectors costs neither registers nor occupancy.
-template <typename VT>
+// h_{j+1,j} = ||w||, Givens rotations (drot/drotg as lss_mkb_core.c:2539-2560),
+// stopping tests (:2562-2590)
+__device__ __forceinline__ void fin_update_body(const SolveArgs& A, int j, int G) {
+  __shared__ double col[MAX_NV + 1], giv[2 * MAX_NV], g2[2];
+  double s = 0.0;
+  for (int b = threadIdx.x; b < G; b += (int)blockDim.x) s += A.norms[b];
+  double* hc = Hcol(A, j + 1);
+  double* gv = Giv(A);
+  for (int i = threadIdx.x; i <= j; i += (int)blockDim.x) col[i] = hc[i];
+  for (int i = threadIdx.x; i < 2 * j; i += (int)blockDim.x) giv[i] = gv[i];
+  s = block_sum_all(s);  // every thread's col and giv entries are visible too
+  if (threadIdx.x == 0) {
+    const int m = A.m;
+    const double hn = sqrt(s);
+    col[j + 1] = hn;
+    Scale(A)[j + 1] = 1.0 / hn;
+    for (int i = 1; i <= j; i++) rot(&col[i - 1], &col[i], giv[2 * (i - 1)], giv[2 * (i - 1) + 1]);
+    double ra = col[j], rb = col[j + 1], c, sn;
+    drotg_dev(&ra, &rb, &c, &sn);
+    gv[2 * j] = c;
+    gv[2 * j + 1] = sn;
+    rot(&col[j], &col[j + 1], c, sn);
+    double* g = Hcol(A, 0);
+    g2[0] = g[j];
+    g2[1] = g[j + 1];
+    rot(&g2[0], &g2[1], c, sn);
+    g[j] = g2[0];
+    g[j + 1] = g2[1];
+    GmresStat* st = A.stat;
+    st->gmiter += 1;
+    st->j_done = j + 1;
+    st->resid = fabs(g2[1]);
+    st->res_rel = st->beta0 != 0.0 ? st->resid / st->beta0 : 0.0;
+    if (st->resid < st->tol_res || st->res_rel < st->tol_rel) {
+      st->converged = 1;
+      st->stop = j + 1;
+    }
+    if (j + 1 == m || st->gmiter == st->max_iter) st->stop = j + 1;
+    if (A.hstat) *A.hstat = *st;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i <= j + 1; i += (int)blockDim.x) hc[i] = col[i];
+}
+
+// Arnoldi step j, part 1 (SELL-64): w = s_j D^-1 A V_j for the block's slices,
+// written to V_{j+1}, and the partial dots V_i . w, i <= j.  A wavefront owns
+// a slice, lane = row; it hands its w to the matrix cores through its own 64
+// doubles of LDS.  sj() gives s_j once the first slice's row sums are formed
+// (it may wait for the block).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int NQ, typename VT, class Scl>
 __device__ __forceinline__ void op_dots_body(const SolveArgs& A, int j, const SliceSet& S, int pb,
-                                             int G, double* ws) {
-  const int ns = S.count();
+                                             int G, Scl sj) {
+  __shared__ double wl[OPB];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   VT* V = basis<VT>(A);
   const VT* x = V + (size_t)j * A.ldv;
   VT* w = V + (size_t)(j + 1) * A.ldv;
-  const double sj = Scale(A)[j];
-  for (int t = wv; t < ns; t += SW) {
-    const int sl = S.slice(t);
-    const double s = sell_row_op(A, x, sl, lane);
+  double acc[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; q++) acc[q] = 0.0;
+  int sl = S.first(wv);
+  double sum = sl < S.end ? sell_row_op(A, x, sl, lane) : 0.0;
+  const double s = sj();
+  while (sl < S.end) {
     const int r = sl * 64 + lane;
     double wr = 0.0;
     if (r < A.n) {
-      const VT wq = (VT)jacobi(A, r, sj * s);
+      const VT wq = (VT)jacobi(A, r, s * sum);
       w[r] = wq;
       wr = (double)wq;
     }
-    ws[t * 64 + lane] = wr;
-  }
-  __syncthreads();
-  for (int i = wv; i <= j; i += SW) {
-    const VT* v = V + (size_t)i * A.ldv + lane;
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-    int t = 0;
+    wl[threadIdx.x] = wr;
+    wave_lds_fence();
+    double b[4];
+    slot_rows_lds<VT>(wl + 64 * wv, lane >> 2, b);
     // rows past n read zero padding of V (ldv covers whole slices) times w = 0
-    for (; t + 3 < ns; t += 4) {
-      a0 += (double)v[(size_t)S.slice(t) * 64] * ws[t * 64 + lane];
-      a1 += (double)v[(size_t)S.slice(t + 1) * 64] * ws[(t + 1) * 64 + lane];
-      a2 += (double)v[(size_t)S.slice(t + 2) * 64] * ws[(t + 2) * 64 + lane];
-      a3 += (double)v[(size_t)S.slice(t + 3) * 64] * ws[(t + 3) * 64 + lane];
+    dots_slice<0, NQ>(V + (size_t)sl * 64, A.ldv, j, lane, b, acc);
+    __builtin_amdgcn_wave_barrier();
+    sl += S.step;
+    if (sl < S.end) sum = sell_row_op(A, x, sl, lane);
+  }
+  dots_finish<NQ>(acc, j, G, pb, A.partials);
+}
+
+// the same for one slice per wavefront (a launch of one round, bound by its
+// chain of loads): the row's entries are requested at once, and the first
+// vectors of the dots and the row's Jacobi inverse behind them
+template <int NQ, typename VT, class Scl>
+__device__ __forceinline__ void op_dots_one(const SolveArgs& A, int j, const SliceSet& S, int pb,
+                                            int G, Scl sj) {
+  __shared__ double wl[OPB];
+  constexpr int NP = NQ < 8 ? NQ : 8;  // quads requested ahead
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  VT* V = basis<VT>(A);
+  const VT* x = V + (size_t)j * A.ldv;
+  double acc[NQ], v[NP][4], d = 1.0, sum = 0.0;
+#pragma unroll
+  for (int q = 0; q < NQ; q++) acc[q] = 0.0;
+  const int sl = __builtin_amdgcn_readfirstlane(S.first(wv));
+  const bool on = sl < S.end;
+  const int r = sl * 64 + lane;
+  const VT* Vs = V + (size_t)sl * 64;
+  if (on)
+    sum = sell_row_one_op(A, x, sl, lane, [&]() {
+      if (r < A.n) d = jacobi(A, r, 1.0);
+      dots_load<NP>(Vs, A.ldv, j, lane, 0, v);
+    });
+  const double s = sj();
+  if (on) {
+    double wr = 0.0;
+    if (r < A.n) {
+      const VT wq = (VT)((s * sum) * d);
+      V[(size_t)(j + 1) * A.ldv + r] = wq;
+      wr = (double)wq;
     }
-    for (; t < ns; t++) a0 += (double)v[(size_t)S.slice(t) * 64] * ws[t * 64 + lane];
-    const double d = wave_sum((a0 + a1) + (a2 + a3));
-    if (lane == 0) A.partials[(size_t)i * G + pb] = d;
+    wl[threadIdx.x] = wr;
+    wave_lds_fence();
+    double b[4];
+    slot_rows_lds<VT>(wl + 64 * wv, lane >> 2, b);
+    dots_add<NP>(v, b, acc);
+    dots_slice<NP, NQ>(Vs, A.ldv, j, lane, b, acc);
+  }
+  dots_finish<NQ>(acc, j, G, pb, A.partials);
+}
+
+template <int NQ, bool ONE, class Scl>
+__device__ __forceinline__ void op_dots_any(const SolveArgs& A, int j, const SliceSet& S, int pb,
+                                            int G, Scl sj) {
+  if constexpr (ONE) {
+    if (A.v32)
+      op_dots_one<NQ, float>(A, j, S, pb, G, sj);
+    else
+      op_dots_one<NQ, double>(A, j, S, pb, G, sj);
+  } else {
+    if (A.v32)
+      op_dots_body<NQ, float>(A, j, S, pb, G, sj);
+    else
+      op_dots_body<NQ, double>(A, j, S, pb, G, sj);
   }
 }
 
-__device__ __forceinline__ void op_dots_any(const SolveArgs& A, int j, const SliceSet& S, int pb,
-                                            int G, double* ws) {
-  if (A.v32)
-    op_dots_body<float>(A, j, S, pb, G, ws);
-  else
-    op_dots_body<double>(A, j, S, pb, G, ws);
+// The first of kFinBlocks extra blocks (dispatched first; eight keep the
+// others' XCDs) finishes step j - 1 (its norm, Givens rotation and stopping
+// test) while the G blocks of the operator run: they form the norm
+// themselves from the Gu partial sums of the last update, in the same order.
+// A stop found here (stop = j) ends the cycle at the next launch; this step's
+// V_{j+1} is then not used.  The blocks of this launch go on whether or not
+// they see it, so all of a block's waves agree.  ONE: a slice per wavefront.
+constexpr int kFinBlocks = 8;
+
+template <int NQ, bool ONE>
+__device__ __forceinline__ void op_dots_step(const SolveArgs& A, int j, int G, int Gu) {
+  const int stop = A.stat->stop;
+  const int bid = (int)blockIdx.x - (j > 0 ? kFinBlocks : 0);
+  if (bid < 0) {
+    if (blockIdx.x == 0 && (stop == 0 || stop >= j)) fin_update_body(A, j - 1, Gu);
+    return;
+  }
+  double p = 0.0;
+  if (j > 0)
+    for (int b = threadIdx.x; b < Gu; b += (int)blockDim.x) p += A.norms[b];
+  if (stop && stop < j) return;
+  const int nsl = (A.n + 63) >> 6, W = blockDim.x >> 6;
+  SliceSet S;
+  if (ONE) {  // block b of the XCD-contiguous order holds slices [b W, (b + 1) W)
+    S.base = xcd_block(bid, G) * W;
+    S.step = S.end = nsl;
+  } else {
+    S = block_slices(nsl, bid, G, W);
+  }
+  op_dots_any<NQ, ONE>(A, j, S, bid, G,
+                       [&]() { return j > 0 ? 1.0 / sqrt(block_sum_all(p)) : Scale(A)[0]; });
 }
 
-__global__ void __launch_bounds__(SB) k_op_dots_sell(SolveArgs A, int j) {
-  if (A.stat->stop) return;
-  extern __shared__ double ws[];  // w of the block's slices, 64 per slice
-  const int nsl = (A.n + 63) >> 6;
-  op_dots_any(A, j, block_slices(nsl), blockIdx.x, gridDim.x, ws);
+template <int NQ>
+__global__ void __launch_bounds__(OPB, 4) k_op_dots_sell(SolveArgs A, int j, int G, int Gu) {
+  op_dots_step<NQ, false>(A, j, G, Gu);
+}
+
+template <int NQ>
+__global__ void __launch_bounds__(OPB, 2) k_op_dots_one(SolveArgs A, int j, int G, int Gu) {
+  op_dots_step<NQ, true>(A, j, G, Gu);
 }
 
 // ILU-preconditioned Arnoldi step (precon 2), part 1a: w = s_j A V_j into
@@ -209,62 +347,60 @@ __global__ void __launch_bounds__(SB) k_op_dots_sell(SolveArgs A, int j) {
 // CGS dots with the preconditioned w
 template <typename VT>
 __device__ __forceinline__ void op_body(const SolveArgs& A, int j, const SliceSet& S) {
-  const int ns = S.count();
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   VT* V = basis<VT>(A);
   const VT* x = V + (size_t)j * A.ldv;
   VT* w = V + (size_t)(j + 1) * A.ldv;
   const double sj = Scale(A)[j];
-  for (int t = wv; t < ns; t += SW) {
-    const int sl = S.slice(t);
+  for (int sl = S.first(wv); sl < S.end; sl += S.step) {
     const double sum = sell_row_op(A, x, sl, lane);
     const int r = sl * 64 + lane;
     if (r < A.n) w[r] = (VT)(sj * sum);
   }
 }
 
-__global__ void __launch_bounds__(SB) k_op_sell(SolveArgs A, int j) {
+__global__ void __launch_bounds__(OPB) k_op_sell(SolveArgs A, int j) {
   if (A.stat->stop) return;
-  const SliceSet S = block_slices((A.n + 63) >> 6);
+  const SliceSet S = block_slices((A.n + 63) >> 6, blockIdx.x, gridDim.x, blockDim.x >> 6);
   if (A.v32)
     op_body<float>(A, j, S);
   else
     op_body<double>(A, j, S);
 }
 
-template <typename VT>
+template <int NQ, typename VT>
 __device__ __forceinline__ void dots_body(const SolveArgs& A, int j, const SliceSet& S, int pb,
                                           int G) {
-  const int ns = S.count();
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const VT* V = basis<VT>(A);
-  const VT* w = V + (size_t)(j + 1) * A.ldv + lane;
-  for (int i = wv; i <= j; i += SW) {
-    const VT* v = V + (size_t)i * A.ldv + lane;
-    double a0 = 0.0, a1 = 0.0;
-    int t = 0;
-    for (; t + 1 < ns; t += 2) {
-      const size_t o0 = (size_t)S.slice(t) * 64, o1 = (size_t)S.slice(t + 1) * 64;
-      a0 += (double)v[o0] * (double)w[o0];
-      a1 += (double)v[o1] * (double)w[o1];
-    }
-    for (; t < ns; t++) {
-      const size_t o = (size_t)S.slice(t) * 64;
-      a0 += (double)v[o] * (double)w[o];
-    }
-    const double d = wave_sum(a0 + a1);
-    if (lane == 0) A.partials[(size_t)i * G + pb] = d;
+  const VT* w = V + (size_t)(j + 1) * A.ldv;
+  double acc[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; q++) acc[q] = 0.0;
+  for (int sl = S.first(wv); sl < S.end; sl += S.step) {
+    double b[4];
+    slot_rows(w + (size_t)sl * 64, lane >> 2, b);
+    dots_slice<0, NQ>(V + (size_t)sl * 64, A.ldv, j, lane, b, acc);
   }
+  dots_finish<NQ>(acc, j, G, pb, A.partials);
 }
 
-__global__ void __launch_bounds__(SB) k_dots_sell(SolveArgs A, int j) {
+template <int NQ>
+__global__ void __launch_bounds__(OPB, 4) k_dots_sell(SolveArgs A, int j) {
   if (A.stat->stop) return;
-  const SliceSet S = block_slices((A.n + 63) >> 6);
+  const SliceSet S = block_slices((A.n + 63) >> 6, blockIdx.x, gridDim.x, blockDim.x >> 6);
   if (A.v32)
-    dots_body<float>(A, j, S, blockIdx.x, gridDim.x);
+    dots_body<NQ, float>(A, j, S, blockIdx.x, gridDim.x);
   else
-    dots_body<double>(A, j, S, blockIdx.x, gridDim.x);
+    dots_body<NQ, double>(A, j, S, blockIdx.x, gridDim.x);
 }
+
+// the instance of a dots kernel with the fewest quads for the vectors i <= j
+// (a step between instances costs at most 12 vectors' worth of repeated,
+// cached loads)
+#define DOTS_KERNEL(k, j)                                                     \
+  ((j) < 4 ? k<1> : (j) < 8 ? k<2> : (j) < 16 ? k<4> : (j) < 24 ? k<6>        \
+   : (j) < 32 ? k<8> : (j) < 40 ? k<10> : (j) < 52 ? k<13> : k<16>)
 
 // GS-smoothed operator (precon 3, lss_mkb_core.c:2001-2054): with
 // X = s_j V_j, w = X - GS(X; b = 0); the sweeps run in place on w
@@ -486,16 +622,24 @@ __global__ void __launch_bounds__(SB) k_fin_dots(SolveArgs A, int j, int G) {
 // rows are updated in groups of W consecutive rows per lane (16-byte
 // loads): W = 2 for the FP64 basis, 4 for the FP32 one
 template <typename VT> struct Grp;
-template <> struct Grp<double> { using T = double2; static constexpr int W = 2; };
-template <> struct Grp<float> { using T = float4; static constexpr int W = 4; };
+template <> struct Grp<double> {
+  typedef double T __attribute__((ext_vector_type(2)));
+  static constexpr int W = 2;
+};
+template <> struct Grp<float> {
+  typedef float T __attribute__((ext_vector_type(4)));
+  static constexpr int W = 4;
+};
 
-// block r of G of a member updates the row groups [r g / G, (r+1) g / G)
-// cs: the coefficients c_i, i <= j, in shared memory (visible to the block)
-template <typename VT>
+// block r of G of a member updates the row groups [r g / G, (r+1) g / G).
+// coef() makes the coefficients c_i, i <= j, visible to the block in cs; the
+// thread's w and first eight vectors are requested before it, and eight
+// vectors ahead from then on.  halt: nothing to do (tested after the requests)
+template <typename VT, class Coefs>
 __device__ __forceinline__ void update_body(const SolveArgs& A, int j, int r, int G, int pb,
-                                            const double* cs) {
+                                            const double* cs, int halt, Coefs coef) {
   using GT = typename Grp<VT>::T;
-  constexpr int W = Grp<VT>::W;
+  constexpr int W = Grp<VT>::W, N = 8;
   __shared__ double red[1];
   const long long ng = (A.n + W - 1) / W;  // ldv is a multiple of W: whole groups stay inside
   const long long p0 = r * ng / G, p1 = (r + 1) * ng / G;
@@ -503,102 +647,112 @@ __device__ __forceinline__ void update_body(const SolveArgs& A, int j, int r, in
   const GT* VG = reinterpret_cast<const GT*>(basis<VT>(A));
   GT* w = reinterpret_cast<GT*>(basis<VT>(A) + (size_t)(j + 1) * A.ldv);
   double acc = 0.0;
-  for (long long p = p0 + threadIdx.x; p < p1; p += SB) {
-    const GT w0 = w[p];
+  auto load = [&](long long p, GT& w0, GT (&v)[N]) {
+    w0 = w[p];
+#pragma unroll
+    for (int q = 0; q < N; q++) v[q] = VG[(size_t)min(q, j) * ldg + p];
+  };
+  auto rows = [&](long long p, const GT& w0, GT (&v)[N]) {
     double wv[W];
 #pragma unroll
-    for (int e = 0; e < W; e++) wv[e] = (double)reinterpret_cast<const VT*>(&w0)[e];
-    int i = 0;
-    for (; i + 7 <= j; i += 8) {
-      GT v[8];
+    for (int e = 0; e < W; e++) wv[e] = (double)w0[e];
+    for (int i = 0; i <= j; i += N) {
+      GT u[N];
 #pragma unroll
-      for (int q = 0; q < 8; q++) v[q] = VG[(size_t)(i + q) * ldg + p];
+      for (int q = 0; q < N; q++) u[q] = v[q];
+      if (i + N <= j)
 #pragma unroll
-      for (int q = 0; q < 8; q++)
+        for (int q = 0; q < N; q++) v[q] = VG[(size_t)min(i + N + q, j) * ldg + p];
 #pragma unroll
-        for (int e = 0; e < W; e++) wv[e] -= cs[i + q] * (double)reinterpret_cast<const VT*>(&v[q])[e];
-    }
-    for (; i <= j; i++) {
-      const GT v = VG[(size_t)i * ldg + p];
+      for (int q = 0; q < N; q++)
+        if (i + q <= j)
 #pragma unroll
-      for (int e = 0; e < W; e++) wv[e] -= cs[i] * (double)reinterpret_cast<const VT*>(&v)[e];
+          for (int e = 0; e < W; e++) wv[e] -= cs[i + q] * (double)u[q][e];
     }
     GT wr;
 #pragma unroll
     for (int e = 0; e < W; e++) {
       const VT q = W * p + e < A.n ? (VT)wv[e] : (VT)0;  // padding rows stay zero
-      reinterpret_cast<VT*>(&wr)[e] = q;
+      wr[e] = q;
       acc += (double)q * (double)q;
     }
     w[p] = wr;
+  };
+  // the first rows apart from the others: with their request carried through
+  // the loop the compiler (ROCm 7.2) overwrote half of a sum with the index
+  long long p = p0 + threadIdx.x;
+  GT w0 = 0, v[N];
+#pragma unroll
+  for (int q = 0; q < N; q++) v[q] = 0;
+  if (p < p1) load(p, w0, v);
+  if (halt) return;
+  coef();
+  if (p < p1) rows(p, w0, v);
+  for (p += SB; p < p1; p += SB) {
+    GT w1, v1[N];
+    load(p, w1, v1);
+    rows(p, w1, v1);
   }
   block_sum_multi<1>(&acc, 1, red);
-  if (threadIdx.x == 0) A.partials[pb] = red[0];
+  if (threadIdx.x == 0) A.norms[pb] = red[0];
 }
 
-__device__ __forceinline__ void update_any(const SolveArgs& A, int j, int r, int G, int pb,
-                                           const double* cs) {
-  if (A.v32)
-    update_body<float>(A, j, r, G, pb, cs);
-  else
-    update_body<double>(A, j, r, G, pb, cs);
-}
-
-__global__ void __launch_bounds__(SB) k_update(SolveArgs A, int j) {
-  if (A.stat->stop) return;
-  __shared__ double cs[MAX_NV];
-  if ((int)threadIdx.x <= j) cs[threadIdx.x] = Coef(A)[threadIdx.x];
-  __syncthreads();
-  const int lb = xcd_block(blockIdx.x, gridDim.x);
-  update_any(A, j, lb, gridDim.x, lb, cs);
-}
-
-// h_{j+1,j} = ||w||, Givens rotations (drot/drotg as lss_mkb_core.c:2539-2560),
-// stopping tests (:2562-2590)
-__device__ __forceinline__ void fin_update_body(const SolveArgs& A, int j, int G) {
-  __shared__ double red[1];
-  __shared__ double col[MAX_NV + 1], giv[2 * MAX_NV], g2[2];
-  double s = 0.0;
-  for (int b = threadIdx.x; b < G; b += SB) s += A.partials[b];
-  double* hc = Hcol(A, j + 1);
-  double* gv = Giv(A);
-  if ((int)threadIdx.x <= j) col[threadIdx.x] = hc[threadIdx.x];
-  if ((int)threadIdx.x < 2 * j) giv[threadIdx.x] = gv[threadIdx.x];
-  block_sum_multi<1>(&s, 1, red);
-  if (threadIdx.x == 0) {
-    const int m = A.m;
-    const double hn = sqrt(red[0]);
-    col[j + 1] = hn;
-    Scale(A)[j + 1] = 1.0 / hn;
-    for (int i = 1; i <= j; i++) rot(&col[i - 1], &col[i], giv[2 * (i - 1)], giv[2 * (i - 1) + 1]);
-    double ra = col[j], rb = col[j + 1], c, sn;
-    drotg_dev(&ra, &rb, &c, &sn);
-    gv[2 * j] = c;
-    gv[2 * j + 1] = sn;
-    rot(&col[j], &col[j + 1], c, sn);
-    double* g = Hcol(A, 0);
-    g2[0] = g[j];
-    g2[1] = g[j + 1];
-    rot(&g2[0], &g2[1], c, sn);
-    g[j] = g2[0];
-    g[j + 1] = g2[1];
-    GmresStat* st = A.stat;
-    st->gmiter += 1;
-    st->j_done = j + 1;
-    st->resid = fabs(g2[1]);
-    st->res_rel = st->beta0 != 0.0 ? st->resid / st->beta0 : 0.0;
-    if (st->resid < st->tol_res || st->res_rel < st->tol_rel) {
-      st->converged = 1;
-      st->stop = 1;
+// the coefficients c_i = s_i h_i, h_i = s_i sum_b partials[i][b], i <= j, of
+// an update into cs, by every block for itself: 2^k threads per vector, one
+// exchange tree per wave.  write: this block keeps H's column
+__device__ __forceinline__ void fin_dots_all(const SolveArgs& A, int j, int G, bool write,
+                                             double* cs) {
+  int T = 64;
+  while (T * (j + 1) > SB) T >>= 1;
+  const int i = threadIdx.x / T, t = threadIdx.x % T;
+  if (i <= j) {
+    const double* p = A.partials + (size_t)i * G;
+    const double si = Scale(A)[i];
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    int b = t;
+    for (; b + 3 * T < G; b += 4 * T) {
+      s0 += p[b];
+      s1 += p[b + T];
+      s2 += p[b + 2 * T];
+      s3 += p[b + 3 * T];
     }
-    if (j + 1 == m || st->gmiter == st->max_iter) st->stop = 1;
-    if (A.hstat) *A.hstat = *st;
+    for (; b < G; b += T) s0 += p[b];
+    double s = (s0 + s1) + (s2 + s3);
+    for (int o = T >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (t == 0) {
+      const double h = si * s;
+      cs[i] = h * si;
+      if (write) Hcol(A, j + 1)[i] = h;
+    }
   }
   __syncthreads();
-  if ((int)threadIdx.x <= j + 1) hc[threadIdx.x] = col[threadIdx.x];
 }
 
-__global__ void __launch_bounds__(SB) k_fin_update(SolveArgs A, int j, int G) {
+template <class Coefs>
+__device__ __forceinline__ void update_any(const SolveArgs& A, int j, int r, int G, int pb,
+                                           const double* cs, int halt, Coefs coef) {
+  if (A.v32)
+    update_body<float>(A, j, r, G, pb, cs, halt, coef);
+  else
+    update_body<double>(A, j, r, G, pb, cs, halt, coef);
+}
+
+// G > 0: the blocks reduce the G partial dots themselves; 0: k_fin_dots did
+__global__ void __launch_bounds__(SB) k_update(SolveArgs A, int j, int G) {
+  const int halt = A.stat->stop;
+  __shared__ double cs[MAX_NV];
+  const int lb = xcd_block_rev(blockIdx.x, gridDim.x);
+  update_any(A, j, lb, gridDim.x, lb, cs, halt, [&]() {
+    if (G > 0) {
+      fin_dots_all(A, j, G, lb == 0, cs);
+    } else {
+      if ((int)threadIdx.x <= j) cs[threadIdx.x] = Coef(A)[threadIdx.x];
+      __syncthreads();
+    }
+  });
+}
+
+__global__ void __launch_bounds__(OPB) k_fin_update(SolveArgs A, int j, int G) {
   if (A.stat->stop) return;
   fin_update_body(A, j, G);
 }
@@ -702,6 +856,8 @@ __global__ void k_diag_ptr(int n, const int* rp, const int* col, int* dp) {
 // ---------------------------------------------------------------------
 static long long ldv_of(int n) { return ((long long)n + 63) / 64 * 64; }
 
+static size_t partials_row(const Problem& P);
+
 static void fill_solve_args(Problem& P, SolveArgs& A, int precon, int m) {
   A.n = P.n; A.ntiles = P.ntiles; A.m = m; A.ldv = ldv_of(P.n);
   A.tile_row = P.d_tile_row; A.row_ptr = P.d_row_ptr; A.col = P.d_col; A.val = P.d_val;
@@ -709,6 +865,7 @@ static void fill_solve_args(Problem& P, SolveArgs& A, int precon, int m) {
   A.val32 = P.d_val32; A.op32 = 0;
   A.dinv = precon ? P.d_dinv : nullptr;
   A.b = P.d_rhs; A.x = P.d_x; A.V = P.d_V; A.H = P.d_H; A.partials = P.d_partials;
+  A.norms = P.d_partials ? P.d_partials + (MAX_NV - 1) * partials_row(P) : nullptr;
   A.stat = P.d_stat; A.hstat = P.h_stat;
   A.Vf = reinterpret_cast<float*>(P.d_V); A.dinv32 = nullptr; A.v32 = 0; A.ilu = 0;
   A.scol16 = P.d_scol16; A.sbase = P.d_sbase;
@@ -719,20 +876,34 @@ static void fill_solve_args(Problem& P, SolveArgs& A, int precon, int m) {
 static int grid_tiles(const Problem& P) {
   return std::max(1, std::min(P.ntiles, std::min(MAX_BLOCKS, num_cus() * 5)));
 }
-// at most MAX_SLICES slices per block: the op kernel stages their w in LDS
-constexpr int MAX_SLICES = 32;
 static int grid_slices(const Problem& P) {
   const int nsl = (P.n + 63) / 64;
-  const int want = std::max(num_cus() * 8, (nsl + MAX_SLICES - 1) / MAX_SLICES);
-  return std::max(1, std::min((nsl + SW - 1) / SW, want));
+  return std::max(1, std::min((nsl + SW - 1) / SW, num_cus() * 8));
 }
-static size_t op_lds_bytes(int n, int G) {
-  // a block holds <= SW * ceil(part / (nq*SW)) slices, part <= ceil(nsl/nx)
-  // the XCD's share and nq >= floor(G/nx) its blocks
-  const int nsl = (n + 63) / 64;
-  const int nx = G < 8 ? G : 8;
-  const int part = (nsl + nx - 1) / nx + 1, nq = G / nx;
-  return (size_t)(SW * ((part + nq * SW - 1) / (nq * SW))) * 64 * sizeof(double);
+// blocks and wavefronts per block of the operator + dots kernels: one slice
+// per wavefront in blocks that spread a small system over all CUs (a CU's
+// address unit serves its wavefronts one after the other: 19 blocks of 8
+// waves took twice as long as 145 of one), at most 4 blocks of 8 per CU
+struct OpGrid {
+  int G, W;
+  bool one;  // the launch has a slice per wavefront and is resident at once
+};
+static OpGrid grid_op(const Problem& P) {
+  const int nsl = (P.n + 63) / 64, cu = num_cus();
+  OpGrid g{1, 1, nsl <= 8 * cu};
+  while (g.W < OPB / 64 && nsl > g.W * cu) g.W *= 2;
+  g.G = std::max(1, std::min((nsl + g.W - 1) / g.W, cu * 4));
+  return g;
+}
+// largest number of dot partials per vector that every block of the update
+// reduces for itself (a launch less: 2.4 us); above it k_fin_dots reduces
+// them once (4.7 us for 1024 partials of up to 50 vectors, which every one of
+// 2048 blocks would read as 400 KB)
+constexpr int kFuseDots = 512;
+// doubles of one row of the partials buffer (MAX_NV rows; the last holds the
+// norms of the updates)
+static size_t partials_row(const Problem& P) {
+  return std::max<size_t>(MAX_BLOCKS, (size_t)grid_slices(P));
 }
 static int grid_rows(const Problem& P) {
   long long pairs = (P.n + 1) / 2;
@@ -956,8 +1127,7 @@ static int ensure_workspace(Problem& P, int m) {
   MF_HIP(hipMemset(P.d_V, 0, (size_t)(m + 1) * ldv * sizeof(double)));
   MF_HIP(hipMalloc(&P.d_H, (size_t)((m + 1) * (m + 1) + 4 * (m + 1)) * sizeof(double)));
   if (!P.d_partials) {
-    const size_t G = std::max<size_t>(MAX_BLOCKS, (size_t)grid_slices(P));
-    MF_HIP(hipMalloc(&P.d_partials, G * MAX_NV * sizeof(double)));
+    MF_HIP(hipMalloc(&P.d_partials, partials_row(P) * MAX_NV * sizeof(double)));
   }
   if (!P.d_stat) MF_HIP(hipMalloc(&P.d_stat, sizeof(GmresStat)));
   if (!P.h_stat) MF_HIP(hipHostMalloc(&P.h_stat, sizeof(GmresStat), hipHostMallocDefault));
@@ -990,50 +1160,84 @@ static int zero_padding(const Problem& P, int m, int v32) {
   return 0;
 }
 
-template <int NV>
-static void launch_step(int G_op, int G_up, SolveArgs& A, int j) {
+// the Gram-Schmidt half of step j after the dots: the coefficients and the
+// update of w, whose norm is finished by fin_step or the next operator launch
+static void launch_update(int G_op, int G_up, const SolveArgs& A, int j) {
   hipStream_t s = stream();
-  hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr, e3 = nullptr;
+  const bool fuse = G_op <= kFuseDots;
+  if (!fuse) hipLaunchKernelGGL(k_fin_dots, dim3(j + 1), dim3(SB), 0, s, A, j, G_op);
+  hipEvent_t e0 = nullptr, e1 = nullptr;
   if (g_ks.on) {
     e0 = ks_event(); e1 = ks_event();
     (void)hipEventRecord(e0, s);
   }
-  if (A.sl_ptr)
-    hipLaunchKernelGGL(k_op_dots_sell, dim3(G_op), dim3(SB), op_lds_bytes(A.n, G_op), s, A, j);
-  else
-    hipLaunchKernelGGL(k_op_dots<NV>, dim3(G_op), dim3(SB), 0, s, A, j);
-  if (g_ks.on) (void)hipEventRecord(e1, s);
-  hipLaunchKernelGGL(k_fin_dots, dim3(j + 1), dim3(SB), 0, s, A, j, G_op);
+  hipLaunchKernelGGL(k_update, dim3(G_up), dim3(SB), 0, s, A, j, fuse ? G_op : 0);
   if (g_ks.on) {
-    e2 = ks_event(); e3 = ks_event();
-    (void)hipEventRecord(e2, s);
-  }
-  hipLaunchKernelGGL(k_update, dim3(G_up), dim3(SB), 0, s, A, j);
-  if (g_ks.on) (void)hipEventRecord(e3, s);
-  hipLaunchKernelGGL(k_fin_update, dim3(1), dim3(SB), 0, s, A, j, G_up);
-  if (g_ks.on) {
-    // algorithmic bytes: op = CRS values+columns, row pointers, input
-    // vector, Jacobi diagonal, output, and V_0..V_{j-1} for the dots;
-    // update = w read+write and V_0..V_j
-    const double n = A.n;
-    g_ks.kind.push_back(0);
-    g_ks.step.push_back(j);
-    g_ks.bytes.push_back(-1.0);  // set by the caller (needs nnz)
+    (void)hipEventRecord(e1, s);
+    // algorithmic bytes: w read and written, V_0..V_j
     g_ks.kind.push_back(1);
     g_ks.step.push_back(j);
-    g_ks.bytes.push_back(8.0 * n * (j + 3));
+    g_ks.bytes.push_back(8.0 * A.n * (j + 3));
   }
 }
 
-static void launch_arnoldi(int G_op, int G_up, SolveArgs& A, int j) {
-  int nv = j + 1;
-  if (nv <= 8) launch_step<8>(G_op, G_up, A, j);
-  else if (nv <= 16) launch_step<16>(G_op, G_up, A, j);
-  else if (nv <= 24) launch_step<24>(G_op, G_up, A, j);
-  else if (nv <= 32) launch_step<32>(G_op, G_up, A, j);
-  else if (nv <= 40) launch_step<40>(G_op, G_up, A, j);
-  else if (nv <= 48) launch_step<48>(G_op, G_up, A, j);
-  else launch_step<64>(G_op, G_up, A, j);
+static void fin_step(int G_up, const SolveArgs& A, int j) {
+  hipLaunchKernelGGL(k_fin_update, dim3(1), dim3(OPB), 0, stream(), A, j, G_up);
+}
+
+template <int NV>
+static void launch_op_dots_crs(int G_op, const SolveArgs& A, int j) {
+  hipLaunchKernelGGL(k_op_dots<NV>, dim3(G_op), dim3(SB), 0, stream(), A, j);
+}
+
+// Arnoldi step j of an unpreconditioned or Jacobi-preconditioned system.  In
+// SELL storage a step is two launches: the operator's finishes the step
+// before it, the update's reduces the dots (large grids: a third launch
+// does); the last step of a cycle is finished by itself.
+static void launch_arnoldi(const OpGrid& op, int G_up, const SolveArgs& A, int j) {
+  hipStream_t s = stream();
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  if (g_ks.on) {
+    e0 = ks_event(); e1 = ks_event();
+    (void)hipEventRecord(e0, s);
+  }
+  if (A.sl_ptr) {
+    auto k = op.one ? DOTS_KERNEL(k_op_dots_one, j) : DOTS_KERNEL(k_op_dots_sell, j);
+    hipLaunchKernelGGL(k, dim3(op.G + (j > 0 ? kFinBlocks : 0)), dim3(64 * op.W), 0, s, A, j, op.G, G_up);
+  } else {
+    const int nv = j + 1;
+    if (nv <= 8) launch_op_dots_crs<8>(op.G, A, j);
+    else if (nv <= 16) launch_op_dots_crs<16>(op.G, A, j);
+    else if (nv <= 24) launch_op_dots_crs<24>(op.G, A, j);
+    else if (nv <= 32) launch_op_dots_crs<32>(op.G, A, j);
+    else if (nv <= 40) launch_op_dots_crs<40>(op.G, A, j);
+    else if (nv <= 48) launch_op_dots_crs<48>(op.G, A, j);
+    else launch_op_dots_crs<64>(op.G, A, j);
+  }
+  if (g_ks.on) {
+    (void)hipEventRecord(e1, s);
+    // algorithmic bytes: CRS values+columns, row pointers, input vector,
+    // Jacobi diagonal, output, and V_0..V_{j-1} for the dots; set by the
+    // caller (needs nnz)
+    g_ks.kind.push_back(0);
+    g_ks.step.push_back(j);
+    g_ks.bytes.push_back(-1.0);
+  }
+  launch_update(op.G, G_up, A, j);
+  if (!A.sl_ptr || j + 1 == A.m) fin_step(G_up, A, j);
+}
+
+// The host enqueues a cycle ahead of the device, but not further than `ahead`
+// steps past the last finished one (read from the pinned status): when the
+// stopping test is met early, only those steps' launches run empty.  Returns
+// false once the cycle has stopped.  Without the mirror the whole cycle is
+// enqueued; a stream that has run dry ends the wait.
+static bool step_wanted(const GmresStat* h, int j, int ahead) {
+  if (!h) return true;
+  const volatile GmresStat* st = h;
+  for (int spin = 0; !st->stop && j - st->j_done > ahead; spin++)
+    if (spin % 4096 == 4095 && hipStreamQuery(stream()) != hipErrorNotReady) break;
+  return !st->stop;
 }
 
 // Restarted left-preconditioned GMRES(m), classical Gram-Schmidt and Givens
@@ -1116,7 +1320,9 @@ static int gmres_core(Problem& P, int precon, int krylbas, int max_iter, double 
     A.dinv = nullptr;
   }
   if (P.sell && zero_padding(P, m, A.v32)) return -2;
-  const int G_op = (P.sell || ext) ? grid_slices(P) : grid_tiles(P), G_up = grid_rows(P);
+  const bool slices = P.sell || ext;
+  const OpGrid op = slices ? grid_op(P) : OpGrid{grid_tiles(P), SB / 64, false};
+  const int G_up = grid_rows(P), G_res = slices ? grid_slices(P) : op.G;
   const double* d_scale = P.d_H + (size_t)(m + 1) * (m + 1) + 2 * (m + 1);
   if (!P.sell) A.sl_ptr = nullptr;
   hipStream_t s = stream();
@@ -1163,23 +1369,23 @@ static int gmres_core(Problem& P, int precon, int krylbas, int max_iter, double 
     MF_HIP(hipMemcpyAsync(P.d_stat, &st, sizeof(GmresStat), hipMemcpyHostToDevice, s));
     if (ext) {
       if (P.ext->residual(A.b, A.x, A.V)) return -2;
-      hipLaunchKernelGGL(k_sumsq_v0, dim3(G_op), dim3(SB), 0, s, A);
+      hipLaunchKernelGGL(k_sumsq_v0, dim3(G_res), dim3(SB), 0, s, A);
     } else if (gs) {
       // V_0 = GS_k(x; b) - x (the smoothing branch, lss_mkb_core.c:2001-2054)
       MF_HIP(hipMemcpyAsync(A.V, A.x, (size_t)P.n * sizeof(double), hipMemcpyDeviceToDevice, s));
       if (gs_sweeps(P, P.gs_sweeps, A.b, A.V, nullptr)) return -2;
       hipLaunchKernelGGL(k_gs_restart_finish, dim3(gn), dim3(256), 0, s, A);
-      hipLaunchKernelGGL(k_sumsq_v0, dim3(G_op), dim3(SB), 0, s, A);
+      hipLaunchKernelGGL(k_sumsq_v0, dim3(G_res), dim3(SB), 0, s, A);
     } else if (P.sell)
-      hipLaunchKernelGGL(k_residual_sell, dim3(G_op), dim3(SB), 0, s, A);
+      hipLaunchKernelGGL(k_residual_sell, dim3(G_res), dim3(SB), 0, s, A);
     else
-      hipLaunchKernelGGL(k_residual, dim3(G_op), dim3(SB), 0, s, A);
+      hipLaunchKernelGGL(k_residual, dim3(G_res), dim3(SB), 0, s, A);
     if (ilu) {
       // V_0 = (LU)^-1 (b - A x), lss_mkb_core.c:1953-1977
       if (A.v32 ? ilu_apply32(P, A.Vf, A.Vf, nullptr) : ilu_apply(P, A.V, A.V, nullptr)) return -2;
-      hipLaunchKernelGGL(k_sumsq_v0, dim3(G_op), dim3(SB), 0, s, A);
+      hipLaunchKernelGGL(k_sumsq_v0, dim3(G_res), dim3(SB), 0, s, A);
     }
-    hipLaunchKernelGGL(k_fin_residual, dim3(1), dim3(SB), 0, s, A, G_op);
+    hipLaunchKernelGGL(k_fin_residual, dim3(1), dim3(SB), 0, s, A, G_res);
     MF_HIP(hipGetLastError());
     MF_HIP(hipStreamSynchronize(s));
     GmresStat rs{};
@@ -1217,7 +1423,7 @@ static int gmres_core(Problem& P, int precon, int krylbas, int max_iter, double 
     MF_HIP(hipMemcpyAsync(P.d_H, H, Hn * sizeof(double), hipMemcpyHostToDevice, s));
     MF_HIP(hipMemcpyAsync(P.d_stat, &st, sizeof(GmresStat), hipMemcpyHostToDevice, s));
     if (ilu || gs || ext) {
-      for (int j = 0; j < m; j++) {
+      for (int j = 0; j < m && step_wanted(A.hstat, j, 2); j++) {
         double* w = A.V + (size_t)(j + 1) * A.ldv;
         if (ext) {
           if (P.ext->apply(A.V + (size_t)j * A.ldv, d_scale, j, w, d_stop)) return -2;
@@ -1226,17 +1432,16 @@ static int gmres_core(Problem& P, int precon, int krylbas, int max_iter, double 
           if (gs_sweeps(P, P.gs_sweeps, nullptr, w, d_stop)) return -2;
           hipLaunchKernelGGL(k_gs_op_finish, dim3(gn), dim3(256), 0, s, A, j);
         } else {
-          hipLaunchKernelGGL(k_op_sell, dim3(G_op), dim3(SB), 0, s, A, j);
+          hipLaunchKernelGGL(k_op_sell, dim3(op.G), dim3(64 * op.W), 0, s, A, j);
           float* wf = A.Vf + (size_t)(j + 1) * A.ldv;
           if (A.v32 ? ilu_apply32(P, wf, wf, d_stop) : ilu_apply(P, w, w, d_stop)) return -2;
         }
-        hipLaunchKernelGGL(k_dots_sell, dim3(G_op), dim3(SB), 0, s, A, j);
-        hipLaunchKernelGGL(k_fin_dots, dim3(j + 1), dim3(SB), 0, s, A, j, G_op);
-        hipLaunchKernelGGL(k_update, dim3(G_up), dim3(SB), 0, s, A, j);
-        hipLaunchKernelGGL(k_fin_update, dim3(1), dim3(SB), 0, s, A, j, G_up);
+        hipLaunchKernelGGL(DOTS_KERNEL(k_dots_sell, j), dim3(op.G), dim3(64 * op.W), 0, s, A, j);
+        launch_update(op.G, G_up, A, j);
+        fin_step(G_up, A, j);
       }
     } else {
-      for (int j = 0; j < m; j++) launch_arnoldi(G_op, G_up, A, j);
+      for (int j = 0; j < m && step_wanted(A.hstat, j, 6); j++) launch_arnoldi(op, G_up, A, j);
     }
     MF_HIP(hipGetLastError());
     MF_HIP(hipMemcpyAsync(H, P.d_H, Hn * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -1472,7 +1677,7 @@ __global__ void k_scatter_perm(int n, const int* __restrict__ perm, const double
 static size_t noalloc_doubles(const Problem& P, int m) {
   auto up = [](size_t d) { return (d + 31) / 32 * 32; };
   const size_t ldv = (size_t)ldv_of(P.n);
-  const size_t G = std::max<size_t>(MAX_BLOCKS, (size_t)grid_slices(P));
+  const size_t G = partials_row(P);
   return up(ldv) * 3                                   // reference x, device x, Jacobi
          + up(((size_t)P.n + 1) / 2)                   // row permutation (int)
          + up(G * MAX_NV)                              // dot-product partials
@@ -1511,7 +1716,7 @@ int gmres_noalloc(Problem& P, int precon, int krylbas, int max_iter, double tol,
   }
   auto up = [](size_t d) { return (d + 31) / 32 * 32; };
   const size_t ldv = (size_t)ldv_of(P.n);
-  const size_t G = std::max<size_t>(MAX_BLOCKS, (size_t)grid_slices(P));
+  const size_t G = partials_row(P);
   double* q = base;
   double* xr = q; q += up(ldv);
   double* xd = q; q += up(ldv);
@@ -1710,30 +1915,52 @@ __global__ void __launch_bounds__(SB) kb_ilu_level(BatchArgs B, const IluMember*
   }
 }
 
-__global__ void __launch_bounds__(SB) kb_op_dots(BatchArgs B, int j) {
-  const int p = B.blk_prob[blockIdx.x], r = B.blk_rank[blockIdx.x], G = B.nblk[p];
+// A batch without ILU members finishes step j - 1 inside the operator launch
+// of step j (fin): block p < nfin finishes member p, and a member's blocks
+// form its norm themselves (as k_op_dots_sell does).  A member that ended
+// before the cycle has done set; a stop found in this launch (stop = j) takes
+// effect at the next one.
+template <int NQ>
+__global__ void __launch_bounds__(SB, 4) kb_op_dots(BatchArgs B, int j, int nfin, int fin) {
+  if ((int)blockIdx.x < nfin) {
+    const int p = blockIdx.x;
+    const SolveArgs A = B.args[p];
+    const int stop = A.stat->stop;
+    if (!A.stat->done && (stop == 0 || stop >= j)) fin_update_body(A, j - 1, B.nblk[p]);
+    return;
+  }
+  const int bid = blockIdx.x - nfin;
+  const int p = B.blk_prob[bid], r = B.blk_rank[bid], G = B.nblk[p];
   const SolveArgs A = B.args[p];
-  if (A.stat->stop) return;
-  extern __shared__ double ws[];
+  const int stop = A.stat->stop;
+  if (fin ? A.stat->done || (stop && stop < j) : stop != 0) return;
   const SliceSet S = member_slices(A.n, r, G);
-  if (!A.ilu)
-    op_dots_any(A, j, S, r, G, ws);
-  else if (A.v32)
-    op_body<float>(A, j, S);  // dots after the substitution (kb_dots)
-  else
-    op_body<double>(A, j, S);
+  if (A.ilu) {  // dots after the substitution (kb_dots)
+    if (A.v32)
+      op_body<float>(A, j, S);
+    else
+      op_body<double>(A, j, S);
+    return;
+  }
+  double q = 0.0;
+  if (fin && j > 0)
+    for (int b = threadIdx.x; b < G; b += SB) q += A.norms[b];
+  op_dots_any<NQ, false>(A, j, S, r, G, [&]() {
+    return fin && j > 0 ? 1.0 / sqrt(block_sum_all(q)) : Scale(A)[j];
+  });
 }
 
 // ILU members: Gram-Schmidt dots with the preconditioned w
-__global__ void __launch_bounds__(SB) kb_dots(BatchArgs B, int j) {
+template <int NQ>
+__global__ void __launch_bounds__(SB, 4) kb_dots(BatchArgs B, int j) {
   const int p = B.blk_prob[blockIdx.x], r = B.blk_rank[blockIdx.x], G = B.nblk[p];
   const SolveArgs A = B.args[p];
   if (!A.ilu || A.stat->stop) return;
   const SliceSet S = member_slices(A.n, r, G);
   if (A.v32)
-    dots_body<float>(A, j, S, r, G);
+    dots_body<NQ, float>(A, j, S, r, G);
   else
-    dots_body<double>(A, j, S, r, G);
+    dots_body<NQ, double>(A, j, S, r, G);
 }
 
 __global__ void __launch_bounds__(SB) kb_fin_dots(BatchArgs B, int j) {
@@ -1742,14 +1969,18 @@ __global__ void __launch_bounds__(SB) kb_fin_dots(BatchArgs B, int j) {
   fin_dots_body(A, j, blockIdx.x, B.nblk[blockIdx.y]);
 }
 
-__global__ void __launch_bounds__(SB) kb_update(BatchArgs B, int j) {
+__global__ void __launch_bounds__(SB) kb_update(BatchArgs B, int j, int fuse) {
   const int p = B.blk_prob[blockIdx.x], r = B.blk_rank[blockIdx.x], G = B.nblk[p];
   const SolveArgs A = B.args[p];
-  if (A.stat->stop) return;
   __shared__ double cs[MAX_NV];
-  if ((int)threadIdx.x <= j) cs[threadIdx.x] = Coef(A)[threadIdx.x];
-  __syncthreads();
-  update_any(A, j, r, G, r, cs);
+  update_any(A, j, r, G, r, cs, A.stat->stop, [&]() {
+    if (fuse) {
+      fin_dots_all(A, j, G, r == 0, cs);
+    } else {
+      if ((int)threadIdx.x <= j) cs[threadIdx.x] = Coef(A)[threadIdx.x];
+      __syncthreads();
+    }
+  });
 }
 
 __global__ void __launch_bounds__(SB) kb_fin_update(BatchArgs B, int j) {
@@ -2159,8 +2390,8 @@ static int batch_build(Batch& B) {
     }
   }
   B.nblk = (int)bp.size();
-  B.lds = (size_t)max_sl * 64 * sizeof(double);
-  if (B.lds > 64 * 1024) {
+  B.max_blk = np ? *std::max_element(nblk.begin(), nblk.end()) : 0;
+  if (max_sl > 128) {
     set_error("batch: a member is too large for the batched operator (> 33M rows)");
     return -1;
   }
@@ -2227,15 +2458,21 @@ static void batch_enqueue_cycle(Batch& B, hipStream_t s, bool refine = true) {
     hipLaunchKernelGGL(kb_sumsq, dim3(B.nblk), dim3(SB), 0, s, a);
   }
   hipLaunchKernelGGL(kb_restart, dim3(np), dim3(SB), 0, s, a);
+  // two launches a step: see k_op_dots_sell and k_update.  ILU members need
+  // s_j in memory before the operator, members of many blocks their dots
+  // reduced once
+  const int fin = !B.has_ilu, fuse = B.max_blk <= kFuseDots;
   for (int j = 0; j < B.m; j++) {
-    hipLaunchKernelGGL(kb_op_dots, dim3(B.nblk), dim3(SB), B.lds, s, a, j);
+    const int nfin = fin && j > 0 ? np : 0;
+    hipLaunchKernelGGL(DOTS_KERNEL(kb_op_dots, j), dim3(nfin + B.nblk), dim3(SB), 0, s, a, j, nfin,
+                       fin);
     if (B.has_ilu) {
       batch_ilu_levels(B, a, j, s);
-      hipLaunchKernelGGL(kb_dots, dim3(B.nblk), dim3(SB), 0, s, a, j);
+      hipLaunchKernelGGL(DOTS_KERNEL(kb_dots, j), dim3(B.nblk), dim3(SB), 0, s, a, j);
     }
-    hipLaunchKernelGGL(kb_fin_dots, dim3(j + 1, np), dim3(SB), 0, s, a, j);
-    hipLaunchKernelGGL(kb_update, dim3(B.nblk), dim3(SB), 0, s, a, j);
-    hipLaunchKernelGGL(kb_fin_update, dim3(np), dim3(SB), 0, s, a, j);
+    if (!fuse) hipLaunchKernelGGL(kb_fin_dots, dim3(j + 1, np), dim3(SB), 0, s, a, j);
+    hipLaunchKernelGGL(kb_update, dim3(B.nblk), dim3(SB), 0, s, a, j, fuse);
+    if (!fin || j + 1 == B.m) hipLaunchKernelGGL(kb_fin_update, dim3(np), dim3(SB), 0, s, a, j);
   }
   hipLaunchKernelGGL(kb_ysolve, dim3(np), dim3(64), 0, s, a);
   hipLaunchKernelGGL(kb_xupdate, dim3(B.nblk), dim3(SB), 0, s, a);

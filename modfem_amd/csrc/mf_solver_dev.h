@@ -14,6 +14,7 @@ constexpr int SB = 256;         // threads per solver block
 constexpr int TILE_NNZ = 4096;  // CRS entries staged per tile (32 KB LDS)
 constexpr int MAX_BLOCKS = 4096;
 constexpr int MAX_NV = 64;
+constexpr int OPB = 512;        // threads per block of the operator + dots kernels
 
 // ---------------------------------------------------------------------
 // device helpers
@@ -24,6 +25,13 @@ __device__ __forceinline__ int xcd_block(int bid, int nb) {
   int xcd = bid & 7, k = bid >> 3;
   int per = nb >> 3, rem = nb & 7;
   return xcd * per + min(xcd, rem) + k;
+}
+
+// the same ranges, taken from their ends backwards
+__device__ __forceinline__ int xcd_block_rev(int bid, int nb) {
+  const int xcd = bid & 7, k = bid >> 3;
+  const int per = nb >> 3, rem = nb & 7;
+  return xcd * per + min(xcd, rem) + per + (xcd < rem ? 1 : 0) - 1 - k;
 }
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -54,6 +62,18 @@ __device__ __forceinline__ void block_sum_multi(const double* acc, int nact, dou
   __syncthreads();
 }
 
+// sum of one value per thread over a block of up to OPB threads, the same in
+// every thread; the same number of threads gives the same rounding
+__device__ __forceinline__ double block_sum_all(double v) {
+  __shared__ double wsum[OPB / 64];
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double s = 0.0;
+  for (int w = 0; w < (int)(blockDim.x >> 6); w++) s += wsum[w];
+  return s;
+}
+
 struct SolveArgs {
   int n, ntiles, m;
   long long ldv;        // stride of the Krylov vectors
@@ -74,7 +94,8 @@ struct SolveArgs {
   double* x;
   double* V;            // (m+1) x ldv
   double* H;            // (m+1)^2 | givens 2(m+1) | scale (m+1) | coef (m+1)
-  double* partials;
+  double* partials;     // dot products V_i . w: [i][block]
+  double* norms;        // ||w||^2 of an update: [block]
   GmresStat* stat;
   GmresStat* hstat;     // pinned host mirror
   // mixed-precision inner solves: the Krylov basis and the Jacobi inverses
@@ -138,76 +159,235 @@ __device__ __forceinline__ void slice_range(int nsl, int lb, int& s0, int& s1) {
   s1 = (int)((long long)(lb + 1) * nsl / gridDim.x);
 }
 
-// The slices of one operator block, in order t = 0, 1, ...: XCD x owns the
-// x-th contiguous part of the slices and its blocks take steps of SW
-// consecutive slices cyclically, so each XCD sweeps one contiguous window of
+// The slices of one operator block: XCD x owns the x-th contiguous part of
+// the slices and its blocks take steps of W consecutive slices (one per
+// wavefront) cyclically, so each XCD sweeps one contiguous window of
 // the matrix at a time (measured 3% faster than a contiguous range per block,
 // which leaves ~2k streams open at scattered addresses).
 struct SliceSet {
   int base, step, end;
-  __device__ __forceinline__ int slice(int t) const { return base + (t / SW) * step + (t % SW); }
-  __device__ __forceinline__ int count() const {
-    if (end <= base) return 0;
-    const int full = (end - base) / step, rem = (end - base) % step;
-    return full * SW + min(rem, SW);
-  }
+  // the slices of wavefront w: first(w), first(w) + step, ... < end
+  __device__ __forceinline__ int first(int w) const { return base + w; }
 };
 
-__device__ __forceinline__ SliceSet block_slices(int nsl) {
+// block bid of G blocks of W wavefronts
+__device__ __forceinline__ SliceSet block_slices(int nsl, int bid, int G, int W) {
   SliceSet S;
-  const int G = gridDim.x;
   const int nx = G < 8 ? G : 8;
-  const int x = blockIdx.x % nx, q = blockIdx.x / nx;
+  const int x = bid % nx, q = bid / nx;
   const int nq = G / nx + (x < G % nx ? 1 : 0);
   const int r0 = (int)((long long)x * nsl / nx), r1 = (int)((long long)(x + 1) * nsl / nx);
-  S.base = r0 + q * SW;
-  S.step = nq * SW;
+  S.base = r0 + q * W;
+  S.step = nq * W;
   S.end = r1;
   return S;
 }
 
-// row sum of the calling lane's row: the slice's column indices and values
-// are loaded first (CH entries in flight per lane), then the vector gathers
-// are issued together, so a chunk costs about two memory round trips instead
-// of one per entry.  Every load is unconditional (indices past the slice's
-// length are clamped to its last entry and their products dropped by a
-// select), so the compiler keeps the loads of a chunk in flight together.
-template <typename VT, typename XT, int CH = 12>
-__device__ __forceinline__ double sell_row(const SolveArgs& A, const VT* val, const XT* x,
-                                           int sl, int lane) {
-  const long long base = A.sl_ptr[sl] + lane;
-  const int len = (int)((A.sl_ptr[sl + 1] - A.sl_ptr[sl]) >> 6);
-  // 16-bit columns where the slice has them (a wave-uniform test)
-  const int cb = A.sbase ? A.sbase[sl] : -1;
+// row sum of the calling lane's row.  The slice is the wavefront's, so its
+// offsets and its smallest column are scalars and a lane's addresses are one
+// 32-bit offset each; CH entries of the row are in flight while the CH before
+// them are gathered and summed (the first chunk costs two dependent trips to
+// memory, every further one a single trip).  Loads past the slice's length
+// repeat its last entry and their products are dropped by a select, so no
+// load waits for a branch.
+template <typename VT, int CH, typename CT>
+__device__ __forceinline__ void sell_chunk(const VT* val, const CT* col, int k0, int len, int lane,
+                                           int (&c)[CH], VT (&v)[CH]) {
+#pragma unroll
+  for (int k = 0; k < CH; k++) {
+    const int q = 64 * min(k0 + k, len - 1);
+    c[k] = (int)col[q + lane];
+    v[k] = val[q + lane];
+  }
+}
+
+template <typename VT, typename XT, int CH, typename CT>
+__device__ __forceinline__ double sell_row_cols(const VT* val, const CT* col, const XT* x, int len,
+                                                int lane) {
   double s = 0.0;
+  int c[CH];
+  VT v[CH];
+  if (len > 0) sell_chunk<VT, CH>(val, col, 0, len, lane, c, v);
   for (int k0 = 0; k0 < len; k0 += CH) {
-    int c[CH];
-    VT v[CH];
-    if (cb >= 0) {
-#pragma unroll
-      for (int k = 0; k < CH; k++) {
-        const long long q = base + 64LL * min(k0 + k, len - 1);
-        c[k] = cb + (int)A.scol16[q];
-        v[k] = val[q];
-      }
-    } else {
-#pragma unroll
-      for (int k = 0; k < CH; k++) {
-        const long long q = base + 64LL * min(k0 + k, len - 1);
-        c[k] = A.scol[q];
-        v[k] = val[q];
-      }
-    }
     XT xv[CH];
 #pragma unroll
-    for (int k = 0; k < CH; k++) xv[k] = x[c[k]];
+    for (int k = 0; k < CH; k++) xv[k] = x[(unsigned)c[k]];
+    VT w[CH];
+#pragma unroll
+    for (int k = 0; k < CH; k++) w[k] = v[k];
+    if (k0 + CH < len) sell_chunk<VT, CH>(val, col, k0 + CH, len, lane, c, v);
 #pragma unroll
     for (int k = 0; k < CH; k++) {
-      const double t = (double)v[k] * (double)xv[k];
+      const double t = (double)w[k] * (double)xv[k];
       s += k0 + k < len ? t : 0.0;
     }
   }
   return s;
+}
+
+constexpr int kSellChunk = 8;
+
+template <typename VT, typename XT, int CH = kSellChunk>
+__device__ __forceinline__ double sell_row(const SolveArgs& A, const VT* val, const XT* x,
+                                           int sl, int lane) {
+  sl = __builtin_amdgcn_readfirstlane(sl);
+  const long long base = A.sl_ptr[sl];
+  const int len = (int)((A.sl_ptr[sl + 1] - base) >> 6);
+  // 16-bit columns where the slice has them
+  const int cb = A.sbase ? A.sbase[sl] : -1;
+  if (cb >= 0)
+    return sell_row_cols<VT, XT, CH>(val + base, A.scol16 + base, x + cb, len, lane);
+  return sell_row_cols<VT, XT, CH>(val + base, A.scol + base, x, len, lane);
+}
+
+// the same row sum for a wavefront that has a single slice: a launch of one
+// round is bound by its chain of dependent loads, so up to kSellWide entries
+// are requested at once (two trips to memory for a row of a box mesh instead
+// of four); groups of four past the slice's length are skipped by a
+// wave-uniform test.  before(): loads to issue behind the first columns and
+// values
+constexpr int kSellWide = 28;
+
+template <typename VT, typename XT, typename CT, class Before>
+__device__ __forceinline__ double sell_row_one_cols(const VT* val, const CT* col, const XT* x,
+                                                    int len, int lane, Before before) {
+  double s = 0.0;
+  for (int k0 = 0; k0 < len; k0 += kSellWide) {
+    int c[kSellWide];
+    VT v[kSellWide];
+    XT xv[kSellWide];
+#pragma unroll
+    for (int g = 0; g < kSellWide; g += 4)
+      if (k0 + g < len)
+#pragma unroll
+        for (int k = g; k < g + 4; k++) {
+          const int q = 64 * min(k0 + k, len - 1);
+          c[k] = (int)col[q + lane];
+          v[k] = val[q + lane];
+        }
+    if (k0 == 0) before();
+#pragma unroll
+    for (int g = 0; g < kSellWide; g += 4)
+      if (k0 + g < len)
+#pragma unroll
+        for (int k = g; k < g + 4; k++) xv[k] = x[(unsigned)c[k]];
+#pragma unroll
+    for (int g = 0; g < kSellWide; g += 4)
+      if (k0 + g < len)
+#pragma unroll
+        for (int k = g; k < g + 4; k++) {
+          const double t = (double)v[k] * (double)xv[k];
+          s += k0 + k < len ? t : 0.0;
+        }
+  }
+  return s;
+}
+
+template <typename VT, typename XT, class Before>
+__device__ __forceinline__ double sell_row_one(const SolveArgs& A, const VT* val, const XT* x,
+                                               int sl, int lane, Before before) {
+  sl = __builtin_amdgcn_readfirstlane(sl);
+  const long long base = A.sl_ptr[sl];
+  const int len = (int)((A.sl_ptr[sl + 1] - base) >> 6);
+  const int cb = A.sbase ? A.sbase[sl] : -1;
+  if (cb >= 0)
+    return sell_row_one_cols(val + base, A.scol16 + base, x + cb, len, lane, before);
+  return sell_row_one_cols(val + base, A.scol + base, x, len, lane, before);
+}
+
+// ---------------------------------------------------------------------
+// Gram-Schmidt dot products V_i . w of a 64-row slice on the matrix cores:
+// v_mfma_f64_4x4x4 multiplies four 4 x 4 by 4 x 4 blocks; lane l holds row l % 4
+// (the vector) and, in block (l / 4) % 4, column l / 16 (the matrix row) of
+// the left operand, and the same place of the right one.  With V_{4q + l % 4}
+// and w at the rows of slot l / 4 in lane l, one instruction adds 16 rows of
+// four dot products to the accumulator, and nothing is exchanged between
+// lanes until the block's rows are done (dots_finish).  One wave-wide sum per
+// vector (six exchanges) made the dots half of a step on small systems.
+// ---------------------------------------------------------------------
+// entries of a vector at the rows of the lane's slot: FP64 rows 2s, 2s + 1
+// and 32 + 2s, 33 + 2s; FP32 rows 4s .. 4s + 3 (16-byte loads)
+__device__ __forceinline__ void slot_rows(const double* v, int slot, double (&r)[4]) {
+  const double2 a = *reinterpret_cast<const double2*>(v + 2 * slot);
+  const double2 b = *reinterpret_cast<const double2*>(v + 32 + 2 * slot);
+  r[0] = a.x; r[1] = a.y; r[2] = b.x; r[3] = b.y;
+}
+__device__ __forceinline__ void slot_rows(const float* v, int slot, double (&r)[4]) {
+  const float4 a = *reinterpret_cast<const float4*>(v + 4 * slot);
+  r[0] = a.x; r[1] = a.y; r[2] = a.z; r[3] = a.w;
+}
+// the same rows of a wave's 64 FP64 values staged in LDS
+template <typename VT>
+__device__ __forceinline__ void slot_rows_lds(const double* v, int slot, double (&r)[4]) {
+  const int a = sizeof(VT) == 8 ? 2 * slot : 4 * slot, b = sizeof(VT) == 8 ? 32 + 2 * slot : a + 2;
+  const double2 x = *reinterpret_cast<const double2*>(v + a);
+  const double2 y = *reinterpret_cast<const double2*>(v + b);
+  r[0] = x.x; r[1] = x.y; r[2] = y.x; r[3] = y.y;
+}
+
+// acc[q] += V_{4q + lane % 4} . w over a slice's 64 rows for the vectors i <=
+// j; V points at the slice's first row of V_0.  NQ quads cover j + 1 vectors
+// (the launch picks the next of kDotQuads); vectors past j repeat the last
+// ones and their sums are not used.  A quad's address is a scalar plus the
+// lane's offset.
+template <int N, typename VT>
+__device__ __forceinline__ void dots_load(const VT* V, long long ldv, int j, int lane, int g,
+                                          double (&v)[N][4]) {
+  const int jq = j >> 2;  // the last quad with a vector <= j
+  const long long off = (lane & 3) * ldv, last = min(lane & 3, j & 3) * ldv;
+#pragma unroll
+  for (int q = 0; q < N; q++)
+    slot_rows(V + 4LL * min(g + q, jq) * ldv + (g + q < jq ? off : last), lane >> 2, v[q]);
+}
+template <int N>
+__device__ __forceinline__ void dots_add(const double (&v)[N][4], const double (&w)[4],
+                                         double* acc) {
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+#pragma unroll
+    for (int q = 0; q < N; q++)
+      acc[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(v[q][k], w[k], acc[q], 0, 0, 0);
+}
+// quads [G, NQ), four in flight together
+template <int G, int NQ, typename VT>
+__device__ __forceinline__ void dots_slice(const VT* V, long long ldv, int j, int lane,
+                                           const double (&w)[4], double (&acc)[NQ]) {
+  if constexpr (G < NQ) {
+    constexpr int N = NQ - G < 4 ? NQ - G : 4;
+    double v[N][4];
+    dots_load<N>(V, ldv, j, lane, G, v);
+    dots_add<N>(v, w, acc + G);
+    dots_slice<G + N, NQ>(V, ldv, j, lane, w, acc);
+  }
+}
+
+// the block's sums to partials[i * G + pb]: lane 16 i + 4 b holds vector i of
+// block b of every quad
+template <int NQ>
+__device__ __forceinline__ void dots_finish(const double (&acc)[NQ], int j, int G, int pb,
+                                            double* partials) {
+  __shared__ double red[OPB / 64][MAX_NV];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+#pragma unroll
+  for (int q = 0; q < NQ; q++) {
+    double d = acc[q];
+    d += __shfl_xor(d, 4, 64);
+    d += __shfl_xor(d, 8, 64);
+    if ((lane & 15) == 0) red[wv][4 * q + (lane >> 4)] = d;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x <= j) {
+    double s = 0.0;
+    for (int w = 0; w < nw; w++) s += red[w][threadIdx.x];
+    partials[(size_t)threadIdx.x * G + pb] = s;
+  }
+}
+
+template <typename XT, class Before>
+__device__ __forceinline__ double sell_row_one_op(const SolveArgs& A, const XT* x, int sl, int lane,
+                                                  Before before) {
+  return A.op32 ? sell_row_one(A, A.val32, x, sl, lane, before)
+                : sell_row_one(A, A.val, x, sl, lane, before);
 }
 
 // row sum with the FP64 or the FP32 copy of the values (accumulated in FP64)
