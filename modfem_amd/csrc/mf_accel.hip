@@ -182,8 +182,9 @@ int tmr_get_crs_structure(int Nrdof_glob, int nnz, int* crs_col_ind, int* crs_ro
   g_acc.d_val = g_acc.d_rhs = nullptr;
   MF_HIP(hipMalloc(&g_acc.d_val, (size_t)nnz * sizeof(double)));
   MF_HIP(hipMalloc(&g_acc.d_rhs, (size_t)Nrdof_glob * sizeof(double)));
-  MF_HIP(hipMemset(g_acc.d_val, 0, (size_t)nnz * sizeof(double)));
-  MF_HIP(hipMemset(g_acc.d_rhs, 0, (size_t)Nrdof_glob * sizeof(double)));
+  MF_HIP(hipMemsetAsync(g_acc.d_val, 0, (size_t)nnz * sizeof(double), stream()));
+  MF_HIP(hipMemsetAsync(g_acc.d_rhs, 0, (size_t)Nrdof_glob * sizeof(double), stream()));
+  MF_HIP(hipStreamSynchronize(stream()));
   g_acc.registered = true;
   return 0;
 }
@@ -318,8 +319,9 @@ int tmr_prepare_final_crs(void) {
   MF_HIP(hipMemcpy(r.data(), g_acc.d_rhs, r.size() * sizeof(double), hipMemcpyDeviceToHost));
   for (size_t i = 0; i < v.size(); i++) g_acc.h_val[i] += v[i];
   for (size_t i = 0; i < r.size(); i++) g_acc.h_rhs[i] += r[i];
-  MF_HIP(hipMemset(g_acc.d_val, 0, v.size() * sizeof(double)));
-  MF_HIP(hipMemset(g_acc.d_rhs, 0, r.size() * sizeof(double)));
+  MF_HIP(hipMemsetAsync(g_acc.d_val, 0, v.size() * sizeof(double), stream()));
+  MF_HIP(hipMemsetAsync(g_acc.d_rhs, 0, r.size() * sizeof(double), stream()));
+  MF_HIP(hipStreamSynchronize(stream()));
   return 0;
 }
 

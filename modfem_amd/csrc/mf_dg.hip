@@ -3401,7 +3401,9 @@ int dg_batch_structure(DgProblem& D) {
   MF_HIP(hipMalloc(&P->d_scol, col.size() * sizeof(int)));
   MF_HIP(hipMemcpy(P->d_scol, col.data(), col.size() * sizeof(int), hipMemcpyHostToDevice));
   MF_HIP(hipMalloc(&P->d_val, (size_t)P->nnz_sell * sizeof(double)));
-  MF_HIP(hipMemset(P->d_val, 0, (size_t)P->nnz_sell * sizeof(double)));  // padding stays zero
+  // padding stays zero
+  MF_HIP(hipMemsetAsync(P->d_val, 0, (size_t)P->nnz_sell * sizeof(double), stream()));
+  MF_HIP(hipStreamSynchronize(stream()));
   MF_HIP(hipMalloc(&P->d_rhs, (size_t)n * sizeof(double)));
   return 0;
 }
@@ -3935,7 +3937,8 @@ int mf_dg_set_multigrid(int did, int nu1, int nu2, int coarse) {
       }
     }
     MF_HIP(hipMalloc(&G.zero, std::max<long long>(D->ndof, 1) * sizeof(double)));
-    MF_HIP(hipMemset(G.zero, 0, std::max<long long>(D->ndof, 1) * sizeof(double)));
+    MF_HIP(hipMemsetAsync(G.zero, 0, std::max<long long>(D->ndof, 1) * sizeof(double), stream()));
+    MF_HIP(hipStreamSynchronize(stream()));
   }
   D->mg->nu1 = nu1;
   D->mg->nu2 = nu2;

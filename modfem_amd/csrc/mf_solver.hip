@@ -1124,7 +1124,8 @@ static int ensure_workspace(Problem& P, int m) {
   if (P.d_V) (void)hipFree(P.d_V);
   if (P.d_H) (void)hipFree(P.d_H);
   MF_HIP(hipMalloc(&P.d_V, (size_t)(m + 1) * ldv * sizeof(double)));
-  MF_HIP(hipMemset(P.d_V, 0, (size_t)(m + 1) * ldv * sizeof(double)));
+  // cleared on the stream that reads it: the null stream does not order with it
+  MF_HIP(hipMemsetAsync(P.d_V, 0, (size_t)(m + 1) * ldv * sizeof(double), stream()));
   MF_HIP(hipMalloc(&P.d_H, (size_t)((m + 1) * (m + 1) + 4 * (m + 1)) * sizeof(double)));
   if (!P.d_partials) {
     MF_HIP(hipMalloc(&P.d_partials, partials_row(P) * MAX_NV * sizeof(double)));
