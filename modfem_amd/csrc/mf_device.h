@@ -95,6 +95,8 @@ struct GmresStat {
 // elimination order (0: the reference's DOF order, 1: multicolour), rows of
 // each forward / backward level, and the factors (strict L, strict U, and
 // 1/u_ii on the diagonal as the reference keeps it).
+int num_cus();  // compute units of the current device
+
 struct IluData {
   int order = 0, n = 0;
   long long nnz = 0;
@@ -112,6 +114,7 @@ struct IluData {
   // rows of one level, entry k of its row r at ptr[s] + 64 k + r % 64
   struct Sweep {
     std::vector<int> lev_sl;               // host: first slice of every level
+    std::vector<char> lev_ent;             // host: the level has entries
     long long* d_ptr = nullptr;            // slices + 1
     int* d_col = nullptr;                  // device row of the column
     int* d_src = nullptr;                  // factor entry, -1 padding

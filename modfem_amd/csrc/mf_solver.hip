@@ -52,7 +52,7 @@ namespace mf {
 
 static int g_ncu = 0;
 
-static int num_cus() {
+int num_cus() {
   if (!g_ncu) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 256;
@@ -1903,17 +1903,10 @@ __global__ void __launch_bounds__(SB) kb_ilu_level(BatchArgs B, const IluMember*
   if (sl >= s1[b]) return;
   const IluMember& M = L[k];
   const size_t v = (size_t)(j < 0 ? 0 : j + 1) * A.ldv;
-  if (A.v32) {
-    if (BWD)
-      ilu_bwd_row(M.b32, sl, lane, A.Vf + v);
-    else
-      ilu_fwd_row(M.f32, sl, lane, A.Vf + v);
-  } else {
-    if (BWD)
-      ilu_bwd_row(M.b, sl, lane, A.V + v);
-    else
-      ilu_fwd_row(M.f, sl, lane, A.V + v);
-  }
+  if (A.v32)
+    ilu_row<BWD>(BWD ? M.b32 : M.f32, sl, lane, A.Vf + v, 0);
+  else
+    ilu_row<BWD>(BWD ? M.b : M.f, sl, lane, A.V + v, 0);
 }
 
 // A batch without ILU members finishes step j - 1 inside the operator launch

@@ -415,50 +415,76 @@ struct IluSweepArgs {
 IluSweepArgs<double> sweep_args(const IluData::Sweep& W);
 IluSweepArgs<float> sweep_args32(const IluData::Sweep& W);
 
-// sum_k val_k v[col_k] over the L entries of one packed row, loads issued
-// in groups of 8 so that a group costs about two memory round trips
-template <typename FT, typename VT>
-__device__ __forceinline__ double packed_row_sum(const int* col, const FT* val, long long base,
-                                                 int L, const VT* v) {
-  constexpr int CH = 8;
+// sum_k val_k v[col_k] over the L entries of one packed row of slice sl (lane
+// = row).  A level or colour holds a few hundred slices, so its launch is
+// bound by its chain of dependent loads: the slice's offsets are scalars, all
+// entries of a row of up to kSellWide are requested at once and the vector
+// entries behind them; groups of four past the slice's width are skipped by
+// a wave-uniform test.  before(): loads to issue behind the entries
+template <typename FT, typename VT, class Before>
+__device__ __forceinline__ double packed_row_sum(const long long* ptr, const int* col,
+                                                 const FT* val, int sl, int lane, int L,
+                                                 const VT* v, Before before) {
+  const long long base = ptr[sl];
+  const int width = (int)((ptr[sl + 1] - base) >> 6);
+  const int* cs = col + base + lane;
+  const FT* vs = val + base + lane;
   double s = 0.0;
-  for (int k0 = 0; k0 < L; k0 += CH) {
-    int c[CH];
-    double w[CH], x[CH];
+  if (width == 0) before();
+  for (int k0 = 0; k0 < width; k0 += kSellWide) {
+    int c[kSellWide];
+    FT w[kSellWide];
+    VT x[kSellWide];
 #pragma unroll
-    for (int k = 0; k < CH; k++) {
-      const bool ok = k0 + k < L;
-      const long long q = base + 64LL * (ok ? k0 + k : k0);
-      c[k] = col[q];
-      w[k] = ok ? (double)val[q] : 0.0;
-    }
+    for (int g = 0; g < kSellWide; g += 4)
+      if (k0 + g < width)
 #pragma unroll
-    for (int k = 0; k < CH; k++) x[k] = (double)v[c[k]];
+        for (int k = g; k < g + 4; k++) {
+          const int q = 64 * min(k0 + k, width - 1);
+          c[k] = cs[q];
+          w[k] = vs[q];
+        }
+    if (k0 == 0) before();
 #pragma unroll
-    for (int k = 0; k < CH; k++) s += w[k] * x[k];
+    for (int g = 0; g < kSellWide; g += 4)
+      if (k0 + g < width)
+#pragma unroll
+        for (int k = g; k < g + 4; k++) x[k] = v[c[k]];
+#pragma unroll
+    for (int g = 0; g < kSellWide; g += 4)
+      if (k0 + g < width)
+#pragma unroll
+        for (int k = g; k < g + 4; k++) {
+          const double t = s + (double)w[k] * (double)x[k];
+          s = k0 + k < L ? t : s;
+        }
   }
   return s;
 }
 
 // forward: v_i <- v_i - sum_{k before i} l_ik v_k (the v_k are already
-// substituted: they belong to earlier levels)
-template <typename FT, typename VT>
-__device__ __forceinline__ void ilu_fwd_row(const IluSweepArgs<FT>& W, int sl, int lane, VT* v) {
+// substituted: they belong to earlier levels); backward: v_i <- (v_i -
+// sum_{k after i} u_ik v_k) / u_ii.  halt is tested once the row's place is
+// known, behind the requests it does not need
+template <bool BWD, typename FT, typename VT>
+__device__ __forceinline__ void ilu_row(const IluSweepArgs<FT>& W, int sl, int lane, VT* v,
+                                        int halt) {
+  sl = __builtin_amdgcn_readfirstlane(sl);
   const int pr = sl * 64 + lane;
-  const int i = W.row[pr];
-  if (i < 0) return;
-  v[i] = (VT)((double)v[i] - packed_row_sum(W.col, W.val, W.ptr[sl] + lane, W.len[pr], v));
+  const int row = W.row[pr], L = W.len[pr];
+  const FT d = BWD ? W.diag[pr] : FT(1);
+  if (halt) return;
+  const int i = max(row, 0);
+  VT own = 0;
+  const double s = packed_row_sum(W.ptr, W.col, W.val, sl, lane, L, v, [&]() { own = v[i]; });
+  if (row < 0) return;
+  const double t = (double)own - s;
+  v[i] = (VT)(BWD ? t * (double)d : t);
 }
 
-// backward: v_i <- (v_i - sum_{k after i} u_ik v_k) / u_ii
-template <typename FT, typename VT>
-__device__ __forceinline__ void ilu_bwd_row(const IluSweepArgs<FT>& W, int sl, int lane, VT* v) {
-  const int pr = sl * 64 + lane;
-  const int i = W.row[pr];
-  if (i < 0) return;
-  v[i] = (VT)(((double)v[i] - packed_row_sum(W.col, W.val, W.ptr[sl] + lane, W.len[pr], v)) *
-              (double)W.diag[pr]);
-}
+// wavefronts per block of a launch over nsl slices: small launches spread
+// over all CUs
+inline int sweep_waves(int nsl, int cus) { return nsl <= cus ? 1 : nsl <= 2 * cus ? 2 : 4; }
 
 // FP64 data of a mixed-precision batch member's refinement steps
 struct RefineArgs {
