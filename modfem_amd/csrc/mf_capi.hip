@@ -68,10 +68,11 @@ void free_problem_device(Problem& P) {
                   P.d_partials, P.d_counter, P.d_stat, P.d_x, P.d_work, P.d_work2, P.d_sl_ptr,
                   P.d_scol, P.d_diag_k, P.d_inc_ptr, P.d_inc_el, P.d_inc_loc,
                   P.d_finc_ptr, P.d_finc_f, P.d_finc_loc, P.d_el_offT, P.d_scol16, P.d_sbase,
-                  P.d_erow, P.d_bf_type};
+                  P.d_erow, P.d_bf_type, P.d_iperm};
   for (void* p : ptrs)
     if (p) hipFree(p);
   if (P.h_stat) hipHostFree(P.h_stat);
+  P.vecs.release();
   ilu_free(P);
   gs_free(P);
 }
@@ -118,17 +119,6 @@ void sell_to_crs(const Setup& S, const double* sell, double* crs) {
   }
 }
 
-// reference-order vector -> device order and back
-std::vector<double> to_device_order(const Setup& S, const double* x) {
-  std::vector<double> d(S.n);
-  for (int i = 0; i < S.n; i++) d[i] = x[S.perm[i]];
-  return d;
-}
-
-void to_reference_order(const Setup& S, const double* d, double* x) {
-  for (int i = 0; i < S.n; i++) x[S.perm[i]] = d[i];
-}
-
 // the assembly mode a problem runs: the row-wise and two-pass modes keep a
 // row's sums in LDS for rows of up to 32 entries; a mesh with longer rows
 // (vertices of high valence) is assembled by element atomics instead
@@ -160,11 +150,9 @@ int assemble_problem(Problem& P, int precision) {
   return 0;
 }
 
-int rhs_to_host(const Problem& P, double* rhs) {
-  std::vector<double> d(P.n);
-  MF_HIP(hipMemcpy(d.data(), P.d_rhs, (size_t)P.n * sizeof(double), hipMemcpyDeviceToHost));
-  to_reference_order(P.setup, d.data(), rhs);
-  return 0;
+int rhs_to_host(Problem& P, double* rhs) {
+  if (host_order(P)) return -2;
+  return vec_to_host(P.d_rhs, P.d_iperm, P.n, rhs);
 }
 
 }  // namespace
@@ -614,12 +602,9 @@ int mf_problem_create_crs(int n, const int* row_ptr, const int* col_ind, const d
     crs_to_sell(P->setup, val, sv.data());
     MF_HIP(hipMemcpy(P->d_val, sv.data(), sv.size() * sizeof(double), hipMemcpyHostToDevice));
   }
-  {
-    std::vector<double> d;
-    if (rhs) d = to_device_order(P->setup, rhs);
-    if (upload<double>(&P->d_rhs, rhs ? d.data() : nullptr, (size_t)n)) return -2;
-  }
+  if (upload<double>(&P->d_rhs, nullptr, (size_t)n)) return -2;
   if (!rhs && launch_zero(P->d_rhs, n)) return -2;
+  if (rhs && (host_order(*P) || vec_to_device(rhs, P->d_iperm, n, P->d_rhs))) return -2;
   MF_HIP(hipStreamSynchronize(stream()));
   int id = g_next_problem++;
   g_problems[id] = std::move(P);
@@ -869,10 +854,7 @@ int mf_set_system(int pid, const double* val, const double* rhs) {
     crs_to_sell(P->setup, val, sv.data());
     MF_HIP(hipMemcpy(P->d_val, sv.data(), sv.size() * sizeof(double), hipMemcpyHostToDevice));
   }
-  if (rhs) {
-    std::vector<double> d = to_device_order(P->setup, rhs);
-    MF_HIP(hipMemcpy(P->d_rhs, d.data(), d.size() * sizeof(double), hipMemcpyHostToDevice));
-  }
+  if (rhs && (host_order(*P) || vec_to_device(rhs, P->d_iperm, P->n, P->d_rhs))) return -2;
   P->dinv_valid = false;  // refilled before the next preconditioned solve
   P->val32_valid = false;
   if (P->ilu) P->ilu->valid = false;
@@ -883,24 +865,11 @@ int mf_set_system(int pid, const double* val, const double* rhs) {
 int mf_spmv(int pid, const double* x, double* y) {
   Problem* P = get_problem(pid);
   if (!P) return -3;
-  double *dx = nullptr, *dy = nullptr;
-  MF_HIP(hipMalloc(&dx, (size_t)P->n * sizeof(double)));
-  MF_HIP(hipMalloc(&dy, (size_t)P->n * sizeof(double)));
-  int rc = 0;
-  std::vector<double> xd = to_device_order(P->setup, x), yd(P->n);
-  hipError_t e = hipMemcpyAsync(dx, xd.data(), (size_t)P->n * sizeof(double), hipMemcpyHostToDevice, stream());
-  if (e == hipSuccess) rc = launch_spmv(*P, dx, dy);
-  if (e == hipSuccess && rc == 0)
-    e = hipMemcpyAsync(yd.data(), dy, (size_t)P->n * sizeof(double), hipMemcpyDeviceToHost, stream());
-  if (e == hipSuccess) e = hipStreamSynchronize(stream());
-  if (e == hipSuccess && rc == 0) to_reference_order(P->setup, yd.data(), y);
-  if (e != hipSuccess) {
-    set_error(hipGetErrorString(e));
-    rc = -2;
-  }
-  hipFree(dx);
-  hipFree(dy);
-  return rc;
+  PoolVec dx(P->vecs), dy(P->vecs);
+  if (host_order(*P) || dx.take(P->n) || dy.take(P->n)) return -2;
+  if (vec_to_device(x, P->d_iperm, P->n, dx.d)) return -2;
+  const int rc = launch_spmv(*P, dx.d, dy.d);
+  return rc ? rc : vec_to_host(dy.d, P->d_iperm, P->n, y);
 }
 
 int mf_fill_precon(int pid, int precon) {
@@ -937,13 +906,10 @@ int mf_gmres(int pid, int precon, int krylbas, int max_iter, double tol, int ini
     set_error("mf_gmres: max_iter >= 1 and tol >= 0 required");
     return -1;
   }
-  std::vector<double> xd;
-  if (x) xd = ini_zero ? std::vector<double>(P->n, 0.0) : to_device_order(P->setup, x);
-  int rc = gmres_solve(*P, precon, krylbas, max_iter, tol, 0.0, ini_zero, x ? xd.data() : nullptr,
-                       iters, res_rel, resid);
-  // rc: 1 converged, 0 not converged, <0 error
-  if (rc >= 0 && x) to_reference_order(P->setup, xd.data(), x);
-  return rc;
+  if (x && host_order(*P)) return -2;
+  // 1 converged, 0 not converged, <0 error
+  return gmres_solve(*P, precon, krylbas, max_iter, tol, 0.0, ini_zero, x, iters, res_rel, resid,
+                     P->d_iperm);
 }
 
 int mf_gmres_noalloc(int pid, int precon, int krylbas, int max_iter, double tol, int ini_zero,
@@ -1010,12 +976,9 @@ int mf_solve_mkb(int pid, const int* params, double conv_meas, int ini_zero, dou
     set_error("mf_solve_mkb: max_iter >= 1 required");
     return -1;
   }
-  std::vector<double> xd;
-  if (x) xd = ini_zero ? std::vector<double>(P->n, 0.0) : to_device_order(P->setup, x);
-  int rc = gmres_solve(*P, precon, krylbas, max_iter, tol_rel, tol_abs, ini_zero,
-                       x ? xd.data() : nullptr, iters, res_rel, resid);
-  if (rc >= 0 && x) to_reference_order(P->setup, xd.data(), x);
-  return rc;
+  if (x && host_order(*P)) return -2;
+  return gmres_solve(*P, precon, krylbas, max_iter, tol_rel, tol_abs, ini_zero, x, iters, res_rel,
+                     resid, P->d_iperm);
 }
 
 int mf_gmres_mixed(int pid, int precon, int krylbas, int max_iter, double tol, double* x,
@@ -1030,11 +993,9 @@ int mf_gmres_mixed(int pid, int precon, int krylbas, int max_iter, double tol, d
     set_error("mf_gmres_mixed: tol > 0 required");
     return -1;
   }
-  std::vector<double> xd(x ? P->n : 0);
-  int rc = gmres_mixed(*P, precon, krylbas, max_iter, tol, x ? xd.data() : nullptr, iters,
-                       res_rel, resid, refinements);
-  if (rc >= 0 && x) to_reference_order(P->setup, xd.data(), x);
-  return rc;
+  if (x && host_order(*P)) return -2;
+  return gmres_mixed(*P, precon, krylbas, max_iter, tol, x, iters, res_rel, resid, refinements,
+                     P->d_iperm);
 }
 
 int mf_set_gs(int pid, int nsweeps) {
@@ -1103,11 +1064,8 @@ int mf_get_solution(int pid, double* x) {
     set_error("mf_get_solution: no solution (run mf_gmres first) or x is null");
     return -1;
   }
-  std::vector<double> d(P->n);
-  MF_HIP(hipStreamSynchronize(stream()));
-  MF_HIP(hipMemcpy(d.data(), P->d_x, d.size() * sizeof(double), hipMemcpyDeviceToHost));
-  to_reference_order(P->setup, d.data(), x);
-  return 0;
+  if (host_order(*P)) return -2;
+  return vec_to_host(P->d_x, P->d_iperm, P->n, x);
 }
 
 int mf_true_residual(int pid, const double* x, double* rel) {

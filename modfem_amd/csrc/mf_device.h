@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -149,6 +150,32 @@ struct GsData {
   bool valid = false;
 };
 
+// device vectors kept for an object's calls with host vectors, so that a call
+// allocates nothing.  At most kKeep stay; calls from several threads each take
+// their own.  One stream runs all of them: a vector given back while a kernel
+// still uses it is written again only behind that kernel.  All vectors of one
+// pool have one length; release() before the object goes
+struct VecPool {
+  static constexpr size_t kKeep = 4;
+  std::mutex m;
+  std::vector<double*> kept;
+  int take(int n, double** d);
+  void give(double* d);
+  void release();
+};
+
+// a vector taken from a pool for a scope
+struct PoolVec {
+  VecPool& pool;
+  double* d = nullptr;
+  explicit PoolVec(VecPool& p) : pool(p) {}
+  PoolVec(const PoolVec&) = delete;
+  ~PoolVec() {
+    if (d) pool.give(d);
+  }
+  int take(int n) { return pool.take(n, &d); }
+};
+
 struct Problem {
   // host side
   Mesh mesh;
@@ -156,6 +183,10 @@ struct Problem {
   int n = 0, nel = 0, nbf = 0;
   long long nnz = 0;
   int el_type = kPrism;  // uniform element type (mixed handled per launch)
+  // calls with host vectors: device vectors, and the device row of every
+  // reference row (host_order)
+  VecPool vecs;
+  int* d_iperm = nullptr;
   // device arrays
   double* d_coor = nullptr;    // 3*n, device row order
   int* d_el_dof = nullptr;     // 6*nel SoA
@@ -338,10 +369,17 @@ int launch_assemble_many(const std::vector<Problem*>& ps, int precision);
 int problem_setup_device(const Mesh& M, Problem& P);
 int launch_faces(Problem& P, int write_faces, double* d_fmat, int f0, int fcount);
 int launch_fill_jacobi(Problem& P);
+// host vectors (mf_hostvec.hip), on the library stream.  Entry r of h belongs
+// to entry d_iperm[r] of d (null: r).  To the device: h has been read on
+// return; to the host: h is written on return
+int vec_to_device(const double* h, const int* d_iperm, int n, double* d);
+int vec_to_host(const double* d, const int* d_iperm, int n, double* h);
+int host_order(Problem& P);  // makes P.d_iperm
+// d_iperm given: h_x is in that order; null: h_x is in the device's order
 // tol: relative to the initial preconditioned residual; tol_abs: absolute
 int gmres_solve(Problem& P, int precon, int krylbas, int max_iter, double tol,
                 double tol_abs, int ini_zero, double* h_x, int* iters, double* res_rel,
-                double* resid);
+                double* resid, const int* d_iperm = nullptr);
 // GMRES(m) with precon 0/1 whose work arrays live in a fixed device array
 // (no device allocation); noalloc_scratch_init looks the array up for the
 // current device (called by mf_init)
@@ -350,7 +388,8 @@ int gmres_noalloc(Problem& P, int precon, int krylbas, int max_iter, double tol,
                   double* h_x, int* iters, double* res_rel, double* resid);
 // FP64 refinement around GMRES with an FP32-valued operator
 int gmres_mixed(Problem& P, int precon, int krylbas, int max_iter, double tol, double* h_x,
-                int* iters, double* res_rel, double* resid, int* refinements);
+                int* iters, double* res_rel, double* resid, int* refinements,
+                const int* d_iperm);
 int launch_spmv(Problem& P, const double* d_x, double* d_y);
 // ms per operator application of a precision variant (mf_bench_spmv_ex)
 int bench_spmv_variant(Problem& P, int prec, int ch, int reps, double* ms);

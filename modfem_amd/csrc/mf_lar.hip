@@ -58,6 +58,7 @@ struct LarMatrix {
   std::unique_ptr<Problem> G;
   std::unique_ptr<ExtOp> op;
   int op_kind = -1, op_sweeps = -1;
+  std::shared_ptr<VecPool> vecs = std::make_shared<VecPool>();  // of ndof() entries
 };
 
 std::vector<LarMatrix> g_mats;  // LIFO like itv_crs_matrices
@@ -90,42 +91,49 @@ int flush(LarMatrix& M) {
   return 0;
 }
 
-bool is_device_ptr(const void* p) {
-  if (!p) return false;
-  hipPointerAttribute_t a;
-  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  return a.type == hipMemoryTypeDevice;
-}
-
-// stage a vector of n doubles on the device (copy when it is host memory)
+// a caller's vector on the device: itself when it is device memory, else one
+// of the matrix's pool.  Plain host memory goes through the pinned ring;
+// memory the runtime knows (pinned, managed) by a copy that the stream orders
 struct Staged {
+  std::shared_ptr<VecPool> pool;  // outlives the matrix if a call is under way
   double* d = nullptr;
-  bool owned = false;
+  bool plain = false;
   ~Staged() {
-    if (owned && d) (void)hipFree(d);
+    if (pool && d) pool->give(d);
   }
 };
 
-int stage_in(const double* p, int n, Staged& s, bool copy) {
+int stage_in(const LarMatrix& M, const double* p, Staged& s, bool copy) {
   if (!p) return 0;
-  if (is_device_ptr(p)) {
+  hipPointerAttribute_t a;
+  const hipError_t e = hipPointerGetAttributes(&a, p);
+  if (e != hipSuccess) (void)hipGetLastError();
+  if (e == hipSuccess && a.type == hipMemoryTypeDevice) {
     s.d = const_cast<double*>(p);
     return 0;
   }
-  MF_HIP(hipMalloc(&s.d, (size_t)n * sizeof(double)));
-  s.owned = true;
-  if (copy)
-    MF_HIP(hipMemcpyAsync(s.d, p, (size_t)n * sizeof(double), hipMemcpyHostToDevice, stream()));
+  s.plain = e != hipSuccess || a.type == hipMemoryTypeUnregistered;
+  const int n = M.ndof();
+  if (M.vecs->take(n, &s.d)) return -2;
+  s.pool = M.vecs;
+  if (!copy) return 0;
+  if (s.plain) return vec_to_device(p, nullptr, n, s.d);
+  MF_HIP(hipMemcpyAsync(s.d, p, (size_t)n * sizeof(double), hipMemcpyHostToDevice, stream()));
   return 0;
 }
 
 int stage_out(double* host, const Staged& s, int n) {
-  if (s.owned)
+  if (s.pool && s.plain) return vec_to_host(s.d, nullptr, n, host);
+  if (s.pool)
     MF_HIP(hipMemcpyAsync(host, s.d, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, stream()));
   MF_HIP(hipStreamSynchronize(stream()));
+  return 0;
+}
+
+// a work vector of the matrix's pool
+int stage_tmp(const LarMatrix& M, Staged& s) {
+  if (M.vecs->take(M.ndof(), &s.d)) return -2;
+  s.pool = M.vecs;
   return 0;
 }
 
@@ -472,6 +480,7 @@ int lar_free_SM_and_LV(int Matrix_id) {
     void* ptrs[] = {B.d_rp, B.d_ci, B.d_val, B.d_rhs, B.d_col_rows};
     for (void* p : ptrs)
       if (p) (void)hipFree(p);
+    M->vecs->release();
     g_mats.pop_back();
     return 0;
   }
@@ -481,6 +490,7 @@ int lar_free_SM_and_LV(int Matrix_id) {
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (P.h_stat) (void)hipHostFree(P.h_stat);
+  M->vecs->release();
   g_mats.pop_back();
   return 0;
 }
@@ -680,9 +690,9 @@ void lar_compute_residual(int Matrix_id, int Use_rhs, int Ini_zero, int Ndof, do
   if (flush(*M)) return;
   if (M->B) {
     Staged sx, sb, sv;
-    if (!Ini_zero && stage_in(X, Ndof, sx, true)) return;
-    if (Use_rhs == 1 && B && stage_in(B, Ndof, sb, true)) return;
-    if (stage_in(V, Ndof, sv, false)) return;
+    if (!Ini_zero && stage_in(*M, X, sx, true)) return;
+    if (Use_rhs == 1 && B && stage_in(*M, B, sb, true)) return;
+    if (stage_in(*M, V, sv, false)) return;
     const double* db = (Use_rhs == 1) ? (B ? sb.d : M->B->d_rhs) : nullptr;
     if (bcrs_residual(*M->B, Ini_zero ? nullptr : sx.d, db, sv.d)) return;
     stage_out(V, sv, Ndof);
@@ -690,9 +700,9 @@ void lar_compute_residual(int Matrix_id, int Use_rhs, int Ini_zero, int Ndof, do
   }
   Problem& P = *M->P;
   Staged sx, sb, sv;
-  if (!Ini_zero && stage_in(X, Ndof, sx, true)) return;
-  if (Use_rhs == 1 && B && stage_in(B, Ndof, sb, true)) return;
-  if (stage_in(V, Ndof, sv, false)) return;
+  if (!Ini_zero && stage_in(*M, X, sx, true)) return;
+  if (Use_rhs == 1 && B && stage_in(*M, B, sb, true)) return;
+  if (stage_in(*M, V, sv, false)) return;
   const double* db = (Use_rhs == 1) ? (B ? sb.d : P.d_rhs) : nullptr;
   if (launch_rowop(P, 0, Use_rhs == 1, Ini_zero ? nullptr : sx.d, db, nullptr, sv.d)) return;
   stage_out(V, sv, Ndof);
@@ -718,14 +728,13 @@ void lar_perform_BJ_or_GS_iterations(int Matrix_id, int Use_rhs, int Ini_zero, i
     }
     if (flush(*M)) return;
     Staged sv, sb;
-    if (stage_in(V, Ndof, sv, true)) return;
-    if (Use_rhs == 1 && B && stage_in(B, Ndof, sb, true)) return;
-    double* tmp = nullptr;
-    if (hipMalloc(&tmp, (size_t)Ndof * sizeof(double)) != hipSuccess) return;
+    if (stage_in(*M, V, sv, true)) return;
+    if (Use_rhs == 1 && B && stage_in(*M, B, sb, true)) return;
+    Staged tmp;
+    if (stage_tmp(*M, tmp)) return;
     const double* db = (Use_rhs == 1) ? (B ? sb.d : M->B->d_rhs) : nullptr;
-    if (bcrs_sweeps(*M->B, M->precon == BLOCK_GS, Nr_prec, db, sv.d, tmp) == 0)
+    if (bcrs_sweeps(*M->B, M->precon == BLOCK_GS, Nr_prec, db, sv.d, tmp.d) == 0)
       stage_out(V, sv, Ndof);
-    (void)hipFree(tmp);
     return;
   }
   if (!M || Ndof != M->P->n || (M->precon != BLOCK_JACOBI && M->precon != BLOCK_GS) ||
@@ -737,27 +746,29 @@ void lar_perform_BJ_or_GS_iterations(int Matrix_id, int Use_rhs, int Ini_zero, i
   if (flush(*M)) return;
   Problem& P = *M->P;
   Staged sv, sb;
-  if (stage_in(V, Ndof, sv, true)) return;
-  if (Use_rhs == 1 && B && stage_in(B, Ndof, sb, true)) return;
-  double* tmp = nullptr;
-  if (hipMalloc(&tmp, (size_t)Ndof * sizeof(double)) != hipSuccess) return;
+  if (stage_in(*M, V, sv, true)) return;
+  if (Use_rhs == 1 && B && stage_in(*M, B, sb, true)) return;
+  Staged tmp;
+  if (stage_tmp(*M, tmp)) return;
   const double* db = (Use_rhs == 1) ? (B ? sb.d : P.d_rhs) : nullptr;
   if (M->precon == BLOCK_GS) {
-    if (crs_gs_chunked(P, M->gs_threads, Nr_prec, db, sv.d, tmp, nullptr) == 0)
+    if (crs_gs_chunked(P, M->gs_threads, Nr_prec, db, sv.d, tmp.d, nullptr) == 0)
       stage_out(V, sv, Ndof);
     else
       fprintf(stderr, "lar_perform_BJ_or_GS_iterations: %s\n", last_error());
-    (void)hipFree(tmp);
     return;
   }
+  double *cur = sv.d, *nxt = tmp.d;
   for (int it = 0; it < Nr_prec; it++) {
-    if (launch_rowop(P, 1, Use_rhs == 1, sv.d, db, P.d_diag_ptr, tmp)) break;
-    if (hipMemcpyAsync(sv.d, tmp, (size_t)Ndof * sizeof(double), hipMemcpyDeviceToDevice,
-                       stream()) != hipSuccess)
-      break;
+    if (launch_rowop(P, 1, Use_rhs == 1, cur, db, P.d_diag_ptr, nxt)) break;
+    std::swap(cur, nxt);
   }
+  if (cur != sv.d && sv.pool)
+    std::swap(sv.d, tmp.d);
+  else if (cur != sv.d && hipMemcpyAsync(sv.d, cur, (size_t)Ndof * sizeof(double),
+                                         hipMemcpyDeviceToDevice, stream()) != hipSuccess)
+    return;
   stage_out(V, sv, Ndof);
-  (void)hipFree(tmp);
 }
 
 // lar_perform_rhsub: V = (LU)^-1 B (B null: the stored rhs) with the BCRS
@@ -774,8 +785,8 @@ void lar_perform_rhsub(int Matrix_id, int Ndof, double* V, double* B) {
   }
   if (flush(*M)) return;
   Staged sb, sv;
-  if (B && stage_in(B, Ndof, sb, true)) return;
-  if (stage_in(V, Ndof, sv, false)) return;
+  if (B && stage_in(*M, B, sb, true)) return;
+  if (stage_in(*M, V, sv, false)) return;
   if (bcrs_ilu_solve(*M->B, B ? sb.d : M->B->d_rhs, sv.d)) return;
   stage_out(V, sv, Ndof);
 }
@@ -1259,7 +1270,7 @@ int lsr_mkb_solve(int Solver_id, int Comp_type, int Ini_zero, double* X, double*
   double* d_rhs_saved = M->B ? M->B->d_rhs : M->P->d_rhs;
   Staged sb;
   if (B) {
-    if (stage_in(B, n, sb, true)) return -2;
+    if (stage_in(*M, B, sb, true)) return -2;
     if (M->B) M->B->d_rhs = sb.d;
     else M->P->d_rhs = sb.d;
   }

@@ -1254,7 +1254,7 @@ static bool step_wanted(const GmresStat* h, int j, int ahead) {
 static int gmres_core(Problem& P, int precon, int krylbas, int max_iter, double tol,
                       double tol_abs, int ini_zero, double* h_x, const double* d_b, double* d_x,
                       int op32, int* iters, double* res_rel_out, double* resid_out,
-                      bool noalloc = false) {
+                      bool noalloc = false, const int* d_iperm = nullptr) {
   const int m = krylbas;
   if (m < 1 || m >= MAX_NV) {
     set_error("GMRES: number of Krylov vectors must be in [1,63]");
@@ -1335,6 +1335,8 @@ static int gmres_core(Problem& P, int precon, int krylbas, int max_iter, double 
   }
   if (ini_zero || (!h_x && !noalloc)) {
     MF_HIP(hipMemsetAsync(d_x, 0, (size_t)P.n * sizeof(double), s));
+  } else if (h_x && d_iperm) {
+    if (vec_to_device(h_x, d_iperm, P.n, d_x)) return -2;
   } else if (h_x) {
     MF_HIP(hipMemcpyAsync(d_x, h_x, (size_t)P.n * sizeof(double), hipMemcpyHostToDevice, s));
   }
@@ -1492,7 +1494,11 @@ static int gmres_core(Problem& P, int precon, int krylbas, int max_iter, double 
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
   }
-  if (h_x) MF_HIP(hipMemcpy(h_x, d_x, (size_t)P.n * sizeof(double), hipMemcpyDeviceToHost));
+  if (h_x && d_iperm) {
+    if (vec_to_host(d_x, d_iperm, P.n, h_x)) return -2;
+  } else if (h_x) {
+    MF_HIP(hipMemcpy(h_x, d_x, (size_t)P.n * sizeof(double), hipMemcpyDeviceToHost));
+  }
   if (iters) *iters = gmiter;
   if (res_rel_out) *res_rel_out = res_rel;
   if (resid_out) *resid_out = resid;
@@ -1500,10 +1506,11 @@ static int gmres_core(Problem& P, int precon, int krylbas, int max_iter, double 
 }
 
 int gmres_solve(Problem& P, int precon, int krylbas, int max_iter, double tol, double tol_abs,
-                int ini_zero, double* h_x, int* iters, double* res_rel_out, double* resid_out) {
+                int ini_zero, double* h_x, int* iters, double* res_rel_out, double* resid_out,
+                const int* d_iperm) {
   if (!P.d_x) MF_HIP(hipMalloc(&P.d_x, (size_t)P.n * sizeof(double)));
   return gmres_core(P, precon, krylbas, max_iter, tol, tol_abs, ini_zero, h_x, P.d_rhs, P.d_x, 0,
-                    iters, res_rel_out, resid_out);
+                    iters, res_rel_out, resid_out, false, d_iperm);
 }
 
 // FP32 copies for mixed-precision inner solves: matrix values, and the
@@ -1545,7 +1552,8 @@ static int round_mixed(Problem& P, int precon) {
 // otherwise solve A d = r_k with the FP32 operator to the relative tolerance
 // max(tol rho_0 / rho_k, 1e-6) and set x_{k+1} = x_k + d.
 int gmres_mixed(Problem& P, int precon, int krylbas, int max_iter, double tol, double* h_x,
-                int* iters, double* res_rel_out, double* resid_out, int* refinements) {
+                int* iters, double* res_rel_out, double* resid_out, int* refinements,
+                const int* d_iperm) {
   if (!P.sell) {
     set_error("mixed-precision GMRES needs a SELL problem");
     return -1;
@@ -1621,7 +1629,7 @@ int gmres_mixed(Problem& P, int precon, int krylbas, int max_iter, double tol, d
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (rc < 0) return rc;
-  if (h_x) MF_HIP(hipMemcpy(h_x, P.d_x, (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
+  if (h_x && vec_to_host(P.d_x, d_iperm, P.n, h_x)) return -2;
   if (iters) *iters = total;
   if (res_rel_out) *res_rel_out = rho0 > 0 ? rho / rho0 : 0.0;
   if (resid_out) *resid_out = rho;
