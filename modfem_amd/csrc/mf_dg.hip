@@ -2041,42 +2041,74 @@ __device__ __forceinline__ int dg_sorted_sides(const int* fnb, int i, bool lower
 
 constexpr int kIluMax = 40;  // largest block (p = 3 in both directions)
 
-// one row of the factorisation per 64-lane block
-__global__ void __launch_bounds__(64) k_dg_ilu_row(int cnt, const int* rows, DgIluLay Y,
-                                                   double* F, double* Finv, int* bad) {
-  __shared__ double D[kIluMax * kIluMax];
-  __shared__ double T[kIluMax * kIluMax];
+// d (ni x n) = sum over l ascending of a (ni x nk) b (nk x n), column-major in
+// LDS; a thread takes four columns of one row at a time: four products per
+// five LDS reads.  use(r, c, d) gets each entry
+template <class Use>
+__device__ __forceinline__ void dg_block_product(const double* a, const double* b, int ni, int nk,
+                                                 int n, Use use) {
+  for (int q = threadIdx.x; q < ni * ((n + 3) / 4); q += blockDim.x) {
+    const int r = q % ni, c = q / ni * 4;
+    const double* bc[4];
+    double d[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      bc[k] = b + nk * min(c + k, n - 1);
+      d[k] = 0.0;
+    }
+#pragma unroll 4
+    for (int l = 0; l < nk; l++) {
+      const double t = a[r + ni * l];
+#pragma unroll
+      for (int k = 0; k < 4; k++) d[k] += t * bc[k][l];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (c + k < n) use(r, c + k, d[k]);
+  }
+}
+
+// One row of the factorisation per block; M: largest block size of the
+// problem, LDS 4 M^2 doubles.  A level holds a few hundred rows, so it is
+// bound by one row's chain.  The operands of a neighbour's products are
+// staged in LDS together and shared by four wavefronts (one for blocks of up
+// to 10 unknowns); the inverse is taken row by row: row l of inv(U), and of
+// inv(U) inv(L), needs only itself and the factors, so a lane does its row
+// without a barrier, every sum in the order of dtrti2 and dgetri.  16^3
+// prisms of degrees 1 to 3, 546 rows a level: 820 us a level with one
+// wavefront, operands from L2 and a column at a time; 162 us
+__global__ void __launch_bounds__(256) k_dg_ilu_row(const int* rows, DgIluLay Y, int M, double* F,
+                                                    double* Finv, int* bad) {
+  extern __shared__ double ilu_lds[];
   __shared__ int piv[kIluMax];
-  const int lane = threadIdx.x;
+  double *D = ilu_lds, *T = D + M * M, *P = T + M * M, *Q = P + M * M;
+  const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63;
   const int i = rows[blockIdx.x];
   const int ni = Y.nse(i);
   const double* Ai = F + Y.so(i, 0);
-  for (int q = lane; q < ni * ni; q += 64) D[q] = Ai[q];
+  for (int q = tid; q < ni * ni; q += nt) D[q] = Ai[q];
   int side[5];
   const int nl = dg_sorted_sides(Y.fnb, i, true, side);
-  __syncthreads();
   for (int t = 0; t < nl; t++) {
     const int s = side[t], k = Y.fnb[5 * (size_t)i + s], nk = Y.nse(k);
     double* Aik = F + Y.so(i, 1 + s);
     const double* Dk = Finv + Y.vo(k);
-    // a_ik inv(D_k), sums from 0 over the inner index
-    for (int q = lane; q < ni * nk; q += 64) {
-      const int r = q % ni, c = q / ni;
-      double d = 0.0;
-      for (int l = 0; l < nk; l++) d += Aik[r + (size_t)ni * l] * Dk[l + (size_t)nk * c];
-      T[q] = d;
-    }
+    // a_ki: row k's block across the side facing i (bits 0-2: that side)
+    const double* Aki = F + Y.so(k, 1 + (Y.fcode[5 * (size_t)i + s] & 7));
     __syncthreads();
-    for (int q = lane; q < ni * nk; q += 64) Aik[q] = T[q];
-    // D_i -= a_ik a_ki (a_ki: row k's block across the side facing i)
-    const int sk = Y.fcode[5 * (size_t)i + s] & 7;  // bits 0-2: the neighbour's side
-    const double* Aki = F + Y.so(k, 1 + sk);
-    for (int q = lane; q < ni * ni; q += 64) {
-      const int r = q % ni, c = q / ni;
-      double d = 0.0;
-      for (int l = 0; l < nk; l++) d += T[r + ni * l] * Aki[l + (size_t)nk * c];
-      D[q] -= d;
+    for (int q = tid; q < ni * nk; q += nt) {
+      P[q] = Aik[q];
+      Q[q] = Aki[q];
     }
+    for (int q = tid; q < nk * nk; q += nt) T[q] = Dk[q];
+    __syncthreads();
+    // a_ik inv(D_k); it takes P's place behind the barrier, from memory
+    dg_block_product(P, T, ni, nk, nk, [&](int r, int c, double d) { Aik[r + ni * c] = d; });
+    __syncthreads();
+    for (int q = tid; q < ni * nk; q += nt) P[q] = Aik[q];
+    __syncthreads();
+    // D_i -= a_ik a_ki
+    dg_block_product(P, Q, ni, nk, ni, [&](int r, int c, double d) { D[r + ni * c] -= d; });
     // a_ij -= a_ik a_kj for neighbours j > k of both
     for (int s2 = 0; s2 < 5; s2++) {
       const int j = Y.fnb[5 * (size_t)i + s2];
@@ -2088,16 +2120,16 @@ __global__ void __launch_bounds__(64) k_dg_ilu_row(int cnt, const int* rows, DgI
       const int nj = Y.nse(j);
       double* Aij = F + Y.so(i, 1 + s2);
       const double* Akj = F + Y.so(k, 1 + t2);
-      for (int q = lane; q < ni * nj; q += 64) {
-        const int r = q % ni, c = q / ni;
-        double d = 0.0;
-        for (int l = 0; l < nk; l++) d += T[r + ni * l] * Akj[l + (size_t)nk * c];
-        Aij[q] -= d;
-      }
+      __syncthreads();
+      for (int q = tid; q < nk * nj; q += nt) T[q] = Akj[q];
+      __syncthreads();
+      dg_block_product(P, T, ni, nk, nj, [&](int r, int c, double d) { Aij[r + ni * c] -= d; });
     }
-    __syncthreads();
   }
-  // LU of D with partial pivoting (dgetf2): lane = row
+  __syncthreads();
+  // LU of D with partial pivoting (dgetf2): lane = row, columns dealt to the
+  // wavefronts; every wavefront finds the pivot
+  const int wv = tid >> 6, nw = nt >> 6;
   for (int j = 0; j < ni; j++) {
     double v = (lane >= j && lane < ni) ? fabs(D[lane + ni * j]) : -1.0;
     int r = lane;
@@ -2108,64 +2140,61 @@ __global__ void __launch_bounds__(64) k_dg_ilu_row(int cnt, const int* rows, DgI
       if (v2 > v || (v2 == v && r2 < r)) { v = v2; r = r2; }
     }
     if (!(v > 0.0)) {
-      if (lane == 0) bad[0] = 1;
+      if (tid == 0) bad[0] = 1;
       return;
     }
-    if (lane == 0) piv[j] = r;
-    if (r != j && lane < ni) {  // swap rows j and r, lane = column
-      const double a = D[j + ni * lane];
-      D[j + ni * lane] = D[r + ni * lane];
-      D[r + ni * lane] = a;
+    if (tid == 0) piv[j] = r;
+    __syncthreads();
+    if (r != j && tid < ni) {  // swap rows j and r, thread = column
+      const double a = D[j + ni * tid];
+      D[j + ni * tid] = D[r + ni * tid];
+      D[r + ni * tid] = a;
     }
     __syncthreads();
-    const double rp = 1.0 / D[j + ni * j];
-    if (lane > j && lane < ni) D[lane + ni * j] *= rp;
+    const bool below = lane > j && lane < ni;
+    const double lij = below ? D[lane + ni * j] * (1.0 / D[j + ni * j]) : 0.0;
+    if (below)
+      for (int c = j + 1 + wv; c < ni; c += nw) D[lane + ni * c] += lij * -D[j + ni * c];
     __syncthreads();
-    if (lane > j && lane < ni) {
-      const double lij = D[lane + ni * j];
-      for (int c = j + 1; c < ni; c++) D[lane + ni * c] += lij * -D[j + ni * c];
-    }
-    __syncthreads();
+    if (below && wv == 0) D[lane + ni * j] = lij;
   }
-  // inv(U) column by column (dtrti2), lane = row
-  for (int j = 0; j < ni; j++) {
-    double x = lane < j ? D[lane + ni * j] : 0.0;
-    const double ujj = 1.0 / D[j + ni * j];
-    for (int jj = 0; jj < j; jj++) {
-      const double t = __shfl(x, jj);
-      if (t != 0.0) {
-        if (lane < jj) x = x + t * D[lane + ni * jj];
-        else if (lane == jj) x = x * D[jj + ni * jj];
+  __syncthreads();
+  if (tid < ni) {  // lane = row of the inverse, kept in T; D holds L and U
+    // inv(U) (dtrti2): x_j = -(x_l u_lj + sum over l < q < j of u_qj x_q) / u_jj
+    T[tid + ni * tid] = 1.0 / D[tid + ni * tid];
+    for (int j = 0; j < ni; j++) {
+      const double* u = D + ni * j;
+      const double ujj = 1.0 / u[j];
+      if (j <= tid) {
+        if (j < tid) T[tid + ni * j] = 0.0;
+        continue;
       }
+      double x = u[tid];
+      x = x != 0.0 ? x * T[tid + ni * tid] : x;
+#pragma unroll 4
+      for (int q = tid + 1; q < j; q++) {
+        const double y = x + u[q] * T[tid + ni * q];
+        x = u[q] != 0.0 ? y : x;
+      }
+      T[tid + ni * j] = -ujj * x;
     }
-    __syncthreads();
-    if (lane < j) D[lane + ni * j] = -ujj * x;
-    if (lane == 0) D[j + ni * j] = ujj;
-    __syncthreads();
-  }
-  // inv(A) = inv(U) inv(L) (dgetri), columns from the last, lane = row
-  for (int j = ni - 1; j >= 0; j--) {
-    const double w = (lane > j && lane < ni) ? D[lane + ni * j] : 0.0;
-    double y = (lane <= j && lane < ni) ? D[lane + ni * j] : 0.0;
-    for (int jj = j + 1; jj < ni; jj++) {
-      const double t = -1.0 * __shfl(w, jj);
-      if (lane < ni) y = y + t * D[lane + ni * jj];
+    // inv(U) inv(L) (dgetri), columns from the last
+    for (int j = ni - 1; j >= 0; j--) {
+      double y = T[tid + ni * j];
+#pragma unroll 4
+      for (int q = j + 1; q < ni; q++) y = y + -D[q + ni * j] * T[tid + ni * q];
+      T[tid + ni * j] = y;
     }
-    __syncthreads();
-    if (lane < ni) D[lane + ni * j] = y;
-    __syncthreads();
-  }
-  for (int j = ni - 2; j >= 0; j--) {  // column interchanges in reverse order
-    const int jp = piv[j];
-    if (jp != j && lane < ni) {
-      const double a = D[lane + ni * j];
-      D[lane + ni * j] = D[lane + ni * jp];
-      D[lane + ni * jp] = a;
+    for (int j = ni - 2; j >= 0; j--) {  // column interchanges in reverse order
+      const int jp = piv[j];
+      const double a = T[tid + ni * j];
+      T[tid + ni * j] = T[tid + ni * jp];
+      T[tid + ni * jp] = a;
     }
-    __syncthreads();
   }
+  __syncthreads();
   double* Di = Finv + Y.vo(i);
-  for (int q = lane; q < ni * ni; q += 64) Di[q] = D[q];
+  for (int q = tid; q < ni * ni; q += nt) Di[q] = T[q];
 }
 
 // ---------------------------------------------------------------------
@@ -2878,10 +2907,14 @@ int fill_block_ilu(DgProblem& D) {
   MF_HIP(hipMalloc(&d_bad, sizeof(int)));
   MF_HIP(hipMemsetAsync(d_bad, 0, sizeof(int), s));
   const DgIluLay Y = ilu_layout(D);
+  int M = D.mixed ? 0 : D.ns;
+  if (D.mixed)
+    for (int d : D.deg) M = std::max(M, ns_of_deg(d));
   for (int l = 0; l < D.ilu_f.launches(); l++) {
     const int c0 = D.ilu_f.row_ptr[l], cnt = D.ilu_f.row_ptr[l + 1] - c0;
-    hipLaunchKernelGGL(k_dg_ilu_row, dim3(cnt), dim3(64), 0, s, cnt,
-                       (const int*)D.ilu_f.d_rows + c0, Y, D.d_ilu, D.d_ilu_inv, d_bad);
+    hipLaunchKernelGGL(k_dg_ilu_row, dim3(cnt), dim3(M <= 10 ? 64 : 256),
+                       4 * M * M * sizeof(double), s, (const int*)D.ilu_f.d_rows + c0, Y, M,
+                       D.d_ilu, D.d_ilu_inv, d_bad);
   }
   int bad = 0;
   hipError_t e = hipGetLastError();
