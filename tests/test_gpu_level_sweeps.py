@@ -92,3 +92,38 @@ def test_substitution(kind, n, order, mixed):
     # FP32: factors, basis and corrections rounded, sums in FP64
     check([sp.csr_matrix(L), U], xe, be, 2.0 ** -24 if mixed else 2.0 ** -53, 12)
     p.free()
+
+
+@pytest.mark.parametrize("kind,n,half", [("grid", 20, 0), ("band", 700, 13), ("band", 700, 16),
+                                         ("band", 700, 31), ("band", 700, 32), ("band", 700, 35),
+                                         ("band", 5, 3), ("band", 900, 110)])
+@pytest.mark.parametrize("order", [0, 1])
+def test_factors(kind, n, half, order):
+    """L U against the matrix on its pattern for rows around 32 and 64
+    entries (one, two and eight per lane), rows of one level that end inside
+    a block: |L U - A| <= gamma |L| |U| entrywise"""
+    print("factors", kind, n, half, order, flush=True)
+    rng = np.random.default_rng(n + half)
+    if kind == "grid":
+        A, b, p = problem(kind, n)
+    else:
+        off = [o for o in range(-half, half + 1) if o and abs(o) < n]
+        A = sp.csr_matrix(sp.diags([1] * len(off), off, shape=(n, n)))
+        A.data = rng.uniform(-1, 1, A.nnz)
+        A = sp.csr_matrix(A + sp.diags(np.asarray(abs(A).sum(1)).ravel() + 0.1))
+        A.sort_indices()
+        p = mf.Problem.from_crs(A.indptr, A.indices, A.data, np.ones(n))
+    p.set_ilu_order(order)
+    lu, pos, _ = p.ilu()
+    rows = np.repeat(np.arange(A.shape[0]), np.diff(A.indptr))
+    r, c = pos[rows], pos[A.indices]
+    low = r > c
+    d = np.where(r == c, 1.0 / lu, lu)
+    L = sp.csr_matrix((lu[low], (r[low], c[low])), shape=A.shape) + sp.identity(A.shape[0])
+    U = sp.csr_matrix((d[~low], (r[~low], c[~low])), shape=A.shape)
+    at = lambda M: np.asarray(sp.csr_matrix(M)[r, c]).ravel()  # noqa: E731
+    g = (np.diff(A.indptr).max() + 4) * 2.0 ** -53
+    err, bound = abs(at(L @ U) - A.data), g * 2 * at(abs(L) @ abs(U))
+    print("worst / bound", (err / bound).max(), flush=True)
+    assert (err <= bound).all()
+    p.free()
