@@ -34,9 +34,9 @@ __global__ void k_ilu_load(long long nnz, const long long* src, const double* va
 // (E each): the lower entries in order, a_ik <- a_ik / u_kk and a_ij <- a_ij -
 // a_ik u_kj.  Row k's entries right of its diagonal are read by the lanes
 // together, those of the next k while this one's are searched for the row's
-// columns (ascending, five steps).  A level is bound by its rows' chains of loads: a thread per row
-// that merged two sorted rows took 197 us a level at 64^3 (25,000 rows of
-// 21), this 32 us
+// columns (ascending, five steps).  A level is bound by its rows' chains of
+// loads: a thread per row that merged two sorted rows took 197 us a level at
+// 64^3 (25,000 rows of 21), this 32 us
 template <int E>
 __global__ void __launch_bounds__(256) k_ilu_factor_level(const int* rows, int count,
                                                           const int* rp, const int* ci,
