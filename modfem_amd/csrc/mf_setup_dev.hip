@@ -164,30 +164,67 @@ __global__ void k_low_half(long long m, const unsigned long long* key, int* out)
   if (i < m) out[i] = (int)(key[i] & 0xffffffffu);
 }
 
+// a few blocks, one atomic per wavefront: 4,287 atomics on one address (one
+// per 64 rows) take 50 us
 __global__ void k_row_max(int n, const int* ptr, int* mx) {
-  const int r = blockIdx.x * TPB + threadIdx.x;
-  if (r < n) atomicMax(mx, ptr[r + 1] - ptr[r]);
+  int m = 0;
+  for (int r = blockIdx.x * TPB + threadIdx.x; r < n; r += gridDim.x * TPB)
+    m = max(m, ptr[r + 1] - ptr[r]);
+  for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o));
+  if ((threadIdx.x & 63) == 0) atomicMax(mx, m);
 }
 
-// compact element table: position of column dof(u) inside row dof(w)
-__global__ void k_el_off(int nel, int K, const int* el_dof, const int* row_ptr,
-                         const int* col_ind, uint8_t* el_off, int* bad) {
-  const long long t = (long long)blockIdx.x * TPB + threadIdx.x;
-  if (t >= (long long)nel * 36) return;
-  const int e = (int)(t % nel), q = (int)(t / nel), w = q / 6, u = q % 6;
-  uint8_t o = 0;
-  if (w < K && u < K) {
-    const int r = el_dof[(size_t)w * nel + e], c = el_dof[(size_t)u * nel + e];
-    int lo = row_ptr[r], hi = row_ptr[r + 1];
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (col_ind[mid] < c) lo = mid + 1;
-      else hi = mid;
+// compact element table: position of column dof(u) inside row dof(w).  32
+// lanes take 32 consecutive elements and one w: each row is read by the lanes
+// together and compared with the element's columns.  Bound by reading the
+// rows, a line or two each; one thread per entry, whose binary search made
+// nine dependent loads of other lines than its neighbours', took 1.06 ms at
+// 64^3 prisms, this 0.18 ms
+__global__ void __launch_bounds__(TPB) k_el_off(int nel, int K, const int* el_dof,
+                                                const int* row_ptr, const int* col_ind,
+                                                uint8_t* el_off, int* bad) {
+  const int nb = (nel + 31) / 32, g = blockIdx.x * (TPB / 32) + threadIdx.x / 32;
+  if (g >= 6 * nb) return;
+  const int w = g / nb, l = threadIdx.x & 31, sh = threadIdx.x & 32, e = g % nb * 32 + l;
+  const bool live = e < nel;
+  int o[6] = {0, 0, 0, 0, 0, 0}, c[6], found = 0;
+  if (w < K) {
+    const int r = live ? el_dof[(size_t)w * nel + e] : 0;
+#pragma unroll
+    for (int u = 0; u < 6; u++) c[u] = live && u < K ? el_dof[(size_t)u * nel + e] : -1;
+    const int a = row_ptr[r], n = live ? row_ptr[r + 1] - a : 0;
+    auto match = [&](int it, int k0, int col) {
+#pragma unroll
+      for (int u = 0; u < 6; u++) {
+        const int cu = __shfl(c[u], it, 32);
+        const unsigned m = (unsigned)(__ballot(col == cu) >> sh);
+        if (m && l == it) {
+          o[u] = k0 + __ffs(m) - 1;
+          found |= 1 << u;
+        }
+      }
+    };
+    constexpr int IF = 8;  // rows in flight
+    for (int i0 = 0; i0 < 32; i0 += IF) {
+      int col[IF];
+#pragma unroll
+      for (int i = 0; i < IF; i++) {
+        const int ai = __shfl(a, i0 + i, 32), ni = __shfl(n, i0 + i, 32);
+        col[i] = l < ni ? col_ind[ai + l] : -2;
+      }
+#pragma unroll
+      for (int i = 0; i < IF; i++) match(i0 + i, 0, col[i]);
     }
-    if (lo < row_ptr[r + 1] && col_ind[lo] == c) o = (uint8_t)(lo - row_ptr[r]);
-    else atomicAdd(bad, 1);
+    for (int i = 0; i < 32; i++) {  // rows of more than 32 entries
+      const int ai = __shfl(a, i, 32), ni = __shfl(n, i, 32);
+      for (int k0 = 32; k0 < ni; k0 += 32)
+        match(i, k0, k0 + l < ni ? col_ind[ai + k0 + l] : -2);
+    }
+    if (live && found != (1 << K) - 1) atomicAdd(bad, 1);
   }
-  el_off[t] = o;
+  if (live)
+#pragma unroll
+    for (int u = 0; u < 6; u++) el_off[(size_t)(w * 6 + u) * nel + e] = (uint8_t)o[u];
 }
 
 // boundary-face incidence pairs through the owning element's DOFs
@@ -427,11 +464,11 @@ int problem_setup_device(const Mesh& M, Problem& P) {
                      row_ptr.p);
   hipLaunchKernelGGL(k_low_half, dim3(grid_of(nnz)), dim3(TPB), 0, s, (long long)nnz, pku.p, col_ind.p);
   MF_HIP(hipMemsetAsync(mx.p, 0, 2 * sizeof(int), s));
-  hipLaunchKernelGGL(k_row_max, dim3(grid_of(n)), dim3(TPB), 0, s, n, row_ptr.p, mx.p);
+  hipLaunchKernelGGL(k_row_max, dim3(std::min(grid_of(n), 64u)), dim3(TPB), 0, s, n, row_ptr.p, mx.p);
   // element tables
   DevArr<uint8_t> el_off;
   if (el_off.alloc(36 * (size_t)nel)) return -2;
-  hipLaunchKernelGGL(k_el_off, dim3(grid_of((long long)nel * 36)), dim3(TPB), 0, s, nel, K,
+  hipLaunchKernelGGL(k_el_off, dim3(grid_of((nel + 31) / 32 * 6 * 32LL)), dim3(TPB), 0, s, nel, K,
                      el_dof.p, row_ptr.p, col_ind.p, el_off.p, mx.p + 1);
   int hm[2];
   MF_HIP(hipMemcpyAsync(hm, mx.p, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
