@@ -482,8 +482,10 @@ __device__ __forceinline__ void ilu_row(const IluSweepArgs<FT>& W, int sl, int l
   v[i] = (VT)(BWD ? t * (double)d : t);
 }
 
-// wavefronts per block of a launch over nsl slices: small launches spread
-// over all CUs
+// wavefronts per block of a launch over nsl slices.  Up to one slice per CU a
+// block of one wavefront reaches a CU of its own, up to two a block of two;
+// beyond that a block of four costs the fewest dispatches.  Measured together
+// with packed_row_sum: a colour of 20 slices 3.9 us in blocks of four, 3.5 us
 inline int sweep_waves(int nsl, int cus) { return nsl <= cus ? 1 : nsl <= 2 * cus ? 2 : 4; }
 
 // FP64 data of a mixed-precision batch member's refinement steps
