@@ -468,13 +468,13 @@ struct DgNb {
   int x, n;
 };
 
-// rows of the block system in an order of launches (dependency levels): the
-// device tables of k_dg_rows and the bounds of its launches
+// rows of the block system in an order of launches (dependency levels,
+// colours): the device tables of k_dg_rows and the bounds of its launches
 struct DgRowSet {
   std::vector<int> row_ptr;   // rows of launch l: [row_ptr[l], row_ptr[l + 1])
-  std::vector<int> task_ptr;  // mixed problems: its blocks
+  std::vector<int> task_ptr;  // mixed problems: its tasks
   int* d_rows = nullptr;
-  int* d_nbl = nullptr;
+  int* d_nbl = nullptr;       // uniform problems: neighbours in the sum, -1 none
   int4* d_tasks = nullptr;
   DgNb* d_nb = nullptr;
   int* d_xoff = nullptr;
@@ -2205,8 +2205,8 @@ __global__ void __launch_bounds__(256) k_dg_ilu_row(const int* rows, DgIluLay Y,
 // q over the row's listed neighbour blocks (OWN: and its own block; s =
 // sc[j], 1 without sc).  In place (y = v) a launch's rows must not be
 // neighbours: one dependency level or colour.  A level holds a few hundred
-// rows, so the launch is bound by the latency of its longest chain of
-// loads, not by bandwidth: one lane per unknown walking its up to 200
+// rows, so the launch is bound by the latency of its longest chain
+// of loads, not by bandwidth: one lane per unknown walking its up to 200
 // columns took 39-43 us a level (16^3 mixed degrees).  Here a row's columns
 // are dealt to S >= 6 lane groups (lane = (row, group, unknown)), so a lane
 // has at most 7 columns of a block, the loads of three blocks and of the
@@ -2370,6 +2370,42 @@ __global__ void __launch_bounds__(256) k_dg_rows(DgRowList R, const double* A, c
   if (act && u == 0) y[xe + r] = s * t;
 }
 
+// the tables of a row set from its list of rows: a uniform problem's
+// neighbours per side; a mixed one's unknowns, blocks and neighbour records,
+// largest neighbour first.  which: all neighbours (0), the lower ones (-1),
+// the upper ones (1)
+__global__ void __launch_bounds__(256) k_dg_row_tables(int cnt, const int* rows, const int* fnb,
+                                                       const int* deg, const long long* xoff,
+                                                       const long long* soff,
+                                                       const long long* voff, int which, int* nbl,
+                                                       DgNb* nb, int* xo, long long* ao,
+                                                       long long* vo) {
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  if (p >= cnt) return;
+  const int e = rows[p];
+  int k[5], n[5];
+#pragma unroll
+  for (int s = 0; s < 5; s++) {
+    k[s] = fnb[5 * (size_t)e + s];
+    if (which < 0 ? k[s] >= e : which > 0 && k[s] <= e) k[s] = -1;
+    if (nbl) nbl[5 * (size_t)p + s] = k[s] < 0 ? -1 : k[s];
+    n[s] = nb && k[s] >= 0 ? ns_of_deg(deg[k[s]]) : 0;
+  }
+  if (!nb) return;
+  const int x = (int)xoff[e];
+  xo[p] = x;
+  ao[p] = soff[6 * (size_t)e];
+  vo[p] = voff[e];
+#pragma unroll
+  for (int s = 0; s < 5; s++) {
+    int at = 0;
+#pragma unroll
+    for (int t = 0; t < 5; t++) at += n[t] > n[s] || (n[t] == n[s] && t < s);
+    nb[5 * (size_t)p + at] =
+        DgNb{soff[6 * (size_t)e + 1 + s], n[s] ? (int)xoff[k[s]] : x, n[s]};
+  }
+}
+
 // w = s_j v and y = w (start of a GS-smoothed operator application)
 __global__ void k_dg_scale2(long long n, const double* v, const double* sc, int j, double* w,
                             double* y, const int* stop) {
@@ -2393,119 +2429,128 @@ __global__ void k_dg_sub(long long n, const double* y, double* w, const int* sto
 namespace {
 
 template <typename T>
+int row_set_up(T** d, size_t n) {
+  MF_HIP(hipMalloc(d, std::max<size_t>(n, 1) * sizeof(T)));
+  return 0;
+}
+
+template <typename T>
 int row_set_up(T** d, const std::vector<T>& h) {
-  MF_HIP(hipMalloc(d, std::max<size_t>(h.size(), 1) * sizeof(T)));
+  if (row_set_up(d, h.size())) return -2;
   MF_HIP(hipMemcpy(*d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
   return 0;
 }
 
-// device tables of the rows listed launch by launch in `rows`; take(e, nb)
-// says which neighbours belong to a row's sum.  Within a launch the rows of
-// a mixed problem are ordered by their own and their neighbours' sizes, so
-// that a block's rows share them
-template <class Take>
+// device tables of the rows listed launch by launch in `rows`, for sums over
+// all neighbours (which 0), the lower (-1) or the upper ones (1)
 int build_row_set(DgProblem& D, DgRowSet& R, std::vector<int> rows, std::vector<int> row_ptr,
-                  Take take) {
+                  int which) {
   const size_t cnt = rows.size();
   R.row_ptr = std::move(row_ptr);
-  if (!D.mixed) {
-    std::vector<int> nbl(5 * cnt);
-    for (size_t p = 0; p < cnt; p++)
-      for (int s = 0; s < 5; s++) {
-        const int nb = D.h_fnb[5 * (size_t)rows[p] + s];
-        nbl[5 * p + s] = nb >= 0 && take(rows[p], nb) ? nb : -1;
-      }
-    return row_set_up(&R.d_nbl, nbl) || row_set_up(&R.d_rows, rows) ? -2 : 0;
-  }
-  auto nse = [&D](int e) { return ns_of_deg(D.deg[e]); };
-  // the sides of a row's sum, largest neighbour first: their columns (0: not
-  // in the sum), and one number to sort the rows by (own size, then columns)
-  struct Sides {
-    uint64_t key;
-    unsigned char n[5], side[5];
-  };
-  std::vector<Sides> sides(D.nel);
-  for (int e = 0; e < D.nel; e++) {
-    Sides& v = sides[e];
-    for (int s = 0; s < 5; s++) {
-      const int nb = D.h_fnb[5 * (size_t)e + s];
-      const unsigned char c = nb >= 0 && take(e, nb) ? (unsigned char)nse(nb) : 0;
-      int t = s;
-      for (; t > 0 && v.n[t - 1] < c; t--) {
-        v.n[t] = v.n[t - 1];
-        v.side[t] = v.side[t - 1];
-      }
-      v.n[t] = c;
-      v.side[t] = (unsigned char)s;
-    }
-    v.key = (uint64_t)nse(e);
-    for (int t = 0; t < 5; t++) v.key = v.key << 8 | (255 - v.n[t]);
-  }
   std::vector<int4> tasks;
-  R.task_ptr.assign(1, 0);
-  for (int l = 0; l < R.launches(); l++) {
-    const int end = R.row_ptr[l + 1];
-    std::stable_sort(rows.begin() + R.row_ptr[l], rows.begin() + end,
-                     [&](int a, int b) { return sides[a].key < sides[b].key; });
-    for (int q = R.row_ptr[l]; q < end;) {
-      const int ns = nse(rows[q]), rb = row_block_rows(ns, true), S = row_groups(ns, true);
-      int c = 0, cols = 0;
-      for (; c < rb && q + c < end && nse(rows[q + c]) == ns; c++) {
-        for (int t = 0; t < 5; t++) {
-          const int kc = (sides[rows[q + c]].n[t] + S - 1) / S;
-          if (kc > (cols >> 3 * t & 7)) cols = (cols & ~(7 << 3 * t)) | kc << 3 * t;
-        }
+  if (D.mixed) {
+    auto nse = [&D](int e) { return ns_of_deg(D.deg[e]); };
+    // the columns of a row's neighbours, largest first (0: not in the sum)
+    auto columns = [&](int e, unsigned char (&n)[5]) {
+      for (int s = 0; s < 5; s++) {
+        const int nb = D.h_fnb[5 * (size_t)e + s];
+        const bool in = nb >= 0 && (which == 0 || (which < 0 ? nb < e : nb > e));
+        const unsigned char c = in ? (unsigned char)nse(nb) : 0;
+        int t = s;
+        for (; t > 0 && n[t - 1] < c; t--) n[t] = n[t - 1];
+        n[t] = c;
       }
-      tasks.push_back(make_int4(q, c, ns, cols));
-      q += c;
+    };
+    R.task_ptr.assign(1, 0);
+    std::vector<uint64_t> key;
+    std::vector<int> list;
+    for (int l = 0; l < R.launches(); l++) {
+      const int p0 = R.row_ptr[l], p1 = R.row_ptr[l + 1];
+      list.assign(rows.begin() + p0, rows.begin() + p1);
+      // rows of one block have one size and share their numbers of columns
+      // per lane: by size, then by the neighbours' columns; six bits each
+      // above the place in the given order
+      key.clear();
+      for (size_t k = 0; k < list.size(); k++) {
+        unsigned char n[5];
+        columns(list[k], n);
+        uint64_t v = (uint64_t)nse(list[k]);
+        for (int t = 0; t < 5; t++) v = v << 6 | (63 - n[t]);
+        key.push_back(v << 28 | k);
+      }
+      std::sort(key.begin(), key.end());
+      for (size_t k = 0; k < key.size(); k++) rows[p0 + k] = list[key[k] & 0xfffffff];
+      for (int q = p0; q < p1;) {
+        const int ns = nse(rows[q]), rb = row_block_rows(ns, true);
+        const int S = row_groups(ns, true);
+        int c = 0, cols = 0;
+        for (; c < rb && q + c < p1 && nse(rows[q + c]) == ns; c++) {
+          unsigned char n[5];
+          columns(rows[q + c], n);
+          for (int t = 0; t < 5; t++) {
+            const int kc = (n[t] + S - 1) / S;
+            if (kc > (cols >> 3 * t & 7)) cols = (cols & ~(7 << 3 * t)) | kc << 3 * t;
+          }
+        }
+        tasks.push_back(make_int4(q, c, ns, cols));
+        q += c;
+      }
+      R.task_ptr.push_back((int)tasks.size());
     }
-    R.task_ptr.push_back((int)tasks.size());
   }
-  std::vector<DgNb> nbs(5 * cnt);
-  std::vector<int> xo(cnt);
-  std::vector<long long> ao(cnt), vo(cnt);
-  for (size_t p = 0; p < cnt; p++) {
-    const size_t e = rows[p];
-    xo[p] = (int)D.xoff[e];
-    ao[p] = D.soff[6 * e];
-    vo[p] = D.voff[e];
-    for (int t = 0; t < 5; t++) {
-      const int s = sides[e].side[t];
-      DgNb& d = nbs[5 * p + t];
-      d.a = D.soff[6 * e + 1 + s];
-      d.n = sides[e].n[t];
-      d.x = d.n ? (int)D.xoff[D.h_fnb[5 * e + s]] : xo[p];
+  // d_rows last: it says that the set is complete
+  int* d_rows = nullptr;
+  int rc = row_set_up(&d_rows, rows);
+  auto room = [&](auto** d, size_t n) {
+    if (rc == 0) rc = row_set_up(d, n);
+  };
+  if (D.mixed) {
+    if (rc == 0) rc = row_set_up(&R.d_tasks, tasks);
+    room(&R.d_nb, 5 * cnt);
+    room(&R.d_xoff, cnt);
+    room(&R.d_aoff, cnt);
+    room(&R.d_voff, cnt);
+  } else {
+    room(&R.d_nbl, 5 * cnt);
+  }
+  if (rc == 0) {
+    hipLaunchKernelGGL(k_dg_row_tables, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, stream(),
+                       (int)cnt, d_rows, D.d_fnb, D.d_deg, D.d_xoff, D.d_soff, D.d_voff, which,
+                       R.d_nbl, R.d_nb, R.d_xoff, R.d_aoff, R.d_voff);
+    if (hipGetLastError() != hipSuccess) {
+      set_error("DG row tables: launch failed");
+      rc = -2;
     }
   }
-  if (row_set_up(&R.d_tasks, tasks) || row_set_up(&R.d_nb, nbs) || row_set_up(&R.d_xoff, xo) ||
-      row_set_up(&R.d_aoff, ao) || row_set_up(&R.d_voff, vo) || row_set_up(&R.d_rows, rows))
-    return -2;
+  if (rc) {
+    (void)hipFree(d_rows);
+    return rc;
+  }
+  R.d_rows = d_rows;
   return 0;
 }
 
+// launch l of the set
 template <bool OWN>
-void launch_row_list(const DgProblem& D, const DgRowList& L, const double* A, const double* Dinv,
-                     const double* b, const double* v, double* y, const double* sc, int j,
-                     const int* stop) {
+void launch_row_list(const DgProblem& D, const DgRowSet& R, int l, const double* A,
+                     const double* Dinv, const double* b, const double* v, double* y,
+                     const double* sc, int j, const int* stop) {
+  const std::vector<int>& ptr = D.mixed ? R.task_ptr : R.row_ptr;
+  const DgRowList L{D.ns,      ptr[l], ptr[l + 1] - ptr[l], R.d_rows,  R.d_nbl,
+                    R.d_tasks, R.d_nb, R.d_xoff,            R.d_aoff, R.d_voff};
   if (L.cnt == 0) return;
   const int rb = D.mixed ? 1 : row_block_rows(D.ns, false);
-  const dim3 g((L.cnt + rb - 1) / rb);
   // the operator of a uniform problem has its own kernel (k_dg_op)
   auto k = D.mixed ? (Dinv ? k_dg_rows<true, true, OWN> : k_dg_rows<true, false, OWN>)
                    : (Dinv ? k_dg_rows<false, true, false> : k_dg_rows<false, false, false>);
-  hipLaunchKernelGGL(k, g, dim3(256), 0, stream(), L, A, Dinv, b, v, y, sc, j, stop);
-}
-
-DgRowList row_list(const DgProblem& D, const DgRowSet& R, int l) {
-  const std::vector<int>& ptr = D.mixed ? R.task_ptr : R.row_ptr;
-  return DgRowList{D.ns,      ptr[l], ptr[l + 1] - ptr[l], R.d_rows,  R.d_nbl,
-                   R.d_tasks, R.d_nb, R.d_xoff,            R.d_aoff, R.d_voff};
+  hipLaunchKernelGGL(k, dim3((L.cnt + rb - 1) / rb), dim3(256), 0, stream(), L, A, Dinv, b, v, y,
+                     sc, j, stop);
 }
 
 // launch l of the set, in place: v_e = [Dinv_e] (b_e - sum A x) over its rows
 void launch_rows(const DgProblem& D, const DgRowSet& R, int l, const double* A, const double* Dinv,
                  const double* b, double* v, const int* stop) {
-  launch_row_list<false>(D, row_list(D, R, l), A, Dinv, b, v, v, nullptr, 0, stop);
+  launch_row_list<false>(D, R, l, A, Dinv, b, v, v, nullptr, 0, stop);
 }
 
 }  // namespace
@@ -2564,17 +2609,7 @@ struct DgOp : ExtOp {
   int op(const double* x, const double* b, const double* sc, int j, const int* stop, double* w,
          int mode) {
     if (D->mixed) {
-      DgRowSet& R = D->op_rows;
-      if (!R.built()) {
-        // one launch over all degrees, rows in the order of their blocks
-        std::vector<int> rows(D->nel);
-        for (int e = 0; e < D->nel; e++) rows[e] = e;
-        std::stable_sort(rows.begin(), rows.end(),
-                         [this](int a, int c) { return D->deg[a] < D->deg[c]; });
-        R.free_all();
-        if (build_row_set(*D, R, rows, {0, D->nel}, [](int, int) { return true; })) return -2;
-      }
-      launch_row_list<true>(*D, row_list(*D, R, 0), D->d_blk, precon == 1 ? D->d_dinv : nullptr,
+      launch_row_list<true>(*D, D->op_rows, 0, D->d_blk, precon == 1 ? D->d_dinv : nullptr,
                             mode == 1 ? b : nullptr, x, w, mode == 1 ? nullptr : sc, j, stop);
       MF_HIP(hipGetLastError());
       return 0;
@@ -2809,7 +2844,7 @@ int build_gs_colors(DgProblem& D) {
   for (int c = 0; c < ncol; c++) ptr[c + 1] += ptr[c];
   std::vector<int> pos(ptr.begin(), ptr.end() - 1), elems(D.nel);
   for (int e = 0; e < D.nel; e++) elems[pos[col[e]]++] = e;
-  if (build_row_set(D, D.gs_rows, elems, ptr, [](int, int) { return true; })) return -2;
+  if (build_row_set(D, D.gs_rows, elems, ptr, 0)) return -2;
   if (!D.d_work) MF_HIP(hipMalloc(&D.d_work, (size_t)D.ndof * sizeof(double)));
   return 0;
 }
@@ -2890,9 +2925,7 @@ int build_ilu_levels(DgProblem& D) {
   };
   std::vector<int> fp, bp;
   const std::vector<int> fr = listed(lf, nlf, fp), br = listed(lb, nlb, bp);
-  if (build_row_set(D, D.ilu_f, fr, fp, [](int e, int nb) { return nb < e; }) ||
-      build_row_set(D, D.ilu_b, br, bp, [](int e, int nb) { return nb > e; }))
-    return -2;
+  if (build_row_set(D, D.ilu_f, fr, fp, -1) || build_row_set(D, D.ilu_b, br, bp, 1)) return -2;
   return 0;
 }
 
@@ -3333,6 +3366,11 @@ int dg_create(int mesh, const std::vector<int>& pdeg) {
     MF_HIP(hipMalloc(&D->d_slots, slots.size() * sizeof(int)));
     MF_HIP(hipMemcpyAsync(D->d_slots, slots.data(), slots.size() * sizeof(int),
                           hipMemcpyHostToDevice, stream()));
+  }
+  // the operator's rows of a mixed problem: one launch over all degrees
+  if (mixed && build_row_set(*D, D->op_rows, grp, {0, (int)nel}, 0)) {
+    free_dg(*D);
+    return -2;
   }
   MF_HIP(hipStreamSynchronize(stream()));
   const int id = g_next_dg++;
@@ -4028,7 +4066,7 @@ int mf_dg_bench(int did, int reps, double* out) {
   DgOp op;
   op.D = D;
   op.precon = 1;
-  int rc = 0;
+  int rc = op.run_all(x, nullptr, nullptr, 0, nullptr, w, 0);  // not timed
   for (int r = 0; r < reps && rc == 0; r++) {
     float ms = 0;
     MF_HIP(hipEventRecord(ev[0], s));
