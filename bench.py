@@ -755,7 +755,7 @@ def bench_dg(args):
                      "traffic": None, "kernel": "k_dg_diag + k_dg_couple, mixed degrees"},
         "roofline_op": {"bound": "hbm", "achieved": r["op_GBs"], "peak": HBM_PEAK_GBS,
                         "unit": "GB/s", "frac": r["op_GBs"] / HBM_PEAK_GBS,
-                        "kernel": "k_dg_rows (operator and block Jacobi), mixed degrees"},
+                        "kernel": "k_dg_rows_wave (operator and block Jacobi), mixed degrees"},
     }
     if not args.no_cpu:
         lv = [res[str(p)] for p in (101, 202, 303) if str(p) in res]

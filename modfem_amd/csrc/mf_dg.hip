@@ -469,9 +469,11 @@ struct DgNb {
 };
 
 // rows of the block system in an order of launches (dependency levels,
-// colours): the device tables of k_dg_rows and the bounds of its launches
+// colours): the device tables of the row-sum kernels and the bounds of their
+// launches
 struct DgRowSet {
   std::vector<int> row_ptr;   // rows of launch l: [row_ptr[l], row_ptr[l + 1])
+  std::vector<char> wave;     // its kernel: k_dg_rows_wave, else k_dg_rows
   std::vector<int> task_ptr;  // mixed problems: its tasks
   int* d_rows = nullptr;
   int* d_nbl = nullptr;       // uniform problems: neighbours in the sum, -1 none
@@ -2204,8 +2206,8 @@ __global__ void __launch_bounds__(256) k_dg_ilu_row(const int* rows, DgIluLay Y,
 //   y_e = s t  or  y_e = s Dinv_e t,
 // q over the row's listed neighbour blocks (OWN: and its own block; s =
 // sc[j], 1 without sc).  In place (y = v) a launch's rows must not be
-// neighbours: one dependency level or colour.  A level holds a few hundred
-// rows, so the launch is bound by the latency of its longest chain
+// neighbours: one dependency level or colour.  This is the kernel of launches
+// of few rows (a level of hundreds), bound by the latency of the longest chain
 // of loads, not by bandwidth: one lane per unknown walking its up to 200
 // columns took 39-43 us a level (16^3 mixed degrees).  Here a row's columns
 // are dealt to S >= 6 lane groups (lane = (row, group, unknown)), so a lane
@@ -2370,6 +2372,103 @@ __global__ void __launch_bounds__(256) k_dg_rows(DgRowList R, const double* A, c
   if (act && u == 0) y[xe + r] = s * t;
 }
 
+// acc + the products of n columns of a block (ld rows) with x, six in flight
+// together; past the last one the loads repeat it and the select drops them
+__device__ __forceinline__ double dg_columns(double acc, const double* B, int ld, const double* x,
+                                             int n) {
+  int c = 0;
+  for (; c + 6 <= n; c += 6) {
+    double m[6], w[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+      m[k] = B[(c + k) * ld];
+      w[k] = x[c + k];
+    }
+#pragma unroll
+    for (int k = 0; k < 6; k++) acc += m[k] * w[k];
+  }
+  for (; c < n; c += 4) {
+    double m[4], w[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int q = min(c + k, n - 1);
+      m[k] = B[q * ld];
+      w[k] = x[q];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) acc += c + k < n ? m[k] * w[k] : 0.0;
+  }
+  return acc;
+}
+
+// The same row sums for a launch of many rows, which is bound by the bytes of
+// its blocks: a wavefront owns 64 / ns rows, lane = (row, unknown), every lane
+// sums its row's columns six at a time, and lanes meet for the inverse only.
+// 96^3 prisms of degrees 1 to 3 (37.7 M unknowns, 52.6 GB of blocks and
+// inverses): operator 13.8 ms with k_dg_rows, 11.5 ms with this (4.6 TB/s);
+// a GMRES step with two Gauss-Seidel sweeps 36.2 -> 22.0 ms
+template <bool MIXED, bool INV, bool OWN>
+__global__ void __launch_bounds__(256) k_dg_rows_wave(DgRowList R, const double* A,
+                                                      const double* Dinv, const double* b,
+                                                      const double* v, double* y,
+                                                      const double* sc, int j, const int* stop) {
+  __shared__ double tw[4][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int t = blockIdx.x * 4 + wave;
+  const int halt = stop ? *stop : 0;
+  const double s = sc ? sc[j] : 1.0;
+  int ns = R.ns, p0, nrow;
+  if (MIXED) {
+    if (t >= R.cnt) return;
+    const int4 tk = R.tasks[R.first + t];
+    p0 = tk.x;
+    nrow = tk.y;
+    ns = tk.z;
+  } else {
+    const int rw = 64 / ns;
+    p0 = R.first + t * rw;
+    nrow = min(rw, R.first + R.cnt - p0);
+    if (nrow <= 0) return;
+  }
+  if (halt) return;
+  const int row = lane / ns, r = lane - row * ns;
+  const bool act = row < nrow;
+  const int p = act ? p0 + row : p0;
+  const int e = MIXED ? 0 : R.rows[p];
+  const int xe = MIXED ? R.xoff[p] : e * ns;
+  double acc = 0.0, own = 0.0;
+  if (act) {
+    if (b) own = b[xe + r];
+#pragma unroll 1
+    for (int q = 0; q < 5; q++) {
+      DgNb d;
+      if (MIXED) {
+        d = R.nb[5 * (size_t)p + q];
+      } else {
+        const int nb = R.nbl[5 * (size_t)p + q];
+        d.a = ((long long)e * 6 + 1 + q) * ns * ns;
+        d.n = nb < 0 ? 0 : ns;
+        d.x = nb < 0 ? 0 : nb * ns;
+      }
+      acc = dg_columns(acc, A + d.a + r, ns, v + d.x, d.n);
+    }
+    if (OWN)
+      acc = dg_columns(acc, A + (MIXED ? R.aoff[p] : (long long)e * 6 * ns * ns) + r, ns, v + xe,
+                       ns);
+    if (!OWN || b) acc = own - acc;
+  }
+  if (INV) {
+    tw[wave][lane] = acc;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (act)
+      acc = dg_columns(0.0, Dinv + (MIXED ? R.voff[p] : (long long)e * ns * ns) + r, ns,
+                       &tw[wave][row * ns], ns);
+  }
+  if (act) y[xe + r] = s * acc;
+}
+
 // the tables of a row set from its list of rows: a uniform problem's
 // neighbours per side; a mixed one's unknowns, blocks and neighbour records,
 // largest neighbour first.  which: all neighbours (0), the lower ones (-1),
@@ -2441,13 +2540,30 @@ int row_set_up(T** d, const std::vector<T>& h) {
   return 0;
 }
 
+// From how many unknowns per CU a launch takes k_dg_rows_wave: about four
+// wavefronts on every CU.  Below, a launch lasts as long as one row's chain
+// and k_dg_rows cuts that chain; above, its idle lanes and barriers cost more
+// than the chain.  Time per GMRES iteration with block ILU(0), split rows
+// against one lane per unknown: uniform degree 1, 32^3 (48 unknowns per CU
+// in the longest level) 0.52 / 0.61 ms, 96^3 (430) 3.97 / 3.40; degree 2,
+// 32^3 (144) 1.19 / 1.30 ms, 40^3 (225) 2.16 / 1.84, 96^3 (1296) 23.6 / 15.4;
+// degree 3, 24^3 (180) 1.78 / 2.09 ms, 32^3 (320) 3.63 / 3.38.  In a mixed
+// launch the rows of a wavefront wait for its widest one: degrees 2 and 3,
+// 32^3 (232) 2.36 / 2.56 ms; degrees 1 to 3, 40^3 (267) 3.01 / 3.00 ms, 96^3
+// (1530) 35.0 / 24.9; 96^3 prisms and tetrahedra 35.1 / 21.7 ms
+constexpr int kWaveUnknowns = 224, kWaveUnknownsMixed = 256;
+
 // device tables of the rows listed launch by launch in `rows`, for sums over
 // all neighbours (which 0), the lower (-1) or the upper ones (1)
 int build_row_set(DgProblem& D, DgRowSet& R, std::vector<int> rows, std::vector<int> row_ptr,
                   int which) {
   const size_t cnt = rows.size();
   R.row_ptr = std::move(row_ptr);
+  R.wave.resize(R.launches());
   std::vector<int4> tasks;
+  if (!D.mixed)
+    for (int l = 0; l < R.launches(); l++)
+      R.wave[l] = (long long)(R.row_ptr[l + 1] - R.row_ptr[l]) * D.ns >= kWaveUnknowns * D.ncu;
   if (D.mixed) {
     auto nse = [&D](int e) { return ns_of_deg(D.deg[e]); };
     // the columns of a row's neighbours, largest first (0: not in the sum)
@@ -2467,24 +2583,38 @@ int build_row_set(DgProblem& D, DgRowSet& R, std::vector<int> rows, std::vector<
     for (int l = 0; l < R.launches(); l++) {
       const int p0 = R.row_ptr[l], p1 = R.row_ptr[l + 1];
       list.assign(rows.begin() + p0, rows.begin() + p1);
-      // rows of one block have one size and share their numbers of columns
-      // per lane: by size, then by the neighbours' columns; six bits each
-      // above the place in the given order
-      key.clear();
-      for (size_t k = 0; k < list.size(); k++) {
-        unsigned char n[5];
-        columns(list[k], n);
-        uint64_t v = (uint64_t)nse(list[k]);
-        for (int t = 0; t < 5; t++) v = v << 6 | (63 - n[t]);
-        key.push_back(v << 28 | k);
+      int at[kIluMax + 2] = {0};
+      long long unknowns = 0;
+      for (int e : list) {
+        at[nse(e) + 1]++;
+        unknowns += nse(e);
       }
-      std::sort(key.begin(), key.end());
-      for (size_t k = 0; k < key.size(); k++) rows[p0 + k] = list[key[k] & 0xfffffff];
+      const bool wave = R.wave[l] = unknowns >= kWaveUnknownsMixed * D.ncu;
+      if (wave) {
+        // by size, in the given order within a size
+        for (int k = 0; k <= kIluMax; k++) at[k + 1] += at[k];
+        for (int e : list) rows[p0 + at[nse(e)]++] = e;
+      } else {
+        // rows of one block have one size and share their numbers of columns
+        // per lane: by size, then by the neighbours' columns; six bits each
+        // above the place in the given order
+        key.clear();
+        for (size_t k = 0; k < list.size(); k++) {
+          unsigned char n[5];
+          columns(list[k], n);
+          uint64_t v = (uint64_t)nse(list[k]);
+          for (int t = 0; t < 5; t++) v = v << 6 | (63 - n[t]);
+          key.push_back(v << 28 | k);
+        }
+        std::sort(key.begin(), key.end());
+        for (size_t k = 0; k < key.size(); k++) rows[p0 + k] = list[key[k] & 0xfffffff];
+      }
       for (int q = p0; q < p1;) {
-        const int ns = nse(rows[q]), rb = row_block_rows(ns, true);
+        const int ns = nse(rows[q]), rb = wave ? 64 / ns : row_block_rows(ns, true);
         const int S = row_groups(ns, true);
         int c = 0, cols = 0;
         for (; c < rb && q + c < p1 && nse(rows[q + c]) == ns; c++) {
+          if (wave) continue;
           unsigned char n[5];
           columns(rows[q + c], n);
           for (int t = 0; t < 5; t++) {
@@ -2539,10 +2669,19 @@ void launch_row_list(const DgProblem& D, const DgRowSet& R, int l, const double*
   const DgRowList L{D.ns,      ptr[l], ptr[l + 1] - ptr[l], R.d_rows,  R.d_nbl,
                     R.d_tasks, R.d_nb, R.d_xoff,            R.d_aoff, R.d_voff};
   if (L.cnt == 0) return;
-  const int rb = D.mixed ? 1 : row_block_rows(D.ns, false);
-  // the operator of a uniform problem has its own kernel (k_dg_op)
-  auto k = D.mixed ? (Dinv ? k_dg_rows<true, true, OWN> : k_dg_rows<true, false, OWN>)
-                   : (Dinv ? k_dg_rows<false, true, false> : k_dg_rows<false, false, false>);
+  // rows or tasks per block; the operator of a uniform problem has its own
+  // kernel (k_dg_op)
+  int rb;
+  auto k = k_dg_rows<true, true, OWN>;
+  if (R.wave[l]) {
+    rb = D.mixed ? 4 : 4 * (64 / D.ns);
+    k = D.mixed ? (Dinv ? k_dg_rows_wave<true, true, OWN> : k_dg_rows_wave<true, false, OWN>)
+                : (Dinv ? k_dg_rows_wave<false, true, false> : k_dg_rows_wave<false, false, false>);
+  } else {
+    rb = D.mixed ? 1 : row_block_rows(D.ns, false);
+    k = D.mixed ? (Dinv ? k_dg_rows<true, true, OWN> : k_dg_rows<true, false, OWN>)
+                : (Dinv ? k_dg_rows<false, true, false> : k_dg_rows<false, false, false>);
+  }
   hipLaunchKernelGGL(k, dim3((L.cnt + rb - 1) / rb), dim3(256), 0, stream(), L, A, Dinv, b, v, y,
                      sc, j, stop);
 }
