@@ -631,69 +631,121 @@ template <> struct Grp<float> {
   static constexpr int W = 4;
 };
 
-// block r of G of a member updates the row groups [r g / G, (r+1) g / G).
-// coef() makes the coefficients c_i, i <= j, visible to the block in cs; the
-// thread's w and first eight vectors are requested before it, and eight
-// vectors ahead from then on.  halt: nothing to do (tested after the requests)
-template <typename VT, class Coefs>
-__device__ __forceinline__ void update_body(const SolveArgs& A, int j, int r, int G, int pb,
-                                            const double* cs, int halt, Coefs coef) {
+// The update of block r of G of a member: the row groups [r g / G, (r+1) g /
+// G) of w, whose vectors V_0 .. V_j are Vg, ldg groups apart; the block's norm
+// goes to norms[pb].  cs: the coefficients c_i, i <= j, in shared memory.
+template <typename VT>
+struct UpdateRows {
   using GT = typename Grp<VT>::T;
-  constexpr int W = Grp<VT>::W, N = 8;
-  __shared__ double red[1];
-  const long long ng = (A.n + W - 1) / W;  // ldv is a multiple of W: whole groups stay inside
-  const long long p0 = r * ng / G, p1 = (r + 1) * ng / G;
-  const long long ldg = A.ldv / W;
-  const GT* VG = reinterpret_cast<const GT*>(basis<VT>(A));
-  GT* w = reinterpret_cast<GT*>(basis<VT>(A) + (size_t)(j + 1) * A.ldv);
+  static constexpr int W = Grp<VT>::W;
+  const GT* VG;
+  GT* w;
+  long long ldg, p0, p1;
+  int n;
   double acc = 0.0;
-  auto load = [&](long long p, GT& w0, GT (&v)[N]) {
-    w0 = w[p];
+  __device__ __forceinline__ UpdateRows(const SolveArgs& A, int j, int r, int G) : n(A.n) {
+    const long long ng = (A.n + W - 1) / W;  // ldv is a multiple of W: whole groups stay inside
+    p0 = r * ng / G;
+    p1 = (r + 1) * ng / G;
+    ldg = A.ldv / W;
+    VG = reinterpret_cast<const GT*>(basis<VT>(A));
+    w = reinterpret_cast<GT*>(basis<VT>(A) + (size_t)(j + 1) * A.ldv);
+  }
+  __device__ __forceinline__ void sub(double (&wv)[W], double c, const GT& v) {
 #pragma unroll
-    for (int q = 0; q < N; q++) v[q] = VG[(size_t)min(q, j) * ldg + p];
+    for (int e = 0; e < W; e++) wv[e] -= c * (double)v[e];
+  }
+  __device__ __forceinline__ void put(long long p, const double (&wv)[W]) {
+    GT wr;
+#pragma unroll
+    for (int e = 0; e < W; e++) {
+      const VT q = W * p + e < n ? (VT)wv[e] : (VT)0;  // padding rows stay zero
+      wr[e] = q;
+      acc += (double)q * (double)q;
+    }
+    w[p] = wr;
+  }
+};
+
+// The thread's w and first eight vectors are requested before coef() makes the
+// coefficients visible (it waits for the whole block, so the first rows stand
+// apart from the others), and eight vectors ahead from then on.  halt: nothing
+// to do (tested after the requests)
+template <typename VT, class Coefs>
+__device__ __forceinline__ void update_ahead(const SolveArgs& A, int j, int r, int G, int pb,
+                                             const double* cs, int halt, Coefs coef) {
+  using U = UpdateRows<VT>;
+  using GT = typename U::GT;
+  constexpr int W = U::W, N = 8;
+  __shared__ double red[1];
+  U u(A, j, r, G);
+  auto load = [&](long long p, GT& w0, GT (&v)[N]) {
+    w0 = u.w[p];
+#pragma unroll
+    for (int q = 0; q < N; q++) v[q] = u.VG[(size_t)min(q, j) * u.ldg + p];
   };
   auto rows = [&](long long p, const GT& w0, GT (&v)[N]) {
     double wv[W];
 #pragma unroll
     for (int e = 0; e < W; e++) wv[e] = (double)w0[e];
     for (int i = 0; i <= j; i += N) {
-      GT u[N];
+      GT x[N];
 #pragma unroll
-      for (int q = 0; q < N; q++) u[q] = v[q];
+      for (int q = 0; q < N; q++) x[q] = v[q];
       if (i + N <= j)
 #pragma unroll
-        for (int q = 0; q < N; q++) v[q] = VG[(size_t)min(i + N + q, j) * ldg + p];
+        for (int q = 0; q < N; q++) v[q] = u.VG[(size_t)min(i + N + q, j) * u.ldg + p];
 #pragma unroll
       for (int q = 0; q < N; q++)
-        if (i + q <= j)
-#pragma unroll
-          for (int e = 0; e < W; e++) wv[e] -= cs[i + q] * (double)u[q][e];
+        if (i + q <= j) u.sub(wv, cs[i + q], x[q]);
     }
-    GT wr;
-#pragma unroll
-    for (int e = 0; e < W; e++) {
-      const VT q = W * p + e < A.n ? (VT)wv[e] : (VT)0;  // padding rows stay zero
-      wr[e] = q;
-      acc += (double)q * (double)q;
-    }
-    w[p] = wr;
+    u.put(p, wv);
   };
-  // the first rows apart from the others: with their request carried through
-  // the loop the compiler (ROCm 7.2) overwrote half of a sum with the index
-  long long p = p0 + threadIdx.x;
+  long long p = u.p0 + threadIdx.x;
   GT w0 = 0, v[N];
 #pragma unroll
   for (int q = 0; q < N; q++) v[q] = 0;
-  if (p < p1) load(p, w0, v);
+  if (p < u.p1) load(p, w0, v);
   if (halt) return;
   coef();
-  if (p < p1) rows(p, w0, v);
-  for (p += SB; p < p1; p += SB) {
+  if (p < u.p1) rows(p, w0, v);
+  for (p += SB; p < u.p1; p += SB) {
     GT w1, v1[N];
     load(p, w1, v1);
     rows(p, w1, v1);
   }
-  block_sum_multi<1>(&acc, 1, red);
+  block_sum_multi<1>(&u.acc, 1, red);
+  if (threadIdx.x == 0) A.norms[pb] = red[0];
+}
+
+// Batches of many blocks per CU: wavefronts enough to hide every chain, so
+// eight vectors at a time, none requested twice, in 72 registers instead of 92
+// (seven wavefronts per SIMD instead of five).  The coefficients are there
+template <typename VT>
+__device__ __forceinline__ void update_stream(const SolveArgs& A, int j, int r, int G, int pb,
+                                              const double* cs) {
+  using U = UpdateRows<VT>;
+  using GT = typename U::GT;
+  constexpr int W = U::W, N = 8;
+  __shared__ double red[1];
+  U u(A, j, r, G);
+  for (long long p = u.p0 + threadIdx.x; p < u.p1; p += SB) {
+    const GT w0 = u.w[p];
+    double wv[W];
+#pragma unroll
+    for (int e = 0; e < W; e++) wv[e] = (double)w0[e];
+    int i = 0;
+    for (; i + N - 1 <= j; i += N) {
+      GT v[N];
+#pragma unroll
+      for (int q = 0; q < N; q++) v[q] = u.VG[(size_t)(i + q) * u.ldg + p];
+#pragma unroll
+      for (int q = 0; q < N; q++) u.sub(wv, cs[i + q], v[q]);
+    }
+    for (; i <= j; i++) u.sub(wv, cs[i], u.VG[(size_t)i * u.ldg + p]);
+    u.put(p, wv);
+  }
+  block_sum_multi<1>(&u.acc, 1, red);
   if (threadIdx.x == 0) A.norms[pb] = red[0];
 }
 
@@ -728,28 +780,31 @@ __device__ __forceinline__ void fin_dots_all(const SolveArgs& A, int j, int G, b
   __syncthreads();
 }
 
-template <class Coefs>
-__device__ __forceinline__ void update_any(const SolveArgs& A, int j, int r, int G, int pb,
-                                           const double* cs, int halt, Coefs coef) {
-  if (A.v32)
-    update_body<float>(A, j, r, G, pb, cs, halt, coef);
-  else
-    update_body<double>(A, j, r, G, pb, cs, halt, coef);
+// the coefficients k_fin_dots left
+__device__ __forceinline__ void load_coefs(const SolveArgs& A, int j, double* cs) {
+  if ((int)threadIdx.x <= j) cs[threadIdx.x] = Coef(A)[threadIdx.x];
+  __syncthreads();
 }
 
-// G > 0: the blocks reduce the G partial dots themselves; 0: k_fin_dots did
-__global__ void __launch_bounds__(SB) k_update(SolveArgs A, int j, int G) {
+// Gd > 0: the blocks reduce the Gd partial dots themselves; 0: k_fin_dots did
+__device__ __forceinline__ void update_ahead_any(const SolveArgs& A, int j, int r, int G, int Gd,
+                                                 double* cs) {
   const int halt = A.stat->stop;
+  auto coef = [&]() {
+    if (Gd > 0)
+      fin_dots_all(A, j, Gd, r == 0, cs);
+    else
+      load_coefs(A, j, cs);
+  };
+  if (A.v32)
+    update_ahead<float>(A, j, r, G, r, cs, halt, coef);
+  else
+    update_ahead<double>(A, j, r, G, r, cs, halt, coef);
+}
+
+__global__ void __launch_bounds__(SB) k_update(SolveArgs A, int j, int G) {
   __shared__ double cs[MAX_NV];
-  const int lb = xcd_block_rev(blockIdx.x, gridDim.x);
-  update_any(A, j, lb, gridDim.x, lb, cs, halt, [&]() {
-    if (G > 0) {
-      fin_dots_all(A, j, G, lb == 0, cs);
-    } else {
-      if ((int)threadIdx.x <= j) cs[threadIdx.x] = Coef(A)[threadIdx.x];
-      __syncthreads();
-    }
-  });
+  update_ahead_any(A, j, xcd_block_rev(blockIdx.x, gridDim.x), gridDim.x, G, cs);
 }
 
 __global__ void __launch_bounds__(OPB) k_fin_update(SolveArgs A, int j, int G) {
@@ -921,6 +976,15 @@ static OpGrid grid_op(const Problem& P) {
 // them once (4.7 us for 1024 partials of up to 50 vectors, which every one of
 // 2048 blocks would read as 400 KB)
 constexpr int kFuseDots = 512;
+// Blocks per CU up to which a batch's update reduces the dots itself and
+// requests ahead (update_ahead, 92 registers: five blocks are resident); a
+// larger batch, bound by bandwidth, takes kb_fin_dots and update_stream.  ms
+// per run of FP64 / mixed members, both ways: 32 of 2,000 to 60,000 prisms in
+// blocks of 8 slices (2 per CU) 5.95 / 5.66 and 6.11 / 5.98, in blocks of 2 (8
+// per CU) 6.65 / 6.74 and 6.48 / 6.56; 256 of 2,000 to 200,000 (43 per CU)
+// 111.0 / 74.4 and 104.5 / 70.7; 24 of 100,000 to 500,000 (24 per CU) 105.2 /
+// 65.0 and 98.9 / 60.3
+constexpr int kFuseBlocks = 5;
 // doubles of one row of the partials buffer (MAX_NV rows; the last holds the
 // norms of the updates)
 static size_t partials_row(const Problem& P) {
@@ -1992,18 +2056,21 @@ __global__ void __launch_bounds__(SB) kb_fin_dots(BatchArgs B, int j) {
   fin_dots_body(A, j, blockIdx.x, B.nblk[blockIdx.y]);
 }
 
-__global__ void __launch_bounds__(SB) kb_update(BatchArgs B, int j, int fuse) {
+template <bool FUSE>
+__global__ void __launch_bounds__(SB) kb_update(BatchArgs B, int j) {
   const int p = B.blk_prob[blockIdx.x], r = B.blk_rank[blockIdx.x], G = B.nblk[p];
   const SolveArgs A = B.args[p];
   __shared__ double cs[MAX_NV];
-  update_any(A, j, r, G, r, cs, A.stat->stop, [&]() {
-    if (fuse) {
-      fin_dots_all(A, j, G, r == 0, cs);
-    } else {
-      if ((int)threadIdx.x <= j) cs[threadIdx.x] = Coef(A)[threadIdx.x];
-      __syncthreads();
-    }
-  });
+  if constexpr (FUSE) {
+    update_ahead_any(A, j, r, G, G, cs);
+  } else {
+    if (A.stat->stop) return;
+    load_coefs(A, j, cs);
+    if (A.v32)
+      update_stream<float>(A, j, r, G, r, cs);
+    else
+      update_stream<double>(A, j, r, G, r, cs);
+  }
 }
 
 __global__ void __launch_bounds__(SB) kb_fin_update(BatchArgs B, int j) {
@@ -2482,9 +2549,9 @@ static void batch_enqueue_cycle(Batch& B, hipStream_t s, bool refine = true) {
   }
   hipLaunchKernelGGL(kb_restart, dim3(np), dim3(SB), 0, s, a);
   // two launches a step: see k_op_dots_sell and k_update.  ILU members need
-  // s_j in memory before the operator, members of many blocks their dots
-  // reduced once
-  const int fin = !B.has_ilu, fuse = B.max_blk <= kFuseDots;
+  // s_j in memory before the operator
+  const int fin = !B.has_ilu;
+  const bool fuse = B.nblk <= kFuseBlocks * num_cus() && B.max_blk <= kFuseDots;
   for (int j = 0; j < B.m; j++) {
     const int nfin = fin && j > 0 ? np : 0;
     hipLaunchKernelGGL(DOTS_KERNEL(kb_op_dots, j), dim3(nfin + B.nblk), dim3(SB), 0, s, a, j, nfin,
@@ -2494,7 +2561,7 @@ static void batch_enqueue_cycle(Batch& B, hipStream_t s, bool refine = true) {
       hipLaunchKernelGGL(DOTS_KERNEL(kb_dots, j), dim3(B.nblk), dim3(SB), 0, s, a, j);
     }
     if (!fuse) hipLaunchKernelGGL(kb_fin_dots, dim3(j + 1, np), dim3(SB), 0, s, a, j);
-    hipLaunchKernelGGL(kb_update, dim3(B.nblk), dim3(SB), 0, s, a, j, fuse);
+    hipLaunchKernelGGL(fuse ? kb_update<true> : kb_update<false>, dim3(B.nblk), dim3(SB), 0, s, a, j);
     if (!fin || j + 1 == B.m) hipLaunchKernelGGL(kb_fin_update, dim3(np), dim3(SB), 0, s, a, j);
   }
   hipLaunchKernelGGL(kb_ysolve, dim3(np), dim3(64), 0, s, a);
