@@ -956,10 +956,15 @@ static int grid_slices(const Problem& P) {
   const int nsl = (P.n + 63) / 64;
   return std::max(1, std::min((nsl + SW - 1) / SW, num_cus() * 8));
 }
-// blocks and wavefronts per block of the operator + dots kernels: one slice
+// Blocks and wavefronts per block of the operator + dots kernels: one slice
 // per wavefront in blocks that spread a small system over all CUs (a CU's
 // address unit serves its wavefronts one after the other: 19 blocks of 8
-// waves took twice as long as 145 of one), at most 4 blocks of 8 per CU
+// waves took twice as long as 145 of one).  Beyond a slice per wavefront of
+// k_op_dots_one, blocks of four, so that CUs differ by little, and no more
+// than are resident (four wavefronts per SIMD), so that none runs in a second
+// round.  us per step, m = 50, against up to 1024 blocks of eight: 185,193
+// rows 39.4 -> 34.7, 300,763 51.8 -> 46.0, 531,441 78.5 -> 72.1, 2,146,689
+// 301.7 -> 298.4
 struct OpGrid {
   int G, W;
   bool one;  // the launch has a slice per wavefront and is resident at once
@@ -967,15 +972,17 @@ struct OpGrid {
 static OpGrid grid_op(const Problem& P) {
   const int nsl = (P.n + 63) / 64, cu = num_cus();
   OpGrid g{1, 1, nsl <= 8 * cu};
-  while (g.W < OPB / 64 && nsl > g.W * cu) g.W *= 2;
+  while (g.W < (g.one ? OPB / 64 : 4) && nsl > g.W * cu) g.W *= 2;
   g.G = std::max(1, std::min((nsl + g.W - 1) / g.W, cu * 4));
   return g;
 }
-// largest number of dot partials per vector that every block of the update
-// reduces for itself (a launch less: 2.4 us); above it k_fin_dots reduces
-// them once (4.7 us for 1024 partials of up to 50 vectors, which every one of
-// 2048 blocks would read as 400 KB)
-constexpr int kFuseDots = 512;
+// largest number of dot partials, of all vectors together, that every block of
+// the update reduces for itself (a launch less: 2.4 us); above it k_fin_dots
+// reduces them once.  250,047 rows (489 partials per vector, 489 blocks), m =
+// 50: 43.8 us per step with all steps' dots in the update, 40.3 with this
+// limit, 40.4 with half of it, 41.3 with twice; 132,651 rows, m = 30: 27.8,
+// 27.3, 27.6 and 27.8
+constexpr int kFuseDots = 8192;
 // Blocks per CU up to which a batch's update reduces the dots itself and
 // requests ahead (update_ahead, 92 registers: five blocks are resident); a
 // larger batch, bound by bandwidth, takes kb_fin_dots and update_stream.  ms
@@ -1250,7 +1257,7 @@ static int zero_padding(const Problem& P, int m, int v32) {
 // update of w, whose norm is finished by fin_step or the next operator launch
 static void launch_update(int G_op, int G_up, const SolveArgs& A, int j) {
   hipStream_t s = stream();
-  const bool fuse = G_op <= kFuseDots;
+  const bool fuse = G_op * (j + 1) <= kFuseDots;
   if (!fuse) hipLaunchKernelGGL(k_fin_dots, dim3(j + 1), dim3(SB), 0, s, A, j, G_op);
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (g_ks.on) {
@@ -2551,7 +2558,6 @@ static void batch_enqueue_cycle(Batch& B, hipStream_t s, bool refine = true) {
   // two launches a step: see k_op_dots_sell and k_update.  ILU members need
   // s_j in memory before the operator
   const int fin = !B.has_ilu;
-  const bool fuse = B.nblk <= kFuseBlocks * num_cus() && B.max_blk <= kFuseDots;
   for (int j = 0; j < B.m; j++) {
     const int nfin = fin && j > 0 ? np : 0;
     hipLaunchKernelGGL(DOTS_KERNEL(kb_op_dots, j), dim3(nfin + B.nblk), dim3(SB), 0, s, a, j, nfin,
@@ -2560,6 +2566,7 @@ static void batch_enqueue_cycle(Batch& B, hipStream_t s, bool refine = true) {
       batch_ilu_levels(B, a, j, s);
       hipLaunchKernelGGL(DOTS_KERNEL(kb_dots, j), dim3(B.nblk), dim3(SB), 0, s, a, j);
     }
+    const bool fuse = B.nblk <= kFuseBlocks * num_cus() && B.max_blk * (j + 1) <= kFuseDots;
     if (!fuse) hipLaunchKernelGGL(kb_fin_dots, dim3(j + 1, np), dim3(SB), 0, s, a, j);
     hipLaunchKernelGGL(fuse ? kb_update<true> : kb_update<false>, dim3(B.nblk), dim3(SB), 0, s, a, j);
     if (!fin || j + 1 == B.m) hipLaunchKernelGGL(kb_fin_update, dim3(np), dim3(SB), 0, s, a, j);
