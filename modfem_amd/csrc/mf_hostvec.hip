@@ -22,7 +22,10 @@ namespace mf {
 namespace {
 
 // the ring is one per process: 4 MB, whatever the number of problems.  A
-// slot is written again only when the kernel that used it last has ended
+// slot is written again only when the kernel that used it last has ended.  It
+// belongs to the library stream: when mf_init has chosen another device since
+// the last vector, the former stream is waited for and the events, which
+// belong to that stream's device, are made anew
 constexpr long long kChunk = 1 << 17;  // doubles per slot
 constexpr int kSlots = 4;
 
@@ -32,12 +35,23 @@ struct Ring {
   hipEvent_t ev[kSlots] = {};
   enum State { kFree, kQueued, kTimed } st[kSlots] = {};  // kTimed: ev tells when it is done
   int next = 0;
+  hipStream_t owner = nullptr;
 
   int init() {
-    if (p) return 0;
+    if (p && owner == stream()) return 0;
+    if (owner && owner != stream()) {
+      MF_HIP(hipStreamSynchronize(owner));
+      all_free();
+      owner = nullptr;
+      for (hipEvent_t& e : ev) {
+        if (e) MF_HIP(hipEventDestroy(e));
+        e = nullptr;
+      }
+    }
     for (hipEvent_t& e : ev)
       if (!e) MF_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    MF_HIP(hipHostMalloc(&p, kSlots * kChunk * sizeof(double), hipHostMallocDefault));
+    if (!p) MF_HIP(hipHostMalloc(&p, kSlots * kChunk * sizeof(double), hipHostMallocPortable));
+    owner = stream();
     return 0;
   }
   void all_free() {
