@@ -92,12 +92,12 @@ struct GmresStat {
   double beta1;
 };
 
+int num_cus();  // compute units of the current device
+
 // ILU(0) preconditioner on the device (mf_ilu.hip): the pattern in an
 // elimination order (0: the reference's DOF order, 1: multicolour), rows of
 // each forward / backward level, and the factors (strict L, strict U, and
 // 1/u_ii on the diagonal as the reference keeps it).
-int num_cus();  // compute units of the current device
-
 struct IluData {
   int order = 0, n = 0;
   long long nnz = 0;

@@ -732,6 +732,10 @@ __device__ __forceinline__ void row_flux(const TermMask& M, const Coefs& C, R gx
 template <class Q, int TS, typename R>
 __device__ __forceinline__ void prism_row(const IntArgs& I, int e, int w, const int* dof,
                                           double* K, R& Fw) {
+  // three triangle points on each of two heights, all of one weight
+  static_assert(Q::NG == 6 && Q::z(0) == Q::z(2) && Q::z(3) == Q::z(5) && Q::x(0) == Q::x(3) &&
+                    Q::x(2) == Q::x(5) && Q::y(1) == Q::y(4) && Q::w(0) == Q::w(5),
+                "prism_row goes through the rule by height and triangle point");
   double x0[3], e1[2][3], e2[2][3], d[3][3];  // edges below and above, half heights
   {
     double xn[6][3];

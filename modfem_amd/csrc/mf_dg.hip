@@ -2013,24 +2013,21 @@ struct DgIluLay {
   const int* fcode;
   const int* deg;
   int ns;
-  const long long* xoff;
   const long long* soff;
   const long long* voff;
   __device__ int nse(int e) const { return deg ? ns_of_deg(deg[e]) : ns; }
-  __device__ long long xo(int e) const { return xoff ? xoff[e] : (long long)e * ns; }
   __device__ long long so(int e, int s) const {
     return soff ? soff[6 * (size_t)e + s] : ((long long)e * 6 + s) * ns * ns;
   }
   __device__ long long vo(int e) const { return voff ? voff[e] : (long long)e * ns * ns; }
 };
 
-// sides of element i towards neighbours below (lower) or above i, ordered by
-// neighbour index
-__device__ __forceinline__ int dg_sorted_sides(const int* fnb, int i, bool lower, int* side) {
+// sides of element i towards neighbours below i, ordered by neighbour index
+__device__ __forceinline__ int dg_lower_sides(const int* fnb, int i, int* side) {
   int n = 0;
   for (int s = 0; s < 5; s++) {
     const int nb = fnb[5 * (size_t)i + s];
-    if (nb < 0 || (lower ? nb >= i : nb <= i)) continue;
+    if (nb < 0 || nb >= i) continue;
     int t = n++;
     while (t > 0 && nb < fnb[5 * (size_t)i + side[t - 1]]) {
       side[t] = side[t - 1];
@@ -2090,7 +2087,7 @@ __global__ void __launch_bounds__(256) k_dg_ilu_row(const int* rows, DgIluLay Y,
   const double* Ai = F + Y.so(i, 0);
   for (int q = tid; q < ni * ni; q += nt) D[q] = Ai[q];
   int side[5];
-  const int nl = dg_sorted_sides(Y.fnb, i, true, side);
+  const int nl = dg_lower_sides(Y.fnb, i, side);
   for (int t = 0; t < nl; t++) {
     const int s = side[t], k = Y.fnb[5 * (size_t)i + s], nk = Y.nse(k);
     double* Aik = F + Y.so(i, 1 + s);
@@ -3022,8 +3019,7 @@ int fill_block_jacobi(DgProblem& D) {
 
 DgIluLay ilu_layout(const DgProblem& D) {
   return DgIluLay{D.d_fnb, D.d_fcode, D.mixed ? D.d_deg : nullptr, D.mixed ? 0 : D.ns,
-                  D.mixed ? D.d_xoff : nullptr, D.mixed ? D.d_soff : nullptr,
-                  D.mixed ? D.d_voff : nullptr};
+                  D.mixed ? D.d_soff : nullptr, D.mixed ? D.d_voff : nullptr};
 }
 
 // level schedules of the ILU: the forward level of element i is one more than

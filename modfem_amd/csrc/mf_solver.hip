@@ -2488,6 +2488,7 @@ static int batch_build(Batch& B) {
   }
   B.nblk = (int)bp.size();
   B.max_blk = np ? *std::max_element(nblk.begin(), nblk.end()) : 0;
+  // MAX_BLOCKS blocks of at most 128 slices: larger blocks are not supported
   if (max_sl > 128) {
     set_error("batch: a member is too large for the batched operator (> 33M rows)");
     return -1;

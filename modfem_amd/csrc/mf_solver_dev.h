@@ -245,7 +245,7 @@ __device__ __forceinline__ double sell_row(const SolveArgs& A, const VT* val, co
 // are requested at once (two trips to memory for a row of a box mesh instead
 // of four); groups of four past the slice's length are skipped by a
 // wave-uniform test.  before(): loads to issue behind the first columns and
-// values
+// values (len >= 1: every row of a problem has its diagonal entry)
 constexpr int kSellWide = 28;
 
 template <typename VT, typename XT, typename CT, class Before>
