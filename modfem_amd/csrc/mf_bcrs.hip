@@ -161,15 +161,18 @@ __device__ __forceinline__ double group_turn(double v) {
 // block Jacobi sweep: every row reads the old v.  With a row list (rows of
 // one colour class, none sharing a block) the same kernel sweeps the class in
 // place (out = v).  16 lanes per row, lane (l, k) owns entry (k, l) of every
-// block, so kBjChunk blocks (128 contiguous bytes each) and their vector
-// entries are in flight together; the products of component k are then
-// subtracted in R's order (blocks in sweep order, l ascending), passed
-// between the lanes of the row by DPP.  A colour class of the 24^3 box holds
-// ~1300 rows: the launch is bound by its chain of dependent loads, and one
-// thread per unknown with two blocks in flight took 11.2 us (GMRES with two
-// sweeps in colour order 21.8 ms, 14.2 ms so).
-constexpr int kBjChunk = 14;
-
+// block, so CH blocks (128 contiguous bytes each) and their vector entries are
+// in flight together; the products of component k are then subtracted in R's
+// order (blocks in sweep order, l ascending), passed between the lanes of the
+// row by DPP; the factors are read behind the blocks, so that they cost no
+// registers before.  A colour class of the 24^3 box holds ~1400 rows: its
+// launch is bound by its chain of dependent loads, and one thread per unknown
+// with two blocks in flight took 139 us per two-sided sweep of 11 classes, CH
+// 14 with the factors ahead 88, CH 4 79, CH 8 71.  A launch of many rows is
+// bound by its bytes and by what is resident: 117,649 rows (340 MB) 87.9 us
+// with one thread per unknown, 106.1 with CH 14 (120 registers), 92.8 with CH
+// 8, 86.9 with CH 4
+template <int CH>
 __global__ void __launch_bounds__(256) k_bcrs_bj(int nrows, const int* rows, int dir,
                                                  const int* rp, const int* ci, const int* diag,
                                                  const double* val, const double* lu,
@@ -187,27 +190,20 @@ __global__ void __launch_bounds__(256) k_bcrs_bj(int nrows, const int* rows, int
   const int nlow = d - r0, nup = r1 - d - 1, nbk = nlow + nup;
   const int n1 = dir == 0 ? nlow : nup;
   const int s1 = dir == 0 ? r0 : d + 1, s2 = (dir == 0 ? d + 1 : r0) - n1;
-  double f[16];
-  int ip[4];
-#pragma unroll
-  for (int q = 0; q < 16; q++) f[q] = lu[16 * (size_t)r + q];
-#pragma unroll
-  for (int q = 0; q < 4; q++) ip[q] = piv[4 * (size_t)r + q];
-  const double bk = b ? b[4 * (size_t)r + k] : 0.0;
   double acc = 0.0;
-  for (int q0 = 0; q0 < nbk; q0 += kBjChunk) {
-    double a[kBjChunk], y[kBjChunk];
-    int c[kBjChunk];
+  for (int q0 = 0; q0 < nbk; q0 += CH) {
+    double a[CH], y[CH];
+    int c[CH];
 #pragma unroll
-    for (int q = 0; q < kBjChunk; q++) {
+    for (int q = 0; q < CH; q++) {
       const int w = min(q0 + q, nbk - 1), s = w < n1 ? s1 + w : s2 + w;
       c[q] = ci[s];
       a[q] = val[16 * (size_t)s + e];
     }
 #pragma unroll
-    for (int q = 0; q < kBjChunk; q++) y[q] = v[4 * (size_t)c[q] + l];
+    for (int q = 0; q < CH; q++) y[q] = v[4 * (size_t)c[q] + l];
 #pragma unroll
-    for (int q = 0; q < kBjChunk; q++) {
+    for (int q = 0; q < CH; q++) {
       const double p = __dmul_rn(a[q], y[q]);
       double z = __dsub_rn(acc, p);
       z = __dsub_rn(z, group_turn<1>(p));
@@ -216,7 +212,13 @@ __global__ void __launch_bounds__(256) k_bcrs_bj(int nrows, const int* rows, int
       acc = q0 + q < nbk ? z : acc;
     }
   }
-  if (b) acc = __dadd_rn(acc, bk);
+  double f[16];
+  int ip[4];
+#pragma unroll
+  for (int q = 0; q < 16; q++) f[q] = lu[16 * (size_t)r + q];
+#pragma unroll
+  for (int q = 0; q < 4; q++) ip[q] = piv[4 * (size_t)r + q];
+  if (b) acc = __dadd_rn(acc, b[4 * (size_t)r + k]);
   // the sums of components 0..3 sit in lanes 0..3 of the group
   const int base = (int)(threadIdx.x & 48u);
   double y[4];
@@ -643,6 +645,17 @@ int bcrs_fill_lu(BcrsDev& M) {
   return 0;
 }
 
+// a launch of k_bcrs_bj: eight blocks of a row in flight up to two wavefronts
+// per SIMD (32 rows per CU), four beyond.  Sweeps of 4,913 rows 9.1 us both
+// ways, 9,261 rows 11.5 / 10.7; classes of 6,265 rows 92.6 / 94.5 us per
+// two-sided sweep, of 10,695 rows 152.8 / 143.5
+static void launch_bj(const BcrsDev& M, int cnt, const int* rows, int dir, const double* b,
+                      const double* v, double* out, const int* stop) {
+  hipLaunchKernelGGL(cnt <= 32 * num_cus() ? k_bcrs_bj<8> : k_bcrs_bj<4>, dim3((cnt + 15) / 16),
+                     dim3(256), 0, stream(), cnt, rows, dir, M.d_rp, M.d_ci, M.d_diag, M.d_val,
+                     M.d_lu, M.d_piv, b, v, out, stop);
+}
+
 int bcrs_sweeps(BcrsDev& M, int gs, int nr_prec, const double* b, double* v, double* tmp,
                 const int* stop, bool sync) {
   const int loops = nr_prec % 2 == 0 ? nr_prec / 2 : nr_prec / 2 + 1;
@@ -657,9 +670,7 @@ int bcrs_sweeps(BcrsDev& M, int gs, int nr_prec, const double* b, double* v, dou
         for (int q = 0; q < ncol; q++) {
           const int c = dir == 0 ? q : ncol - 1 - q;
           const int cnt = M.col_ptr[c + 1] - M.col_ptr[c];
-          hipLaunchKernelGGL(k_bcrs_bj, dim3((cnt + 15) / 16), dim3(256), 0, stream(), cnt,
-                             M.d_col_rows + M.col_ptr[c], 0, M.d_rp, M.d_ci, M.d_diag, M.d_val,
-                             M.d_lu, M.d_piv, b, v, v, stop);
+          launch_bj(M, cnt, M.d_col_rows + M.col_ptr[c], 0, b, v, v, stop);
         }
     MF_HIP(hipGetLastError());
     if (sync) MF_HIP(hipStreamSynchronize(stream()));
@@ -668,8 +679,7 @@ int bcrs_sweeps(BcrsDev& M, int gs, int nr_prec, const double* b, double* v, dou
   for (int it = 0; it < loops; it++)
     for (int dir = 0; dir < dirs; dir++) {
       if (!gs) {
-        hipLaunchKernelGGL(k_bcrs_bj, dim3((M.nb + 15) / 16), dim3(256), 0, stream(), M.nb, nullptr, dir,
-                           M.d_rp, M.d_ci, M.d_diag, M.d_val, M.d_lu, M.d_piv, b, v, tmp, stop);
+        launch_bj(M, M.nb, nullptr, dir, b, v, tmp, stop);
       } else {
         const std::vector<int>& lp = M.lev_ptr[dir];
         for (size_t l = 0; l + 1 < lp.size(); l++) {
